@@ -17,15 +17,18 @@ constexpr int kMaxDepthSlots = 64; // histogram slots for node depths
 // node's WalkHead below).  128 bytes = one L2 line.
 constexpr int32_t kLinkZeroMass = 1 << 30;   // link flag: zero mass, skipped whole
 struct alignas(128) RefNode {
-  double cx, cy, cz, m;    // centre of mass, mass
+  double cx, cy, cz;       // centre of mass
+  double dmk;              // 2*size / m^0.333333333 (softening floor of a dark-matter target, octree.h:146-148)
+  double m;                // mass
+  double esum;             // size*0.015 + cbrt(m)*0.002 (softening numerator)
   int32_t skip;            // preorder index of the first node after this subtree
   int32_t body;            // leaf: sorted body index; internal: -1
   int32_t depth;
   int32_t first;           // first body (sorted index) of the subtree
-  double size;             // half-width: root half-width * 2^-depth
-  double esum;             // size*0.015 + cbrt(m)*0.002 (softening numerator)
+  // internal nodes only
   double qxx, qyy, qzz, qxy, qxz, qyz;
-  double pad_[2];
+  double size;             // half-width: root half-width * 2^-depth
+  double pad_;
 };
 static_assert(sizeof(RefNode) == 128, "RefNode layout");
 
@@ -85,7 +88,7 @@ struct SysArrays {
   int32_t nsys;
 };
 
-// One wave of walk targets: up to 64 consecutive bodies of one system.
+// One wave of walk targets: consecutive bodies of one system, at most 64.
 struct Group {
   int32_t first, count, sys, pad;
 };

@@ -66,7 +66,7 @@ struct nbx_ctx {
   // systems
   std::vector<int64_t> sys_n;              // bodies per system
   DBuf s_root, s_dt, s_v2, s_soff, s_sroot, s_send;
-  DBuf groups, boxes, box_off, box_part;
+  DBuf groups, boxes, box_off, box_part;   // groups: reference mode's walk groups
   int64_t ngroups = 0;
   DBuf tgroups;               // physics mode: walk groups packed from the tree
   DBuf gmarks;                // physics mode: per-body group counts and marks
@@ -275,18 +275,36 @@ nbx_status ensure_particles(nbx_ctx* c, int64_t n, int64_t keep_n) {
   return NBX_OK;
 }
 
-// Host-built tables for the current systems: body offsets, walk groups (64
-// bodies of one system each), bounding-box blocks.
+// Reference mode's walk groups: runs of walk_width bodies of one system each.
+nbx_status set_groups(nbx_ctx* c) {
+  std::vector<Group> groups;
+  int32_t at = 0;
+  for (size_t s = 0; s < c->sys_n.size(); ++s) {
+    const int32_t end = at + (int32_t)c->sys_n[s], width = walk_width(c->sys_n[s], c->cfg.theta);
+    for (int32_t b = at; b < end; b += width)
+      groups.push_back(Group{b, std::min<int32_t>(width, end - b), (int32_t)s, 0});
+    at = end;
+  }
+  NBXCHK(ensure(c, c->groups, std::max<size_t>(groups.size(), 1) * sizeof(Group)));
+  if (!groups.empty()) {
+    HIPCHK(c, hipMemcpyAsync(c->groups.p, groups.data(), groups.size() * sizeof(Group), hipMemcpyHostToDevice,
+                             c->stream));
+    HIPCHK(c, hipStreamSynchronize(c->stream));   // the host vector goes out of scope
+  }
+  c->ngroups = (int64_t)groups.size();
+  ++c->gen;
+  return NBX_OK;
+}
+
+// Host-built tables for the current systems: body offsets, walk groups,
+// bounding-box blocks.
 nbx_status set_systems(nbx_ctx* c) {
   const int S = (int)c->sys_n.size();
   std::vector<int32_t> soff(S + 1, 0);
   for (int s = 0; s < S; ++s) soff[s + 1] = soff[s] + (int32_t)c->sys_n[s];
-  std::vector<Group> groups;
   std::vector<BoxBlock> boxes;
   std::vector<int32_t> box_off(S + 1, 0);
   for (int s = 0; s < S; ++s) {
-    for (int32_t b = soff[s]; b < soff[s + 1]; b += kWave)
-      groups.push_back(Group{b, std::min<int32_t>(kWave, soff[s + 1] - b), s, 0});
     for (int32_t b = soff[s]; b < soff[s + 1]; b += kBoxSpan)
       boxes.push_back(BoxBlock{s, b, std::min<int32_t>(b + kBoxSpan, soff[s + 1]), 0});
     box_off[s + 1] = (int32_t)boxes.size();
@@ -298,22 +316,18 @@ nbx_status set_systems(nbx_ctx* c) {
   NBXCHK(ensure(c, c->s_soff, (SS + 1) * 4));
   NBXCHK(ensure(c, c->s_sroot, SS * 4));
   NBXCHK(ensure(c, c->s_send, SS * 4));
-  NBXCHK(ensure(c, c->groups, std::max<size_t>(groups.size(), 1) * sizeof(Group)));
   NBXCHK(ensure(c, c->boxes, std::max<size_t>(boxes.size(), 1) * sizeof(BoxBlock)));
   NBXCHK(ensure(c, c->box_off, (SS + 1) * 4));
   NBXCHK(ensure(c, c->box_part, std::max<size_t>(boxes.size(), 1) * 6 * 8));
   NBXCHK(ensure(c, c->epart, std::max<size_t>(boxes.size(), 1) * 5 * 8));
   NBXCHK(ensure(c, c->eout, SS * 5 * 8));
   HIPCHK(c, hipMemcpyAsync(c->s_soff.p, soff.data(), soff.size() * 4, hipMemcpyHostToDevice, c->stream));
-  if (!groups.empty())
-    HIPCHK(c, hipMemcpyAsync(c->groups.p, groups.data(), groups.size() * sizeof(Group), hipMemcpyHostToDevice,
-                             c->stream));
   if (!boxes.empty())
     HIPCHK(c, hipMemcpyAsync(c->boxes.p, boxes.data(), boxes.size() * sizeof(BoxBlock), hipMemcpyHostToDevice,
                              c->stream));
   HIPCHK(c, hipMemcpyAsync(c->box_off.p, box_off.data(), box_off.size() * 4, hipMemcpyHostToDevice, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));   // the host vectors go out of scope
-  c->ngroups = (int64_t)groups.size();
+  if (!c->physics) NBXCHK(set_groups(c));
   c->nboxes = (int)boxes.size();
   ++c->gen;
   c->acc_valid = false;
@@ -1235,6 +1249,10 @@ nbx_status nbx_set_theta(nbx_ctx* c, double theta) {
   c->cfg.theta = theta;
   c->acc_valid = false;
   ++c->gen;
+  if (!c->physics && !c->sys_n.empty()) {                  // the group width depends on theta
+    NBXCHK(check_ctx(c));
+    NBXCHK(set_groups(c));
+  }
   return NBX_OK;
 }
 
@@ -1640,8 +1658,21 @@ nbx_status nbx_debug_groups(nbx_ctx* c, int64_t cap, int32_t* first, int32_t* co
     NBXCHK(sync_scalars(c));
     c->ntgroups = c->hsc->tree_groups;
   }
-  const int64_t ng = c->physics ? c->ntgroups : c->ngroups;
-  const Group* dg = P<Group>(c->physics ? c->tgroups : c->groups);
+  if (!c->physics) {                                       // runs of 64 (the walk may split them)
+    int32_t at = 0;
+    for (size_t s = 0; s < c->sys_n.size(); ++s)
+      for (const int32_t end = at + (int32_t)c->sys_n[s]; at < end; at = std::min<int32_t>(at + kWave, end)) {
+        if (*ngroups < cap) {
+          first[*ngroups] = at;
+          count[*ngroups] = std::min<int32_t>(kWave, end - at);
+          sys[*ngroups] = (int32_t)s;
+        }
+        ++*ngroups;
+      }
+    return NBX_OK;
+  }
+  const int64_t ng = c->ntgroups;
+  const Group* dg = P<Group>(c->tgroups);
   *ngroups = ng;
   const int64_t k = std::min(ng, cap);
   if (k == 0) return NBX_OK;

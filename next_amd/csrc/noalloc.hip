@@ -32,7 +32,7 @@ namespace {
 
 constexpr int64_t kNaBodies = NBX_NOALLOC_MAX_BODIES;
 constexpr int64_t kNaNodes = NBX_NOALLOC_MAX_NODES;   // tree nodes, leaves included
-constexpr int64_t kNaGroups = (kNaBodies + kWave - 1) / kWave;
+constexpr int64_t kNaGroups = (kNaBodies + 7) / 8;            // the narrowest walk groups hold 8 bodies
 constexpr int64_t kNaBoxes = (kNaBodies + kBoxSpan - 1) / kBoxSpan;
 
 constexpr size_t align256(size_t b) { return (b + 255) & ~size_t(255); }
@@ -64,7 +64,7 @@ constexpr Layout make_layout() {
   const size_t sw = sort_scratch_words(big);
   const size_t cw = (size_t)((big + kScanTile - 1) / kScanTile + 2);
   L.sortscr = take((sw > cw ? sw : cw) * 4);
-  L.nodes = take((size_t)(kNaNodes + 1) * sizeof(RefNode));   // one spare record for the walk
+  L.nodes = take((size_t)(kNaNodes + 1) * sizeof(RefNode));   // one all-zero record after the last node
   L.heads = take((size_t)(kNaNodes + 1) * sizeof(WalkHead));
   L.level_list = take((size_t)kNaNodes * 4);
   L.end_list = take((size_t)kNaNodes * 4);
@@ -99,13 +99,13 @@ std::mutex g_lock[kMaxDevices];
 unsigned char* g_ptr[kMaxDevices] = {};   // device address of `scratch` per device (under g_lock)
 
 // Caller's bodies into the first state buffers (velocities zero, upload
-// index, system 0), and the one-system tables: walk groups of 64 bodies,
+// index, system 0), and the one-system tables: walk groups of `width` bodies,
 // bounding-box blocks, body offsets.
 __global__ __launch_bounds__(kBlock) void k_na_setup(int64_t n, const double* __restrict__ x,
                                                      const double* __restrict__ y, const double* __restrict__ z,
                                                      const double* __restrict__ m, const int32_t* __restrict__ type,
                                                      StateArrays st, Group* groups, BoxBlock* boxes,
-                                                     int32_t* box_off, int32_t* soff) {
+                                                     int32_t* box_off, int32_t* soff, int32_t width) {
   const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
   if (i < n) {
     st.x[i] = x[i]; st.y[i] = y[i]; st.z[i] = z[i];
@@ -113,10 +113,10 @@ __global__ __launch_bounds__(kBlock) void k_na_setup(int64_t n, const double* __
     st.m[i] = m[i]; st.type[i] = type[i];
     st.id[i] = (int32_t)i; st.sys[i] = 0;
   }
-  const int64_t ng = (n + kWave - 1) / kWave, nb = (n + kBoxSpan - 1) / kBoxSpan;
+  const int64_t ng = (n + width - 1) / width, nb = (n + kBoxSpan - 1) / kBoxSpan;
   if (i < ng) {
-    const int32_t f = (int32_t)(i * kWave);
-    groups[i] = Group{f, (int32_t)std::min<int64_t>(kWave, n - f), 0, 0};
+    const int32_t f = (int32_t)(i * width);
+    groups[i] = Group{f, (int32_t)std::min<int64_t>(width, n - f), 0, 0};
   }
   if (i < nb) {
     const int32_t b = (int32_t)(i * kBoxSpan);
@@ -185,7 +185,7 @@ nbx_status accel_in_arena(const Arena& A, int64_t n, const double* x, const doub
   const int64_t nb = (n + kBoxSpan - 1) / kBoxSpan;
   hipLaunchKernelGGL(k_na_setup, dim3((unsigned)div_up(n, kBlock)), dim3(kBlock), 0, s,
                      n, x, y, z, m, type, St, A.at<Group>(kLayout.groups), A.at<BoxBlock>(kLayout.boxes),
-                     A.at<int32_t>(kLayout.box_off), A.at<int32_t>(kLayout.soff));
+                     A.at<int32_t>(kLayout.box_off), A.at<int32_t>(kLayout.soff), walk_width(n, theta));
   launch_bbox(St, A.at<BoxBlock>(kLayout.boxes), (int)nb, A.at<int32_t>(kLayout.box_off),
               A.at<double>(kLayout.box_part), sy, nullptr, s);
   launch_fill_scalars(sc, 1 | 4 | 8, s);
@@ -227,7 +227,7 @@ nbx_status accel_in_arena(const Arena& A, int64_t n, const double* x, const doub
               (uint32_t)kNaNodes, s);
   launch_upward_all(h.level_count, level_list, end_list, nodes, heads, theta, St.sys, sy.root, s);
   double* acc[3] = {A.at<double>(kLayout.acc[0]), A.at<double>(kLayout.acc[1]), A.at<double>(kLayout.acc[2])};
-  launch_walk(A.at<Group>(kLayout.groups), div_up(n, kWave), nodes, heads, St, sy, theta, acc[0], acc[1], acc[2], sc,
+  launch_walk(A.at<Group>(kLayout.groups), div_up(n, walk_width(n, theta)), nodes, heads, St, sy, theta, acc[0], acc[1], acc[2], sc,
               false, false, s);
   hipLaunchKernelGGL(k_na_scatter, dim3((unsigned)div_up(n, kBlock)), dim3(kBlock), 0, s, n, St.id, acc[0], acc[1],
                      acc[2], ax, ay, az);

@@ -14,10 +14,10 @@
 //         the rule "an internal node exists for every digit prefix shared by
 //         two or more bodies", with skip pointers for stackless traversal
 //   upward pass, one launch per depth, deepest first (octree.h:92-127)
-//   walk: one wave per 64 consecutive targets; the wave visits the union of
-//         its lanes' depth-first paths in preorder, each lane applying its own
-//         acceptance test (octree.h:133-179), so every lane accumulates the
-//         same terms in the same order as the recursive reference.
+//   walk: one wave per group of consecutive targets; the group decides once
+//         what all its targets decide alike, each target walks the rest with
+//         its own acceptance test (octree.h:133-179), so every target
+//         accumulates the reference's terms.
 #include "common.hpp"
 #include "layout.hpp"
 #include "prims.hpp"
@@ -155,6 +155,18 @@ __device__ __forceinline__ void key_digits(double px, double py, double pz, cons
     cz = cz + ((o & 4u) ? hs : -hs);
     s = hs;
   }
+}
+
+// m^0.333333333 (the exponent of octree.h:146) from cbrt(m): the exponents
+// differ by d = 3.3e-10, and m^-d = 1 - d ln m + (d ln m)^2 / 2 with
+// |d ln m| < 2.5e-7, so ln m is needed to about 1e-6 only.  Odd in m, and 0
+// at 0.
+__device__ __forceinline__ double dm_power(double m, double cbrt_m) {
+  if (m == 0.0) return 0.0;
+  int e;
+  const float f = (float)frexp(fabs(m), &e);
+  const double t = (1.0 / 3.0 - 0.333333333) * (double)(__logf(f) + 0.69314718f * (float)e);
+  return cbrt_m * ((1.0 - t) + 0.5 * t * t);
 }
 
 __device__ __forceinline__ void sys_root(const SysArrays& sy, int32_t s, double root[4]) {
@@ -422,8 +434,8 @@ __global__ __launch_bounds__(kBlock) void k_emit(int64_t n, const int32_t* __res
   place_internal_nodes(valid, lp, li, pre, skipv, part, sc, level_list, end_list,
                        cap_int);
   if (!valid) return;
-  // One all-zero record after the last node: the walk's evaluation reads it
-  // for a lane with no entry left and for a leaf's quadrupole.
+  // One all-zero record after the last node: the walk reads a leaf's
+  // quadrupole there.
   if (i == n - 1) {
     const uint32_t z = (uint32_t)sc->total_nodes;
     if (z < cap_nodes) nodes[z] = RefNode{};
@@ -446,9 +458,10 @@ __global__ __launch_bounds__(kBlock) void k_emit(int64_t n, const int32_t* __res
     nd.body = (int32_t)i;
     nd.depth = d;
     nd.first = (int32_t)i;
-    nd.size = size;
     // softening.h:26-27: size*0.015 + cbrt(m)*0.002, summed before the taper
-    nd.esum = size * 0.015 + cbrt(m) * 0.002;
+    const double cm = cbrt(m);
+    nd.esum = size * 0.015 + cm * 0.002;
+    nd.dmk = 2.0 * size / dm_power(m, cm);
     // a leaf is accepted whatever its distance: no threshold
     heads[p] = WalkHead{px, py, pz, 0.0f, m == 0.0 ? (int32_t)(p + 1) | kLinkZeroMass : ~(int32_t)i};
   }
@@ -534,12 +547,14 @@ __device__ __forceinline__ void upward_node(int32_t id, int32_t end, int d, RefN
   p.depth = d;
   p.first = first;
   p.size = size;
-  p.esum = size * 0.015 + cbrt(M) * 0.002;
+  const double cm = cbrt(M);
+  p.esum = size * 0.015 + cm * 0.002;
+  p.dmk = 2.0 * size / dm_power(M, cm);
   p.qxx = qxx; p.qyy = qyy; p.qzz = qzz; p.qxy = qxy; p.qxz = qxz; p.qyz = qyz;
   RefNode& out = nodes[id];                  // the record but its padding
   out.cx = p.cx; out.cy = p.cy; out.cz = p.cz; out.m = p.m;
   out.skip = p.skip; out.body = p.body; out.depth = p.depth; out.first = p.first;
-  out.size = p.size; out.esum = p.esum;
+  out.size = p.size; out.esum = p.esum; out.dmk = p.dmk;
   out.qxx = p.qxx; out.qyy = p.qyy; out.qzz = p.qzz; out.qxy = p.qxy; out.qxz = p.qxz; out.qyz = p.qyz;
   // Upper edge of the opening test's band for r^2 (NEXT tests r^2 + 1e-20,
   // so the 1e-20 is taken off the edge); NaN, and every decision exact, where
@@ -623,251 +638,335 @@ __device__ __forceinline__ double rcp_nr(double x) {
   return __builtin_fma(y, e, y);
 }
 
-// Softening floor of a dark-matter target (octree.h:146-148), out of line:
-// expanded in place, the FP64 pow raises the walk's register count by about
-// half for every target.
-__device__ __noinline__ double dm_softening(double eps, double size, double m, double mi) {
-  const double alt = 2.0 * size / pow(m / mi, 0.333333333);
-  return eps < alt ? alt : eps;
-}
-
-// k < 2^25, checked on the host: the byte offset fits 32 bits and becomes the
-// scalar load's offset register.
-// The per-visit fields of a node as the traversal holds them: the head,
-// loaded as one 8-dword value (one scalar load), with the FP32 threshold
-// kept as its bits until it is used.  (Read as a float straight from the
-// loaded vector, the threshold was folded to element 0 instead of 6 by the
-// ROCm 7.2 compiler, which wrecked every opening decision; the integer
-// extraction compiles correctly.)
-typedef uint32_t u32x8 __attribute__((ext_vector_type(8)));
-struct HeadRegs {
-  double cx, cy, cz;
-  uint32_t acc2_bits;
-  int32_t link;
-};
-__device__ __forceinline__ HeadRegs load_head(const WalkHead* __restrict__ heads, uint32_t k) {
-  const u32x8 r = *reinterpret_cast<const u32x8*>(reinterpret_cast<const char*>(heads) + (k << 5));
-  HeadRegs h;
-  h.cx = __builtin_bit_cast(double, (uint64_t)r[0] | ((uint64_t)r[1] << 32));
-  h.cy = __builtin_bit_cast(double, (uint64_t)r[2] | ((uint64_t)r[3] << 32));
-  h.cz = __builtin_bit_cast(double, (uint64_t)r[4] | ((uint64_t)r[5] << 32));
-  h.acc2_bits = r[6];
-  h.link = (int32_t)r[7];
-  return h;
-}
-
 // Lower edge of the opening test's band from its upper edge acc2 (FP32,
 // (size/theta)^2 (1 + 2e-6) - 1e-20 rounded up, for (size/theta)^2 > 1e-16):
 // r^2 below it has r^2 + 1e-20 below (size/theta)^2 (1 - 2e-6).  Squared
 // distances between the edges are decided by NEXT's expression.
 constexpr double kBandLow = (1.0 - 2e-6) / (1.0 + 2.2e-6);
 
-// Accepted nodes a lane holds (a ring in LDS), and how many of each lane's
-// oldest entries one evaluation round takes.  Evaluating only the oldest
-// entries when some lane's ring is full keeps more lanes busy per
-// evaluation step than draining every ring: lanes fill at different rates.
-// The walk is bound by the latency of its dependent node loads, so resident
-// waves count: 24 entries (6 KB of LDS per wave) with the registers held to
-// 80 (a few spills outside the loops) give 6 waves per SIMD, 6 % faster
-// than 32 entries at 5; 20 entries at 7 waves (17 spills) were slower, and so
-// were 16 (fewer lanes busy per evaluation step) and 64 (2.5 waves).
-constexpr int kWalkList = 24;
-// One wave per workgroup: a wave's registers and LDS are released as soon as
-// its group is done instead of when the slowest wave of a larger workgroup
-// is (measured 2.39 -> 2.34 ms against four waves per workgroup).
-constexpr int kWalkBlock = 64;
-constexpr int kWalkFlush = 4;
-static_assert(kWalkFlush <= kWalkList, "walk ring");
+// The walk.  One wave per group of up to 64 targets (fewer targets: 64 / width
+// lanes on each), three parts:
+//  - Group traversal.  Each lane tests another node against the group's box:
+//    a node that every target accepts goes to a list, one that every target
+//    opens is descended (the rest of the lane's preorder range handed to idle
+//    lanes through a stack in LDS), and a subtree on which the targets may
+//    differ goes to a second list.  About 26 wave steps per group of 64.
+//  - Nodes the whole group accepts (44 of a target's 174 on the cold sphere
+//    of 2^20 bodies): with one lane per target their records come in by
+//    scalar loads, every lane busy.
+//  - The mixed subtrees: each lane walks them on its own with NEXT's test
+//    (192 lane steps for 130 accepted nodes), so the wave's steps are its
+//    slowest lane's visits, not the union of all lanes' (725 of which 28 % of
+//    lanes decided anything), and nothing waits in a ring.
+// Each target's terms are NEXT's; they are added in another order than
+// NEXT's recursion (group part first).  Measured, walk per step, against one
+// union traversal per 64 targets with deferred evaluation: cold sphere 2^20
+// 1.69 -> 1.31 ms; 200,003 bodies at theta 0.3, a tenth dark matter 2.83 ->
+// 0.83; Plummer 16,384 0.37 -> 0.11; 50,021 with a fifth dark matter 0.82 ->
+// 0.16.  Bound at 2^20 by the lanes' record loads: the texture units are busy
+// 88 % of the time and the vector cache misses 38 % of its lines (16 waves of
+// some 80 KB each on 32 KB), VALU 45 %.  Loading the records cooperatively (4
+// lanes per record, through LDS, by DMA or registers) cut the accesses by a
+// third and was as fast (1.29-1.34), several waves per workgroup and lanes
+// kept to windows of the list were slower, and so are 5 or 6 waves per SIMD
+// (1.36, 1.43; 6 and more registers spilled) instead of 4.
+constexpr int kWalkStack = 64;     // donated node ranges per wave (a full stack only means a lane keeps its range)
+constexpr int kWalkCommon = 192;   // nodes the whole group accepts, per flush
+constexpr int kWalkMixed = 192;    // subtrees on which the group's targets differ, per flush
+static_assert(kWalkCommon > kWave && kWalkMixed > kWave, "a wave step appends up to 64 entries");
 
-// Node records come in through the scalar cache: the traversal loads one
-// 32-byte WalkHead per visited node, the evaluation a lane's accepted
-// records by vector loads.  Loading the next entry's record while the
-// current one is evaluated measured slower (it costs the registers of a
-// sixth wave).
-//
-// Two phases per wave.  Traversal: every lane follows its own depth-first
-// path (open: go to the first child, cur+1; accept or skip: go past the
-// subtree, skip[cur]).  The wave visits node `cur` and the lanes whose own
-// next node is `cur` decide it.  No lane that is waiting can point inside
-// cur's subtree (its pointer came from a skip of an ancestor or an earlier
-// sibling, both of which end at or after skip[cur]), so the wave's next node
-// is cur+1 when any lane opened cur and skip[cur] otherwise: one ballot, no
-// reduction.  An accepted node is only appended to the lane's ring in LDS.
-// Evaluation: when some lane's ring is full, the wave evaluates up to
-// kWalkFlush of every lane's oldest entries in step, entry k of every lane
-// at once (and everything at the end), so the costly interaction (two square
-// roots, two divides, the quadrupole) runs with most lanes busy instead of
-// only the lanes that accepted the node being visited.  Each lane still adds
-// its interactions in its own depth-first order, the order of
-// octree.h:158-177, so the sums are NEXT's bit for bit.
-//
-// Opening test of octree.h:153, (size/dist) < theta with
-// dist = sqrt(r2 + 1e-20): decided from r2 against the node's FP32 band
-// edges around (size/theta)^2 - 1e-20 (relative width about 4e-6; rounding
-// errors of either form are below 1e-15), and by NEXT's exact expression
-// inside the band, so the decision is NEXT's bit for bit and opened nodes
-// cost no sqrt or divide.
-template <bool KICK, bool COUNT>
-__global__ __launch_bounds__(kWalkBlock) __attribute__((amdgpu_waves_per_eu(6)))
-void k_walk(const Group* __restrict__ groups, int64_t ngroups,
-                                                 const RefNode* __restrict__ nodes,
-                                                 const WalkHead* __restrict__ heads, StateArrays st, SysArrays sy,
-                                                 double theta, double* __restrict__ ax, double* __restrict__ ay,
-                                                 double* __restrict__ az, DevScalars* sc) {
-  __shared__ int32_t lists[kWalkBlock / kWave][kWalkList][kWave];
-  // kWalkBlock / 64 waves per block, one group per wave.  The wave index goes through
-  // readfirstlane so the compiler sees it as wave-uniform: the group, its
-  // system's tree bounds and every node visited are then uniform too, and
-  // the node records come in through scalar loads into scalar registers.
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-  const int64_t gi = xcd_block(gridDim.x) * (kWalkBlock / kWave) + wave;
-  if (gi >= ngroups || sc->abort_flags) return;            // whole wave past the end, or an aborted build
-  int32_t* const mine = &lists[wave][0][lane_id()];      // ring slot k at mine[k * kWave]
-  const Group g = groups[gi];
-  const int64_t i = g.first + lane_id();
-  const bool valid = lane_id() < g.count;
-  const int32_t total = sy.send[g.sys];                    // this system's tree: [sroot, send)
-  double px = 0, py = 0, pz = 0, pm = 1;
-  int pt = 0;
-  if (valid) { px = st.x[i]; py = st.y[i]; pz = st.z[i]; pm = st.m[i]; pt = st.type[i]; }
-  const int32_t self_link = valid ? ~(int32_t)i : INT_MAX;   // link of this lane's own leaf
-  double a0 = 0.0, a1 = 0.0, a2 = 0.0;
-  uint32_t npp = 0, npc = 0, nop = 0, nit = 0, nev = 0;
-  int ws = 0, len = 0;                                     // this lane's ring: next free slot, entries before it
-  const uint32_t zoff = (uint32_t)sc->total_nodes << 7;   // the all-zero record (k_emit)
+// The running sums of a target.
+struct Sum3 { double x, y, z; };
 
-  // Evaluate up to `limit` of the oldest entries (octree.h:139-176 for an
-  // accepted node); an entry is the node index, with bit 31 set for a leaf
-  // (Q = 0).  DM: some target of the wave is dark matter (its softening
-  // floor, octree.h:146-148, is a call); without one the loop is straight
-  // code.
-  auto evaluate = [&](auto dm, int limit) {
-    const int take = len < limit ? len : limit;
-    int rs = ws - len;                                     // the oldest entry's slot
-    if (rs < 0) rs += kWalkList;
-    for (int k = 0; __builtin_amdgcn_ballot_w64(k < take); ++k) {
-      if (COUNT) ++nev;
-      // Every lane runs every round: a lane with no entry left reads the
-      // all-zero record after the last node, and so does a leaf entry for
-      // its quadrupole (leaf records carry none); both add exact zeros
-      // (m = 0, Q = 0, every factor finite).  Byte offsets: e << 7 drops
-      // the leaf bit.
-      const int32_t e = mine[rs * kWave];
-      rs = rs == kWalkList - 1 ? 0 : rs + 1;
-      const bool on = k < take;
-      const uint32_t off = on ? (uint32_t)e << 7 : zoff;
-      const uint32_t qoff = (on && e >= 0) ? off : zoff;
-      const RefNode* nd = reinterpret_cast<const RefNode*>(reinterpret_cast<const char*>(nodes) + off);
-      const RefNode* qn = reinterpret_cast<const RefNode*>(reinterpret_cast<const char*>(nodes) + qoff);
-      const double dx = nd->cx - px, dy = nd->cy - py, dz = nd->cz - pz;
-      const double m = nd->m;
-      // octree.h:139-172 with products fused into FMAs and the square
-      // roots and divides faithfully rounded (a few ulp per interaction):
-      // r2 = |d|^2, dist = sqrt(r2 + 1e-20), eps from softening.h:26-36,
-      // dinv = 1/sqrt(r2 + eps^2).
-      const double r2 = __builtin_fma(dz, dz, __builtin_fma(dy, dy, dx * dx));
-      const double r2e = r2 + 1e-20;
-      const double dist = r2e * rsq_nr(r2e);
-      double eps = nd->esum * rcp_nr(__builtin_fma(dist, 10.0, 1.0));
-      if (eps < 1e-4) eps = 1e-4;
-      if (decltype(dm)::value && pt == 1) eps = dm_softening(eps, nd->size, m, pm);   // octree.h:146-148
-      const double dinv = rsq_nr(__builtin_fma(eps, eps, r2));
-      const double inv2 = dinv * dinv;
-      const double inv3 = inv2 * dinv;
-      const double inv5 = inv3 * inv2;
-      const double inv7 = inv5 * inv2;
-      // quadrupole term 0.5 (2 (Q d) inv5 - 5 q inv7 d), q = d.Q.d
-      // (octree.h:159-172), as (Q d) inv5 + d (-(2.5 q) inv7)
-      const double qxx = qn->qxx, qyy = qn->qyy, qzz = qn->qzz;
-      const double qxy = qn->qxy, qxz = qn->qxz, qyz = qn->qyz;
-      const double sx = __builtin_fma(qxz, dz, __builtin_fma(qxy, dy, qxx * dx));
-      const double sy = __builtin_fma(qyz, dz, __builtin_fma(qyy, dy, qxy * dx));
-      const double sz = __builtin_fma(qzz, dz, __builtin_fma(qyz, dy, qxz * dx));
-      const double q = __builtin_fma(dz, sz, __builtin_fma(dy, sy, dx * sx));
-      const double c = __builtin_fma(-2.5 * q, inv7, m * inv3);   // G = 1
-      a0 = __builtin_fma(dx, c, __builtin_fma(sx, inv5, a0));
-      a1 = __builtin_fma(dy, c, __builtin_fma(sy, inv5, a1));
-      a2 = __builtin_fma(dz, c, __builtin_fma(sz, inv5, a2));
-    }
-    len -= take;
-  };
-  // dark-matter targets in this wave (wave-uniform)
-  const bool any_dm = __builtin_amdgcn_ballot_w64(pt == 1) != 0;
-
-  const int32_t root = sy.sroot[g.sys];
-  int32_t next = valid ? root : INT_MAX;
-  int32_t cur = root;
-  HeadRegs h = load_head(heads, root);
-  // Traversal runs until some lane's ring is full (or the tree is done),
-  // then one evaluation round; the running sums are not touched inside the
-  // traversal loop, which keeps them out of its loop-carried registers.
-  for (;;) {
-    while (cur < total) {
-      // successors, loaded while this node is processed
-      // (the node array has one spare record after the last node, so both
-      // successors, at most total, are readable)
-      const bool leaf = h.link < 0;
-      const int32_t lk = leaf ? cur + 1 : (h.link & ~kLinkZeroMass);
-      const int32_t sk = lk > cur ? lk : cur + 1;           // skip > cur by construction
-      const HeadRegs h1 = load_head(heads, (uint32_t)cur + 1u);
-      const HeadRegs h2 = load_head(heads, (uint32_t)sk);
-      // This lane decides cur if its own path is at cur.  The decision is
-      // formed without branching on it: every lane computes the test, and
-      // every lane writes cur into its ring's free slot ws (each ring holds
-      // fewer than kWalkList entries inside this loop), which becomes an
-      // entry only if the lane accepts.
-      const bool here = next == cur;
-      const bool pass = (h.link >= 0 && (h.link & kLinkZeroMass)) || h.link == self_link;   // octree.h:134-135
-      bool accept = leaf;
-      if (!leaf) {                                            // wave-uniform
-        const double dx = h.cx - px, dy = h.cy - py, dz = h.cz - pz;
-        // Against the band edges (for r^2, about 4e-6 wide) any rounding of
-        // r^2 decides alike: FMAs here, NEXT's expression, as NEXT rounds
-        // it, inside the band.
-        const double r2f = __builtin_fma(dz, dz, __builtin_fma(dy, dy, dx * dx));
-        const double hi = (double)__uint_as_float(h.acc2_bits);   // NaN: no fast decision
-        accept = r2f > hi;
-        const bool band = here && !accept && !(r2f < hi * kBandLow);
-        if (band) {                                           // rare: NEXT's exact expression
-          const double r2e = (dx * dx + dy * dy + dz * dz) + 1e-20;
-          accept = (nodes[cur].size / sqrt(r2e)) < theta;
-        }
-      }
-      const bool take = here && !pass && accept;
-      const bool open = here && !pass && !accept;
-      mine[ws * kWave] = leaf ? (int32_t)(cur | 0x80000000u) : cur;
-      const int tk = take ? 1 : 0;
-      len += tk;
-      ws += tk;
-      if (ws == kWalkList) ws = 0;
-      // an opening lane is here (next == cur): its next node is next + 1
-      const int op = open ? 1 : 0;
-      next = (here && !open) ? sk : next + op;
-      if (COUNT) {
-        npp += (take && leaf) ? 1u : 0u;
-        npc += (take && !leaf) ? 1u : 0u;
-        nop += open ? 1u : 0u;
-      }
-      if (COUNT) ++nit;
-      if (__builtin_amdgcn_ballot_w64(op != 0)) { cur = cur + 1; h = h1; }
-      else { cur = sk; h = h2; }
-      if (__builtin_amdgcn_ballot_w64(len == kWalkList)) break;
-    }
-    if (cur >= total) break;
-    if (any_dm) evaluate(std::true_type{}, kWalkFlush);
-    else evaluate(std::false_type{}, kWalkFlush);
+// One accepted node on one target (octree.h:139-172, G = 1): products fused
+// into FMAs and the square roots and divides faithfully rounded (a few ulp
+// per interaction).  d: node minus target, r2 = |d|^2 as the opening test
+// forms it; dist = sqrt(r2 + 1e-20), eps from softening.h:26-36, dinv =
+// 1/sqrt(r2 + eps^2).  DM: some target is dark matter: its softening floor
+// (octree.h:146-148) is 2 size / (m/mi)^p = dmk mi^p, with mip = mi^p for
+// a dark-matter target and 0 otherwise.  QUAD: the quadrupole term
+// 0.5 (2 (Q d) inv5 - 5 q inv7 d), q = d.Q.d, as (Q d) inv5 + d (-(2.5 q) inv7).
+template <bool DM, bool QUAD>
+__device__ __forceinline__ void interact(double dx, double dy, double dz, double r2, double m, double esum,
+                                         double dmk, double mip, double qxx, double qyy, double qzz, double qxy,
+                                         double qxz, double qyz, Sum3& a) {
+  const double r2e = r2 + 1e-20;
+  const double dist = r2e * rsq_nr(r2e);
+  double eps = esum * rcp_nr(__builtin_fma(dist, 10.0, 1.0));
+  if (eps < 1e-4) eps = 1e-4;
+  if (DM) {
+    const double alt = dmk * mip;
+    if (eps < alt) eps = alt;
   }
-  if (any_dm) evaluate(std::true_type{}, kWalkList);
-  else evaluate(std::false_type{}, kWalkList);
-  (void)h;
+  const double dinv = rsq_nr(__builtin_fma(eps, eps, r2));
+  const double inv2 = dinv * dinv;
+  const double inv3 = inv2 * dinv;
+  if (QUAD) {
+    const double inv5 = inv3 * inv2;
+    const double inv7 = inv5 * inv2;
+    const double sx = __builtin_fma(qxz, dz, __builtin_fma(qxy, dy, qxx * dx));
+    const double sy = __builtin_fma(qyz, dz, __builtin_fma(qyy, dy, qxy * dx));
+    const double sz = __builtin_fma(qzz, dz, __builtin_fma(qyz, dy, qxz * dx));
+    const double q = __builtin_fma(dz, sz, __builtin_fma(dy, sy, dx * sx));
+    const double c = __builtin_fma(-2.5 * q, inv7, m * inv3);
+    a.x = __builtin_fma(dx, c, __builtin_fma(sx, inv5, a.x));
+    a.y = __builtin_fma(dy, c, __builtin_fma(sy, inv5, a.y));
+    a.z = __builtin_fma(dz, c, __builtin_fma(sz, inv5, a.z));
+  } else {
+    const double c = m * inv3;
+    a.x = __builtin_fma(dx, c, a.x);
+    a.y = __builtin_fma(dy, c, a.y);
+    a.z = __builtin_fma(dz, c, a.z);
+  }
+}
+
+__device__ __forceinline__ const RefNode& node_at(const RefNode* nodes, uint32_t off) {
+  return *reinterpret_cast<const RefNode*>(reinterpret_cast<const char*>(nodes) + off);
+}
+
+// Nodes every target of the group accepts (bit 31: a leaf, which carries no
+// quadrupole).  One lane per target (parts == 1): the entry is wave-uniform,
+// so its record comes in through scalar loads and every lane is busy.  With
+// more lanes per target, each part takes every parts-th entry.
+template <bool DM>
+__device__ __forceinline__ void walk_common(const int32_t* list, int n, int part, int parts,
+                                            const RefNode* __restrict__ nodes, uint32_t zoff, double px, double py,
+                                            double pz, double mip, Sum3& a) {
+  if (parts == 1) {
+#pragma unroll 2
+    for (int k = 0; k < n; ++k) {
+      const int32_t e = __builtin_amdgcn_readfirstlane(list[k]);
+      const RefNode& nd = node_at(nodes, (uint32_t)e << 7);
+      const double dx = nd.cx - px, dy = nd.cy - py, dz = nd.cz - pz;
+      const double r2 = __builtin_fma(dz, dz, __builtin_fma(dy, dy, dx * dx));
+      if (e < 0)
+        interact<DM, false>(dx, dy, dz, r2, nd.m, nd.esum, nd.dmk, mip, 0, 0, 0, 0, 0, 0, a);
+      else
+        interact<DM, true>(dx, dy, dz, r2, nd.m, nd.esum, nd.dmk, mip, nd.qxx, nd.qyy, nd.qzz, nd.qxy, nd.qxz,
+                           nd.qyz, a);
+    }
+  } else {
+    for (int k = part; k < n; k += parts) {
+      const int32_t e = list[k];
+      const uint32_t off = (uint32_t)e << 7;
+      const RefNode& nd = node_at(nodes, off);
+      const RefNode& qn = node_at(nodes, e < 0 ? zoff : off);
+      const double dx = nd.cx - px, dy = nd.cy - py, dz = nd.cz - pz;
+      const double r2 = __builtin_fma(dz, dz, __builtin_fma(dy, dy, dx * dx));
+      interact<DM, true>(dx, dy, dz, r2, nd.m, nd.esum, nd.dmk, mip, qn.qxx, qn.qyy, qn.qzz, qn.qxy, qn.qxz, qn.qyz,
+                         a);
+    }
+  }
+}
+
+// Subtrees on which the group's targets differ: every lane walks them on its
+// own, with its own target's opening test, and evaluates a node as it
+// accepts it.  The next node's head is loaded while the accepted node is
+// evaluated.
+template <bool DM, bool COUNT>
+__device__ __forceinline__ void walk_mixed(const int32_t* list, int n, bool valid, int part, int parts, int32_t self,
+                                           const RefNode* __restrict__ nodes, const WalkHead* __restrict__ heads,
+                                           uint32_t zoff, double theta, double px, double py, double pz, double mip,
+                                           Sum3& a, uint32_t& npp, uint32_t& npc, uint32_t& nop, uint32_t& nit) {
+  int k = part;
+  bool live = valid && k < n;
+  int32_t cur = live ? list[k] : 0, root = cur, end = 0;
+  WalkHead h = heads[cur];
+  while (live) {
+    const bool leaf = h.link < 0;
+    int32_t skip = leaf ? cur + 1 : (h.link & ~kLinkZeroMass);
+    if (skip <= cur) skip = cur + 1;                         // skip > cur by construction
+    if (cur == root) end = skip;
+    const double dx = h.cx - px, dy = h.cy - py, dz = h.cz - pz;
+    const double r2 = __builtin_fma(dz, dz, __builtin_fma(dy, dy, dx * dx));
+    // octree.h:134-135: massless nodes and the target itself
+    const bool pass = (h.link >= 0 && (h.link & kLinkZeroMass)) || h.link == self;
+    bool accept = leaf;
+    if (!leaf) {
+      // Against the band edges (about 4e-6 wide) any rounding of r^2 decides
+      // alike: FMAs here, NEXT's expression, as NEXT rounds it, inside.
+      const double hi = (double)h.acc2;                      // NaN: no fast decision
+      accept = r2 > hi;
+      if (!accept && !(r2 < hi * kBandLow)) {                // rare
+        const double r2e = (dx * dx + dy * dy + dz * dz) + 1e-20;
+        accept = (nodes[cur].size / sqrt(r2e)) < theta;
+      }
+    }
+    const bool take = !pass && accept;
+    int32_t next = (pass || accept) ? skip : cur + 1;
+    if (COUNT) {
+      npp += (take && leaf) ? 1u : 0u;
+      npc += (take && !leaf) ? 1u : 0u;
+      nop += (!pass && !accept) ? 1u : 0u;
+      nit += 1u;
+    }
+    if (next >= end) {                                       // this subtree is done
+      k += parts;
+      live = k < n;
+      next = live ? list[k] : 0;
+      root = next;
+    }
+    const WalkHead hn = heads[next];
+    if (take) {
+      const uint32_t off = (uint32_t)cur << 7;
+      const RefNode& nd = node_at(nodes, off);
+      const RefNode& qn = node_at(nodes, leaf ? zoff : off);
+      interact<DM, true>(dx, dy, dz, r2, nd.m, nd.esum, nd.dmk, mip, qn.qxx, qn.qyy, qn.qzz, qn.qxy, qn.qxz, qn.qyz,
+                         a);
+    }
+    cur = next;
+    h = hn;
+  }
+}
+
+template <bool KICK, bool COUNT>
+__global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(4)))
+void k_walk(const Group* __restrict__ groups, int64_t ngroups, const RefNode* __restrict__ nodes,
+            const WalkHead* __restrict__ heads, StateArrays st, SysArrays sy, double theta, double* __restrict__ ax,
+            double* __restrict__ ay, double* __restrict__ az, DevScalars* sc) {
+  __shared__ int32_t stk_b[kWalkStack], stk_e[kWalkStack];   // donated ranges [stk_b, stk_e)
+  __shared__ int32_t common[kWalkCommon], mixed[kWalkMixed];
+  const int64_t gi = xcd_block(gridDim.x);
+  if (gi >= ngroups || sc->abort_flags) return;            // past the end, or an aborted build
+  const int lane = threadIdx.x;
+  const Group g = groups[gi];
+  int width = kWave;
+  while (width > 1 && (width >> 1) >= g.count) width >>= 1;
+  const int parts = kWave / width;
+  const int slot = lane & (width - 1), part = lane / width;
+  const bool valid = slot < g.count;
+  const int64_t i = g.first + (valid ? slot : 0);
+  const double px = st.x[i], py = st.y[i], pz = st.z[i], pm = st.m[i];
+  const bool dark = valid && st.type[i] == 1;
+  const double mip = dark ? dm_power(pm, cbrt(pm)) : 0.0;
+  const bool any_dm = __ballot(dark) != 0;
+  const int32_t self = ~(int32_t)i;                          // link of this target's own leaf
+  const uint64_t ltmask = lanemask_lt();
+  const uint32_t zoff = (uint32_t)sc->total_nodes << 7;      // the all-zero record (k_emit)
+
+  // The group's box.
+  double lo[3] = {px, py, pz}, hi[3] = {px, py, pz};
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) {
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      lo_upd(lo[k], __shfl_xor(lo[k], off, kWave));
+      hi_upd(hi[k], __shfl_xor(hi[k], off, kWave));
+    }
+  }
+
+  Sum3 a{0.0, 0.0, 0.0};
+  uint32_t npp = 0, npc = 0, nop = 0, nit = 0, nev = 0, nlane = 0;
+  int nc = 0, nm = 0, sp = 0;
+  auto flush_common = [&]() {
+    __syncthreads();
+    if (any_dm) walk_common<true>(common, nc, part, parts, nodes, zoff, px, py, pz, mip, a);
+    else walk_common<false>(common, nc, part, parts, nodes, zoff, px, py, pz, mip, a);
+    if (COUNT) nev += (nc + parts - 1) / parts;
+    __syncthreads();
+    nc = 0;
+  };
+  auto flush_mixed = [&]() {
+    __syncthreads();
+    uint32_t steps = 0;
+    if (any_dm)
+      walk_mixed<true, COUNT>(mixed, nm, valid, part, parts, self, nodes, heads, zoff, theta, px, py, pz, mip, a, npp,
+                              npc, nop, steps);
+    else
+      walk_mixed<false, COUNT>(mixed, nm, valid, part, parts, self, nodes, heads, zoff, theta, px, py, pz, mip, a,
+                               npp, npc, nop, steps);
+    if (COUNT) {
+#pragma unroll
+      for (int off = 32; off >= 1; off >>= 1) {
+        const uint32_t o = __shfl_xor(steps, off, kWave);
+        steps = o > steps ? o : steps;
+      }
+      nlane += steps;
+    }
+    __syncthreads();
+    nm = 0;
+  };
+
+  const int32_t root = sy.sroot[g.sys], total = sy.send[g.sys];   // this system's tree
+  int32_t cur = lane == 0 ? root : total, end = total;
+  for (;;) {
+    // idle lanes take ranges from the top of the stack
+    const bool idle = cur >= end;
+    const uint64_t im = __ballot(idle);
+    const int avail = (int)__popcll(im);
+    const int give = avail < sp ? avail : sp;
+    if (idle) {
+      const int r = (int)__popcll(im & ltmask);
+      if (r < give) { cur = stk_b[sp - 1 - r]; end = stk_e[sp - 1 - r]; }
+    }
+    sp -= give;
+    const bool busy = cur < end;
+    if (!__ballot(busy)) break;
+    if (COUNT) ++nit;
+    if (nc > kWalkCommon - kWave) flush_common();
+    if (nm > kWalkMixed - kWave) flush_mixed();
+    bool acc = false, mix = false, donate = false, leaf = false, opened = false;
+    int32_t skip = 0;
+    if (busy) {
+      const WalkHead h = heads[cur];
+      leaf = h.link < 0;
+      skip = leaf ? cur + 1 : (h.link & ~kLinkZeroMass);
+      if (skip <= cur) skip = cur + 1;
+      const bool zero = h.link >= 0 && (h.link & kLinkZeroMass);
+      if (leaf) {
+        const int32_t body = ~h.link;
+        mix = body >= g.first && body < g.first + g.count;   // some target's own leaf
+        acc = !mix;
+      } else if (!zero) {
+        // |fl(c - p)| lies between the distances of the box's near and far
+        // faces (rounding is monotone), and so does r^2, formed alike: a
+        // decision outside the band for both faces is every target's.
+        const double nx = fmax(fmax(lo[0] - h.cx, h.cx - hi[0]), 0.0), fx = fmax(h.cx - lo[0], hi[0] - h.cx);
+        const double ny = fmax(fmax(lo[1] - h.cy, h.cy - hi[1]), 0.0), fy = fmax(h.cy - lo[1], hi[1] - h.cy);
+        const double nz = fmax(fmax(lo[2] - h.cz, h.cz - hi[2]), 0.0), fz = fmax(h.cz - lo[2], hi[2] - h.cz);
+        const double r2n = __builtin_fma(nz, nz, __builtin_fma(ny, ny, nx * nx));
+        const double r2f = __builtin_fma(fz, fz, __builtin_fma(fy, fy, fx * fx));
+        const double e = (double)h.acc2;                     // NaN: mixed
+        acc = r2n > e;
+        opened = r2f < e * kBandLow;
+        mix = !acc && !opened;
+        donate = opened && skip < end;
+      }
+    }
+    const uint64_t am = __ballot(acc), mm = __ballot(mix), dm = __ballot(donate);
+    if (acc) common[nc + (int)__popcll(am & ltmask)] = leaf ? (int32_t)(cur | 0x80000000u) : cur;
+    if (mix) mixed[nm + (int)__popcll(mm & ltmask)] = cur;
+    nc += (int)__popcll(am);
+    nm += (int)__popcll(mm);
+    if (COUNT) {
+      if (acc) { if (leaf) npp += g.count; else npc += g.count; }
+      if (opened) nop += g.count;
+    }
+    // opened nodes hand [skip, end) to the stack while it has room
+    const int room = kWalkStack - sp;
+    if (donate) {
+      const int r = (int)__popcll(dm & ltmask);
+      if (r < room) { stk_b[sp + r] = skip; stk_e[sp + r] = end; end = skip; }
+    }
+    sp += (int)__popcll(dm) < room ? (int)__popcll(dm) : room;
+    if (busy) cur = opened ? cur + 1 : skip;
+    __syncthreads();
+  }
+  if (nc) flush_common();
+  if (nm) flush_mixed();
+  for (int off = width; off < kWave; off <<= 1) {
+    a.x += __shfl_xor(a.x, off, kWave);
+    a.y += __shfl_xor(a.y, off, kWave);
+    a.z += __shfl_xor(a.z, off, kWave);
+  }
   double v2 = 0.0;
-  if (valid) {
-    ax[i] = a0; ay[i] = a1; az[i] = a2;
+  if (valid && part == 0) {
+    ax[i] = a.x; ay[i] = a.y; az[i] = a.z;
     if (KICK) {                                             // step.h:171-173
       const double half = sy.dt[g.sys] * 0.5;
-      const double vx = st.vx[i] + a0 * half;
-      const double vy = st.vy[i] + a1 * half;
-      const double vz = st.vz[i] + a2 * half;
+      const double vx = st.vx[i] + a.x * half;
+      const double vy = st.vy[i] + a.y * half;
+      const double vz = st.vz[i] + a.z * half;
       st.vx[i] = vx; st.vy[i] = vy; st.vz[i] = vz;
       v2 = vx * vx + vy * vy + vz * vz;
       if (!(v2 > 0.0)) v2 = 0.0;
@@ -879,16 +978,16 @@ void k_walk(const Group* __restrict__ groups, int64_t ngroups,
       const double o = __shfl_xor(v2, off, kWave);
       if (o > v2) v2 = o;
     }
-    if (lane_id() == 0 && v2 > 0.0) atomicMax(&sy.v2max[g.sys], (unsigned long long)__double_as_longlong(v2));
+    if (lane == 0 && v2 > 0.0) atomicMax(&sy.v2max[g.sys], (unsigned long long)__double_as_longlong(v2));
   }
   if (COUNT) {
-    const uint32_t sp = wave_sum_u32(npp), sc2 = wave_sum_u32(npc), so = wave_sum_u32(nop);
-    if (lane_id() == 0) {
-      atomicAdd(&sc->n_pp, (unsigned long long)sp);
+    const uint32_t sp2 = wave_sum_u32(npp), sc2 = wave_sum_u32(npc), so = wave_sum_u32(nop);
+    if (lane == 0) {
+      atomicAdd(&sc->n_pp, (unsigned long long)sp2);
       atomicAdd(&sc->n_pc, (unsigned long long)sc2);
       atomicAdd(&sc->n_open, (unsigned long long)so);
-      atomicAdd(&sc->n_iter, (unsigned long long)nit);
-      atomicAdd(&sc->n_eval, (unsigned long long)nev);
+      atomicAdd(&sc->n_iter, (unsigned long long)(nit + nlane));
+      atomicAdd(&sc->n_eval, (unsigned long long)(nev + nlane));
     }
   }
 }
@@ -1135,10 +1234,9 @@ void launch_walk(const Group* groups, int64_t ngroups, const RefNode* nodes, con
                  const SysArrays& sy, double theta, double* ax, double* ay, double* az, DevScalars* sc, bool kick,
                  bool count, hipStream_t s) {
   if (ngroups <= 0) return;
-  const int wpb = kWalkBlock / kWave;
-  const unsigned nb = (unsigned)(div_up(div_up(ngroups, wpb), 8) * 8);
+  const unsigned nb = (unsigned)(div_up(ngroups, 8) * 8);
 #define NBX_RW(K, C) \
-  hipLaunchKernelGGL((k_walk<K, C>), dim3(nb), dim3(kWalkBlock), 0, s, groups, ngroups, nodes, heads, st, sy, theta, \
+  hipLaunchKernelGGL((k_walk<K, C>), dim3(nb), dim3(kWave), 0, s, groups, ngroups, nodes, heads, st, sy, theta, \
                      ax, ay, az, sc)
   if (kick && count) NBX_RW(true, true);
   else if (kick) NBX_RW(true, false);

@@ -102,6 +102,23 @@ void launch_upward(const int32_t* level_list, const uint32_t* end_list, int64_t 
 void launch_upward_all(const int32_t* counts, const int32_t* level_list, const uint32_t* end_list, RefNode* nodes,
                        WalkHead* heads, double theta, const int32_t* sys, const double* root, hipStream_t s);
 void launch_fill_u32(int64_t n, uint32_t* a, uint32_t v, hipStream_t s);
+// Bodies per walk group of a system of n bodies, 8 to 64 (a group narrower
+// than 64 puts 64 / width lanes on each target).  It depends on the system
+// alone, so a system's sums are the same alone and in a batch.  Narrow
+// groups give a small system enough waves and short ones; wide groups share
+// more of the traversal.  Measured walk times (us, theta 0.5, Plummer), width
+// 64 / 32 / 16 / 8: n = 1,000 150 / 92 / 69 / 54; 4,000 182 / 118 / 82 / 67;
+// 16,000 196 / 148 / 108 / 92 (64 such systems in one batch 1,519 / 1,665 /
+// 1,832 / 2,358, so 16 there); 64,000 242 / 188 / 177 / 232; 128,000 299 / 294
+// / 319 / 387; 256,000 516 / 536 / 588 / 732; 2^20 (cold sphere) 1,359 / 1,403
+// / 1,636 / 2,256.  At theta 0.3 each target's own walk is long and 16 is
+// fastest or within 3 % of it from 32,000 bodies on (256,000: 1,981 / 1,719 /
+// 1,611 / 1,612).
+inline int32_t walk_width(int64_t n, double theta) {
+  if (n <= 4096) return 8;
+  if (n <= 98304 || theta < 0.4) return 16;
+  return n <= 196608 ? 32 : 64;
+}
 void launch_walk(const Group* groups, int64_t ngroups, const RefNode* nodes, const WalkHead* heads,
                  const StateArrays& st,
                  const SysArrays& sy, double theta, double* ax, double* ay, double* az, DevScalars* sc, bool kick,

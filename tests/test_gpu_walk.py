@@ -1,0 +1,74 @@
+"""The reference-mode walk at the sizes where its group width changes.
+
+The walk puts 64 / width lanes on each target of a group of `width` bodies;
+the width follows the system's size (8 up to 4,096 bodies, 16 up to 98,304,
+32 up to 196,608, then 64; 16 for larger systems below theta 0.4).
+Accelerations against the oracle's walk (octree.h:133-179) at the edges of
+those ranges and of a group, with dark-matter targets (octree.h:146-148).
+Tolerance: the accelerations' own, median <= 1e-12 and 99th percentile <=
+1e-10 relative (the terms are the same, their order and the last bits of the
+square roots differ: a few ulp each).
+"""
+import numpy as np
+import pytest
+
+import oracle_lib as orc
+from next_amd import ic
+from next_amd.nbx import Engine
+
+pytestmark = pytest.mark.gpu
+
+
+def check(p, theta, what):
+    with Engine(theta=theta) as e:
+        e.upload(p)
+        a = e.accel()
+    n = len(p)
+    tg = np.arange(n) if n <= 8192 else np.unique(np.concatenate(
+        [np.arange(128), n - 1 - np.arange(128), np.random.Generator(np.random.PCG64(5)).choice(n, 4096, False)]))
+    ao = orc.accel_subset(p.x, p.y, p.z, p.m, p.type, theta, tg.astype(np.int64))
+    d = np.linalg.norm(ao, axis=1)
+    err = np.linalg.norm(a[tg] - ao, axis=1) / np.where(d > 0, d, 1.0)
+    print(f"{what}: median {np.median(err):.2e} p99 {np.percentile(err, 99):.2e} max {err.max():.2e}", flush=True)
+    assert np.median(err) <= 1e-12 and np.percentile(err, 99) <= 1e-10
+
+
+@pytest.mark.parametrize("theta", [0.0, 0.3, 0.5, 0.9])
+@pytest.mark.parametrize("n", [1, 2, 7, 8, 9, 63, 64, 65, 257, 4095])
+def test_small(n, theta):
+    check(ic.plummer(n, seed=n, virial=None, type_fraction_dm=0.3), theta, f"n={n} theta={theta}")
+
+
+@pytest.mark.parametrize("n,theta", [(4096, 0.5), (4097, 0.5), (98304, 0.39), (98305, 0.4), (98305, 0.39),
+                                     (196608, 0.5), (196609, 0.5), (196609, 0.39)])
+def test_width_edges(n, theta):
+    check(ic.plummer(n, seed=3, virial=None, type_fraction_dm=0.1), theta, f"n={n} theta={theta}")
+
+
+@pytest.mark.parametrize("lo,hi", [(-30, 30), (-3, 3), (200, 210), (-210, -200)])
+def test_dark_matter_masses(lo, hi):
+    """Masses over many orders of magnitude (zero among them): the softening
+    floor's power of the mass ratio."""
+    rng = np.random.Generator(np.random.PCG64(11))
+    p = ic.plummer(600, seed=4, virial=None, type_fraction_dm=0.5)
+    p.m[:] = 10.0 ** rng.uniform(lo, hi, len(p))
+    p.m[::37] = 0.0
+    # a zero-mass dark-matter target divides by its mass (octree.h:146): its floor is zero
+    check(p, 0.5, f"masses 1e{lo}..1e{hi}")
+
+
+def test_theta_changes_the_width():
+    """A context whose theta moves across the width rule gives the forces of
+    a fresh context at that theta."""
+    p = ic.plummer(100000, seed=6, virial=None)
+    with Engine(theta=0.5) as e:
+        e.upload(p)
+        e.accel()
+        e.set_theta(0.35)
+        a = e.accel()
+        e.set_theta(0.5)
+        b = e.accel()
+    for theta, got in ((0.35, a), (0.5, b)):
+        with Engine(theta=theta) as f:
+            f.upload(p)
+            assert np.array_equal(got, f.accel())
