@@ -278,6 +278,43 @@ __global__ __launch_bounds__(kBlock) void k_gather_state(int64_t n, const uint32
   b.m[i] = a.m[p]; b.type[i] = a.type[p]; b.id[i] = a.id[p]; b.sys[i] = a.sys[p];
 }
 
+__global__ __launch_bounds__(kBlock) void k_set_ids(int64_t n, int32_t* __restrict__ id, int32_t id0,
+                                                    int32_t* __restrict__ sys, int32_t sys_no) {
+  const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+  if (i < n) { id[i] = id0 + (int32_t)i; sys[i] = sys_no; }
+}
+
+// inv[id[i] - base] = i for the indices in range.
+__global__ __launch_bounds__(kBlock) void k_out_index(int64_t cnt, const int32_t* __restrict__ id, int32_t base,
+                                                      uint32_t* __restrict__ inv) {
+  const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+  if (i >= cnt) return;
+  const int64_t j = (int64_t)id[i] - base;
+  if (j >= 0 && j < cnt) inv[j] = (uint32_t)i;
+}
+
+// The cnt slots hold a permutation exactly when some slot holds each index:
+// inv[j] (stale where no slot wrote it) must be a slot that holds j.
+__global__ __launch_bounds__(kBlock) void k_out_check(int64_t cnt, const int32_t* __restrict__ id, int32_t base,
+                                                      const uint32_t* __restrict__ inv, int32_t* bad) {
+  const int64_t j = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+  if (j >= cnt) return;
+  const uint32_t i = inv[j];
+  if (i >= (uint64_t)cnt || (int64_t)id[i] - base != j) *bad = 1;
+}
+
+__global__ __launch_bounds__(kBlock) void k_out_gather(int64_t j0, int64_t len, int64_t cnt,
+                                                       const uint32_t* __restrict__ inv, OutArrays src, int m,
+                                                       double* __restrict__ dst) {
+  const int64_t j = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+  if (j >= len) return;
+  const uint32_t i = inv[j0 + j];
+  if (i >= (uint64_t)cnt) return;                            // not a permutation (k_out_check)
+#pragma unroll
+  for (int k = 0; k < kOutArrays; ++k)
+    if (k < m) dst[k * len + j] = src.p[k][i];
+}
+
 __global__ __launch_bounds__(kBlock) void k_gather_sys(int64_t n, const uint32_t* __restrict__ perm,
                                                        const int32_t* __restrict__ sys, uint32_t* __restrict__ dst) {
   const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
@@ -1149,6 +1186,19 @@ void launch_keys_export(int64_t n, const StateArrays& st, const SysArrays& sy, u
 void launch_fix_runs(int64_t n, const StateArrays& st, const SysArrays& sy, uint64_t* key, uint64_t* key2,
                      uint32_t* amag, int lo, hipStream_t s) {
   if (n > 1) hipLaunchKernelGGL(k_fix_runs, dim3(grid_of(n)), dim3(kBlock), 0, s, n, st, sy, key, key2, amag, lo);
+}
+void launch_set_ids(int64_t n, int32_t* id, int32_t id0, int32_t* sys, int32_t sys_no, hipStream_t s) {
+  if (n > 0) hipLaunchKernelGGL(k_set_ids, dim3(grid_of(n)), dim3(kBlock), 0, s, n, id, id0, sys, sys_no);
+}
+void launch_out_index(int64_t cnt, const int32_t* id, int32_t base, uint32_t* inv, int32_t* bad, hipStream_t s) {
+  if (cnt <= 0) return;
+  hipLaunchKernelGGL(k_out_index, dim3(grid_of(cnt)), dim3(kBlock), 0, s, cnt, id, base, inv);
+  hipLaunchKernelGGL(k_out_check, dim3(grid_of(cnt)), dim3(kBlock), 0, s, cnt, id, base, inv, bad);
+}
+void launch_out_gather(int64_t j0, int64_t len, int64_t cnt, const uint32_t* inv, const OutArrays& src, int m,
+                       double* dst, hipStream_t s) {
+  if (len > 0 && m > 0)
+    hipLaunchKernelGGL(k_out_gather, dim3(grid_of(len)), dim3(kBlock), 0, s, j0, len, cnt, inv, src, m, dst);
 }
 void launch_iota(int64_t n, uint32_t* idx, hipStream_t s) {
   if (n > 0) hipLaunchKernelGGL(k_iota, dim3(grid_of(n)), dim3(kBlock), 0, s, n, idx);

@@ -102,6 +102,20 @@ void launch_upward(const int32_t* level_list, const uint32_t* end_list, int64_t 
 void launch_upward_all(const int32_t* counts, const int32_t* level_list, const uint32_t* end_list, RefNode* nodes,
                        WalkHead* heads, double theta, const int32_t* sys, const double* root, hipStream_t s);
 void launch_fill_u32(int64_t n, uint32_t* a, uint32_t v, hipStream_t s);
+// Upload indices id0, id0 + 1, ... and system number of n slots.
+void launch_set_ids(int64_t n, int32_t* id, int32_t id0, int32_t* sys, int32_t sys_no, hipStream_t s);
+// inv[j] = the slot (of cnt) that holds upload index base + j; *bad (host
+// memory, 0 before) is set unless the slots hold a permutation of [base, base
+// + cnt).
+void launch_out_index(int64_t cnt, const int32_t* id, int32_t base, uint32_t* inv, int32_t* bad, hipStream_t s);
+// Values of upload indices [j0, j0 + len) of m arrays, one array after
+// another, len values each, into dst (host memory the device can write).
+constexpr int kOutArrays = 6;
+struct OutArrays {
+  const double* p[kOutArrays];
+};
+void launch_out_gather(int64_t j0, int64_t len, int64_t cnt, const uint32_t* inv, const OutArrays& src, int m,
+                       double* dst, hipStream_t s);
 // Bodies per walk group of a system of n bodies, 8 to 64 (a group narrower
 // than 64 puts 64 / width lanes on each target).  It depends on the system
 // alone, so a system's sums are the same alone and in a batch.  Narrow

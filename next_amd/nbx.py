@@ -268,16 +268,16 @@ class Engine:
 
     def download_system(self, s: int):
         k = self.system_size(s)
-        out = [np.zeros(max(k, 1)) for _ in range(6)]
+        out = np.empty((6, max(k, 1)))
         self._check(lib().nbx_download_system(self._h, s, *out))
-        return np.stack([o[:k] for o in out])
+        return out[:, :k]
 
     def remove_system(self, s: int):
         k = self.system_size(s)
-        out = [np.zeros(max(k, 1)) for _ in range(6)]
+        out = np.empty((6, max(k, 1)))
         self._check(lib().nbx_remove_system(self._h, s, *out))
         self.n -= k
-        return np.stack([o[:k] for o in out])
+        return out[:, :k]
 
     def energy_systems(self, direct: bool = False):
         out = np.zeros(5 * max(self.num_systems(), 1))
@@ -285,9 +285,9 @@ class Engine:
         return out[: 5 * self.num_systems()].reshape(-1, 5)
 
     def download(self):
-        out = [np.zeros(max(self.n, 1)) for _ in range(6)]
+        out = np.empty((6, max(self.n, 1)))
         self._check(lib().nbx_download(self._h, *out))
-        return np.stack([o[: self.n] for o in out])
+        return out[:, : self.n]
 
     def adaptive_dt(self, base_dt: float) -> float:
         dt = C.c_double()
@@ -436,12 +436,12 @@ class Server:
     def wait(self, rid: int):
         """(state 6 x n, queue_ms, latency_ms)."""
         n = self._n.pop(rid)
-        out = [np.zeros(max(n, 1)) for _ in range(6)]
+        out = np.empty((6, max(n, 1)))
         tm = RequestTiming()
         st = lib().nbx_server_wait(self._h, rid, *out, C.byref(tm))
         if st != 0:
             raise NbxError(st, f"request {rid} failed")
-        return np.stack([o[:n] for o in out]), tm.queue_ms, tm.latency_ms
+        return out[:, :n], tm.queue_ms, tm.latency_ms
 
     def stats(self) -> dict:
         s = ServerStats()
