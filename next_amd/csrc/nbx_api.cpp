@@ -63,7 +63,7 @@ struct nbx_ctx {
   DBuf level_list, end_list;  // internal nodes by depth, and their skip targets
   DBuf scratch, dts, lvl_part;
   DBuf pnodes, paux, pot, epart, eout;     // physics-mode tree, moments, potential, energy
-  DBuf dacc;                  // forces of the diagnostic passes (potential, direct energy)
+  DBuf dacc, dpart;           // forces of the diagnostic passes (potential, direct sum), partial direct sums
   // systems
   std::vector<int64_t> sys_n;              // bodies per system
   DBuf s_root, s_dt, s_v2, s_soff, s_sroot, s_send;
@@ -214,7 +214,7 @@ void each_buf(nbx_ctx* c, F f) {
   for (DBuf* a : {c->acc, c->key, c->idx, c->key2, c->amag})
     for (int k = 0; k < (a == c->acc ? 3 : 2); ++k) f(a[k]);
   for (DBuf* b : {&c->lcp, &c->cnt_s, &c->nodes, &c->heads, &c->level_list, &c->end_list, &c->scratch, &c->dts,
-                  &c->lvl_part, &c->pnodes, &c->paux, &c->pot, &c->dacc, &c->epart, &c->eout, &c->s_root, &c->s_dt,
+                  &c->lvl_part, &c->pnodes, &c->paux, &c->pot, &c->dacc, &c->dpart, &c->epart, &c->eout, &c->s_root, &c->s_dt,
                   &c->s_v2, &c->s_soff, &c->s_sroot, &c->s_send, &c->groups, &c->boxes, &c->box_off, &c->box_part,
                   &c->tgroups, &c->gmarks, &c->snap_amag})
     f(*b);
@@ -1546,20 +1546,29 @@ nbx_status nbx_potential(nbx_ctx* c, double* pot) {
   return copy_out(c, 0, c->n, 0, dev, &pot, 1);
 }
 
+// Direct-sum forces and potentials into the diagnostic buffers.
+static nbx_status direct_forces(nbx_ctx* c) {
+  const size_t n = (size_t)c->n;
+  NBXCHK(ensure(c, c->pot, n * 8));
+  NBXCHK(ensure(c, c->dacc, n * 3 * 8));
+  const int splits = direct_splits(c->n);
+  if (splits > 1) NBXCHK(ensure(c, c->dpart, (size_t)splits * 4 * n * 8));
+  double* da = P<double>(c->dacc);
+  launch_direct64(c->n, view(c, c->cur), sysa(c), c->cfg.eps, P<double>(c->dpart), da, da + n, da + 2 * n,
+                  P<double>(c->pot), c->stream);
+  HIPCHK(c, hipGetLastError());
+  return NBX_OK;
+}
+
 nbx_status nbx_direct(nbx_ctx* c, double* ax, double* ay, double* az, double* pot) {
   NBXCHK(check_ctx(c));
   if (c->n == 0) return NBX_OK;
   if (!(c->cfg.eps >= 0.0)) return fail(c, NBX_ERR_ARG, "negative softening");
-  DBuf tmp;
-  NBXCHK(ensure(c, tmp, (size_t)c->n * 8 * 4));
-  double* d = P<double>(tmp);
-  launch_direct64(c->n, view(c, c->cur), sysa(c), c->cfg.eps, d, d + c->n, d + 2 * c->n, d + 3 * c->n, c->stream);
-  const double* dev[4] = {d, d + c->n, d + 2 * c->n, d + 3 * c->n};
+  NBXCHK(direct_forces(c));
+  const double* d = P<double>(c->dacc);
+  const double* dev[4] = {d, d + c->n, d + 2 * c->n, P<double>(c->pot)};
   double* outs[4] = {ax, ay, az, pot};
-  const nbx_status st = copy_out(c, 0, c->n, 0, dev, outs, 4);
-  (void)hipStreamSynchronize(c->stream);
-  release(tmp);
-  return st;
+  return copy_out(c, 0, c->n, 0, dev, outs, 4);
 }
 
 nbx_status nbx_energy_systems(nbx_ctx* c, int source, double* out) {
@@ -1573,10 +1582,7 @@ nbx_status nbx_energy_systems(nbx_ctx* c, int source, double* out) {
   if (source == 0) {
     NBXCHK(tree_potential(c));
   } else {
-    NBXCHK(ensure(c, c->dacc, (size_t)c->n * 3 * 8));
-    double* da = P<double>(c->dacc);
-    launch_direct64(c->n, view(c, c->cur), sysa(c), c->cfg.eps, da, da + c->n, da + 2 * c->n, P<double>(c->pot),
-                    c->stream);
+    NBXCHK(direct_forces(c));
   }
   launch_energy(view(c, c->cur), P<double>(c->pot), P<BoxBlock>(c->boxes), c->nboxes, P<int32_t>(c->box_off), S,
                 P<double>(c->epart), P<double>(c->eout), c->stream);

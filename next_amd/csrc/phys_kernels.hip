@@ -602,47 +602,91 @@ __global__ __launch_bounds__(kPhysBlock) void k_phys_walk(const Group* __restric
   }
 }
 
-// FP64 direct sum: each thread owns one target; source bodies are staged
-// through LDS in tiles of one block.  Only bodies of the target's own system
-// act on it; the block loops over the union of its targets' systems.
-__global__ __launch_bounds__(kBlock) void k_direct64(int64_t n, StateArrays st, SysArrays sy, double e2,
-                                                     double* __restrict__ ax, double* __restrict__ ay,
-                                                     double* __restrict__ az, double* __restrict__ pot) {
-  __shared__ double sx[kBlock], sy_[kBlock], sz[kBlock], sm[kBlock];
-  __shared__ int32_t ss[kBlock];
-  const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+// FP64 direct sum.  One target per lane, 64 consecutive bodies per wave; the
+// sources are wave-uniform, so they come in by scalar loads and cost no LDS,
+// no barrier and no vector load.  blockIdx.y takes one of `splits` equal parts
+// of every system's sources, so that a small system fills the chip too; the
+// parts are summed in order by k_direct_sum.  A pair issues 18 FP64
+// instructions and v_rsq_f64 (one Newton step: a few ulp), so the sum is bound
+// by FP64 issue: 65,537 bodies 18.1 -> 3.3 ms per call against one target per thread
+// with sources staged in LDS, a correctly rounded square root and divide per
+// pair and 257 workgroups.
+//
+// Only bodies of the target's own system act on it: a wave whose targets lie
+// in several systems takes them one after another.  The lanes' own bodies are
+// among 64 sources only; the rest of the loop does not test for the self pair.
+constexpr int kDirectWaves = 4;    // waves per workgroup, each with its own 64 targets
+
+struct DirectSum { double x, y, z, p; };
+
+// Sources [j, end).  SELF: some of them are targets of the wave (body i of
+// this lane).  ZERO: eps is 0, so a pair at distance 0 has an infinite 1 / r.
+template <bool SELF, bool ZERO>
+__device__ __forceinline__ void direct_range(const StateArrays& st, int64_t j, int64_t end, int64_t i, double px,
+                                             double py, double pz, double e2, DirectSum& a) {
+  typedef const __attribute__((address_space(4))) double* cptr;   // scalar loads
+  const cptr X = (cptr)st.x, Y = (cptr)st.y, Z = (cptr)st.z, M = (cptr)st.m;
+#pragma unroll 4
+  for (; j < end; ++j) {
+    const double dx = X[j] - px, dy = Y[j] - py, dz = Z[j] - pz;
+    const double m = M[j];
+    const double r2 = fma(dz, dz, fma(dy, dy, fma(dx, dx, e2)));
+    const double y = __builtin_amdgcn_rsq(r2);
+    // (the minimum keeps inf * 0 out: an overflowing distance contributes 0)
+    double ri = fma(0.5 * y, fma(-(fmin(r2, 1.7976931348623157e308) * y), y, 1.0), y);
+    if (ZERO && r2 == 0.0) ri = INFINITY;
+    double mr = m * ri;
+    double mr3 = mr * (ri * ri);
+    if (SELF && j == i) { mr = 0.0; mr3 = 0.0; }
+    a.x = fma(dx, mr3, a.x);
+    a.y = fma(dy, mr3, a.y);
+    a.z = fma(dz, mr3, a.z);
+    a.p -= mr;
+  }
+}
+
+template <bool ZERO>
+__global__ __launch_bounds__(kDirectWaves* kWave) void k_direct64(int64_t n, StateArrays st, SysArrays sy, double e2,
+                                                                  int splits, double* __restrict__ ax,
+                                                                  double* __restrict__ ay, double* __restrict__ az,
+                                                                  double* __restrict__ pot) {
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int64_t i0 = ((int64_t)blockIdx.x * kDirectWaves + wave) * kWave;
+  if (i0 >= n) return;
+  const int64_t i1 = i0 + kWave < n ? i0 + kWave : n;        // targets [i0, i1)
+  const int64_t i = i0 + lane_id();
   const bool valid = i < n;
-  const int64_t last = ((int64_t)blockIdx.x + 1) * kBlock - 1 < n ? ((int64_t)blockIdx.x + 1) * kBlock - 1 : n - 1;
-  const int32_t me = valid ? st.sys[i] : -1;
-  const int64_t lo = sy.soff[st.sys[(int64_t)blockIdx.x * kBlock]];
-  const int64_t hi = sy.soff[st.sys[last] + 1];
-  const double px = valid ? st.x[i] : 0, py = valid ? st.y[i] : 0, pz = valid ? st.z[i] : 0;
-  double a0 = 0, a1 = 0, a2 = 0, p = 0;
-  for (int64_t t = lo; t < hi; t += kBlock) {
-    const int64_t j = t + threadIdx.x;
-    const bool in = j < hi;
-    sx[threadIdx.x] = in ? st.x[j] : 0;
-    sy_[threadIdx.x] = in ? st.y[j] : 0;
-    sz[threadIdx.x] = in ? st.z[j] : 0;
-    sm[threadIdx.x] = in ? st.m[j] : 0;
-    ss[threadIdx.x] = in ? st.sys[j] : -2;
-    __syncthreads();
-    const int lim = (int)(hi - t < kBlock ? hi - t : kBlock);
-    for (int k = 0; k < lim; ++k) {
-      if (t + k == i || ss[k] != me) continue;
-      const double dx = sx[k] - px, dy = sy_[k] - py, dz = sz[k] - pz;
-      const double r2 = dx * dx + dy * dy + dz * dz + e2;
-      const double ri = 1.0 / sqrt(r2);
-      const double mr3 = sm[k] * ri * ri * ri;
-      a0 += dx * mr3; a1 += dy * mr3; a2 += dz * mr3;
-      p -= sm[k] * ri;
+  const int64_t ii = valid ? i : n - 1;
+  const double px = st.x[ii], py = st.y[ii], pz = st.z[ii];
+  const int32_t me = st.sys[ii];
+  const int32_t s0 = __builtin_amdgcn_readfirstlane(st.sys[i0]), s1 = __builtin_amdgcn_readfirstlane(st.sys[i1 - 1]);
+  DirectSum a{0.0, 0.0, 0.0, 0.0};
+  for (int32_t s = s0; s <= s1; ++s) {
+    const int64_t lo = sy.soff[s], cnt = sy.soff[s + 1] - lo;
+    const int64_t b = lo + cnt * blockIdx.y / splits, e = lo + cnt * (blockIdx.y + 1) / splits;
+    if (me == s) {
+      const int64_t c0 = i0 < b ? b : i0 < e ? i0 : e, c1 = i1 < b ? b : i1 < e ? i1 : e;   // own targets in [b, e)
+      direct_range<false, ZERO>(st, b, c0, i, px, py, pz, e2, a);
+      direct_range<true, ZERO>(st, c0, c1, i, px, py, pz, e2, a);
+      direct_range<false, ZERO>(st, c1, e, i, px, py, pz, e2, a);
     }
-    __syncthreads();
   }
-  if (valid) {
-    ax[i] = a0; ay[i] = a1; az[i] = a2;
-    if (pot) pot[i] = p;
-  }
+  if (!valid) return;
+  const int64_t at = (splits > 1 ? (int64_t)blockIdx.y * 4 * n : 0) + i;   // parts: x y z p, n each
+  if (splits > 1) { ax[at] = a.x; ax[at + n] = a.y; ax[at + 2 * n] = a.z; ax[at + 3 * n] = a.p; }
+  else { ax[i] = a.x; ay[i] = a.y; az[i] = a.z; if (pot) pot[i] = a.p; }
+}
+
+__global__ __launch_bounds__(kBlock) void k_direct_sum(int64_t n, int splits, const double* __restrict__ part,
+                                                       double* __restrict__ ax, double* __restrict__ ay,
+                                                       double* __restrict__ az, double* __restrict__ pot) {
+  const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+  if (i >= n) return;
+  double v[4] = {0.0, 0.0, 0.0, 0.0};
+  for (int q = 0; q < splits; ++q)
+    for (int k = 0; k < 4; ++k) v[k] += part[((int64_t)q * 4 + k) * n + i];
+  ax[i] = v[0]; ay[i] = v[1]; az[i] = v[2];
+  if (pot) pot[i] = v[3];
 }
 
 // Energy and momentum per system, over the segmented blocks of the
@@ -794,11 +838,27 @@ void launch_phys_walk(const Group* groups, int64_t grid_groups, const PhysNode* 
                               th2, s);
 }
 
-void launch_direct64(int64_t n, const StateArrays& st, const SysArrays& sy, double eps, double* ax, double* ay,
-                     double* az, double* pot, hipStream_t s) {
-  if (n > 0)
-    hipLaunchKernelGGL(k_direct64, dim3(grid_of(n, kBlock)), dim3(kBlock), 0, s, n, st, sy, eps * eps, ax, ay, az,
-                       pot);
+// Parts of the sources: enough for 8 waves on each of the 1,024 SIMDs, of 64
+// sources or more.
+int direct_splits(int64_t n) {
+  const int64_t waves = div_up(std::max<int64_t>(n, 1), kWave);
+  return (int)std::max<int64_t>(1, std::min<int64_t>({8192 / waves, waves, 64}));
+}
+
+void launch_direct64(int64_t n, const StateArrays& st, const SysArrays& sy, double eps, double* part, double* ax,
+                     double* ay, double* az, double* pot, hipStream_t s) {
+  if (n <= 0) return;
+  const int splits = direct_splits(n);
+  const dim3 grid(grid_of(n, kDirectWaves * kWave), (unsigned)splits);
+  double* const ox = splits > 1 ? part : ax;
+  if (eps * eps > 0.0)
+    hipLaunchKernelGGL(k_direct64<false>, grid, dim3(kDirectWaves * kWave), 0, s, n, st, sy, eps * eps, splits, ox, ay,
+                       az, pot);
+  else
+    hipLaunchKernelGGL(k_direct64<true>, grid, dim3(kDirectWaves * kWave), 0, s, n, st, sy, eps * eps, splits, ox, ay,
+                       az, pot);
+  if (splits > 1)
+    hipLaunchKernelGGL(k_direct_sum, dim3(grid_of(n, kBlock)), dim3(kBlock), 0, s, n, splits, part, ax, ay, az, pot);
 }
 
 void launch_energy(const StateArrays& st, const double* pot, const BoxBlock* blocks, int nblocks,
