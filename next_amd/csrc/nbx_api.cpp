@@ -374,6 +374,19 @@ const uint64_t* sort_bodies(nbx_ctx* c, int digits, bool patch) {
   launch_bbox(St, P<BoxBlock>(c->boxes), c->nboxes, P<int32_t>(c->box_off), P<double>(c->box_part), sy, c->sc, s);
   launch_keys(n, St, sy, P<uint64_t>(c->key[0]), P<uint32_t>(c->idx[0]), c->sc, s);
   record(c, EV_KEYS);
+  if (S == 1 && n <= (patch ? kRankAlways : kRankSortMax)) {
+    const bool rel = c->amag_live;
+    launch_rank_sort(n, P<uint64_t>(c->key[0]), P<uint64_t>(c->key[1]), St, view(c, 1 - c->cur),
+                     rel ? P<uint32_t>(c->amag[c->acur]) : nullptr, rel ? P<uint32_t>(c->amag[1 - c->acur]) : nullptr,
+                     s);
+    c->sort_patched = false;
+    c->cur = 1 - c->cur;
+    if (rel) c->acur = 1 - c->acur;
+    launch_fix_runs(n, view(c, c->cur), sy, P<uint64_t>(c->key[1]), P<uint64_t>(c->key2[0]),
+                    rel ? P<uint32_t>(c->amag[c->acur]) : nullptr, 0, s);
+    record(c, EV_SORT);
+    return P<uint64_t>(c->key[1]);
+  }
   uint32_t* scr = P<uint32_t>(c->scratch);
   c->sort_patched = patch && S == 1;
   const int passes = digits > 0 && digits < kKeyDigits ? (3 * digits + 7) / 8 : 8;

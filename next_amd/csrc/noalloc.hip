@@ -31,6 +31,7 @@ namespace nbx {
 namespace {
 
 constexpr int64_t kNaBodies = NBX_NOALLOC_MAX_BODIES;
+static_assert(kNaBodies <= kRankSortMax, "one sort for every size");
 constexpr int64_t kNaNodes = NBX_NOALLOC_MAX_NODES;   // tree nodes, leaves included
 constexpr int64_t kNaGroups = (kNaBodies + 7) / 8;            // the narrowest walk groups hold 8 bodies
 constexpr int64_t kNaBoxes = (kNaBodies + kBoxSpan - 1) / kBoxSpan;
@@ -40,7 +41,7 @@ constexpr size_t align256(size_t b) { return (b + 255) & ~size_t(255); }
 // Byte offsets of every buffer inside the array, for kNaBodies bodies and
 // kNaNodes nodes.
 struct Layout {
-  size_t sc, st[2][10], acc[3], key[2], idx[2], key2[2], lcp, cnt_s, part, sortscr, nodes, heads, level_list, end_list;
+  size_t sc, st[2][10], acc[3], key[2], idx, key2, lcp, cnt_s, part, scanscr, nodes, heads, level_list, end_list;
   size_t root, dt, v2, soff, sroot, send, groups, boxes, box_off, box_part, total;
 };
 
@@ -52,18 +53,13 @@ constexpr Layout make_layout() {
   for (int w = 0; w < 2; ++w)
     for (int k = 0; k < 10; ++k) L.st[w][k] = take((size_t)kNaBodies * (k < 7 ? 8 : 4));
   for (int k = 0; k < 3; ++k) L.acc[k] = take((size_t)kNaBodies * 8);
-  for (int w = 0; w < 2; ++w) {
-    L.key[w] = take((size_t)kNaBodies * 8);
-    L.idx[w] = take((size_t)kNaBodies * 4);
-    L.key2[w] = take((size_t)kNaBodies * 8);
-  }
+  for (int w = 0; w < 2; ++w) L.key[w] = take((size_t)kNaBodies * 8);
+  L.idx = take((size_t)kNaBodies * 4);
+  L.key2 = take((size_t)kNaBodies * 8);
   L.lcp = take((size_t)kNaBodies * 4);
   L.cnt_s = take((size_t)kNaBodies * 4);
   L.part = take((size_t)(((kNaBodies + kBlock - 1) / kBlock) * kPartW) * 4);
-  const int64_t big = kNaBodies > kNaNodes ? kNaBodies : kNaNodes;
-  const size_t sw = sort_scratch_words(big);
-  const size_t cw = (size_t)((big + kScanTile - 1) / kScanTile + 2);
-  L.sortscr = take((sw > cw ? sw : cw) * 4);
+  L.scanscr = take(scan_scratch_words(kNaBodies) * 4);
   L.nodes = take((size_t)(kNaNodes + 1) * sizeof(RefNode));   // one all-zero record after the last node
   L.heads = take((size_t)(kNaNodes + 1) * sizeof(WalkHead));
   L.level_list = take((size_t)kNaNodes * 4);
@@ -179,7 +175,7 @@ nbx_status accel_in_arena(const Arena& A, int64_t n, const double* x, const doub
                           hipStream_t s) {
   DevScalars* sc = A.at<DevScalars>(kLayout.sc);
   SysArrays sy = A.sys();
-  uint32_t* scr = A.at<uint32_t>(kLayout.sortscr);
+  uint32_t* scr = A.at<uint32_t>(kLayout.scanscr);
   int cur = 0;
   StateArrays St = A.state(cur);
   const int64_t nb = (n + kBoxSpan - 1) / kBoxSpan;
@@ -191,21 +187,19 @@ nbx_status accel_in_arena(const Arena& A, int64_t n, const double* x, const doub
   launch_fill_scalars(sc, 1 | 4 | 8, s);
   launch_set_run(sc, 0, s);                                // no abort flag: the walk runs
   uint64_t* key[2] = {A.at<uint64_t>(kLayout.key[0]), A.at<uint64_t>(kLayout.key[1])};
-  uint32_t* idx[2] = {A.at<uint32_t>(kLayout.idx[0]), A.at<uint32_t>(kLayout.idx[1])};
-  uint64_t* key2[2] = {A.at<uint64_t>(kLayout.key2[0]), A.at<uint64_t>(kLayout.key2[1])};
-  launch_keys(n, St, sy, key[0], idx[0], sc, s);
-  const bool in1 = radix_sort_u64(key[0], idx[0], key[1], idx[1], n, 0, 63, scr, &sc->err, s);
-  launch_gather_state(n, idx[in1 ? 1 : 0], St, A.state(1 - cur), s);
+  uint64_t* key2 = A.at<uint64_t>(kLayout.key2);
+  launch_keys(n, St, sy, key[0], A.at<uint32_t>(kLayout.idx), sc, s);
+  launch_rank_sort(n, key[0], key[1], St, A.state(1 - cur), nullptr, nullptr, s);
   cur = 1 - cur;
   St = A.state(cur);
-  uint64_t* skey = key[in1 ? 1 : 0];
+  uint64_t* skey = key[1];
   int32_t* lcp = A.at<int32_t>(kLayout.lcp);
   uint32_t* cnt_s = A.at<uint32_t>(kLayout.cnt_s);
   uint32_t* part = A.at<uint32_t>(kLayout.part);
   uint32_t* tot_nodes = reinterpret_cast<uint32_t*>(&sc->total_nodes);
   // bodies sharing all digits of the first word: ordered by the second
-  launch_fix_runs(n, St, sy, skey, key2[0], nullptr, 0, s);
-  launch_lcp_count(n, skey, key2[0], St.sys, lcp, cnt_s, part, sc, s);
+  launch_fix_runs(n, St, sy, skey, key2, nullptr, 0, s);
+  launch_lcp_count(n, skey, key2, St.sys, lcp, cnt_s, part, sc, s);
   scan_u32(cnt_s, cnt_s, n, tot_nodes, scr, s);
   DevScalars h;
   {
@@ -213,7 +207,6 @@ nbx_status accel_in_arena(const Arena& A, int64_t n, const double* x, const doub
     if (r != NBX_OK) return r;
   }
   if (h.err & 1) return NBX_ERR_NONFINITE;
-  if (h.err & kSortErrTimeout) return NBX_ERR_HIP;
   if (h.coincident > 0) return NBX_ERR_DEPTH;
   const int64_t total = (uint32_t)h.total_nodes;
   const int64_t mi = internal_count(h);

@@ -102,6 +102,16 @@ void launch_upward(const int32_t* level_list, const uint32_t* end_list, int64_t 
 void launch_upward_all(const int32_t* counts, const int32_t* level_list, const uint32_t* end_list, RefNode* nodes,
                        WalkHead* heads, double theta, const int32_t* sys, const double* root, hipStream_t s);
 void launch_fill_u32(int64_t n, uint32_t* a, uint32_t v, hipStream_t s);
+// Keys and body arrays (amag may be null) in ascending order of the keys,
+// equal keys in their previous order: sort and gather in one launch, for
+// systems of at most kRankSortMax bodies (n^2 compares).
+constexpr int kRankWaves = 16;
+constexpr int64_t kRankSortMax = 16384;
+// Up to here also in place of the nearly-sorted path (three launches and the
+// gather, 45 us at any small size).
+constexpr int64_t kRankAlways = 4096;
+void launch_rank_sort(int64_t n, const uint64_t* key, uint64_t* kout, const StateArrays& src, const StateArrays& dst,
+                      const uint32_t* amag, uint32_t* amag_out, hipStream_t s);
 // Upload indices id0, id0 + 1, ... and system number of n slots.
 void launch_set_ids(int64_t n, int32_t* id, int32_t id0, int32_t* sys, int32_t sys_no, hipStream_t s);
 // inv[j] = the slot (of cnt) that holds upload index base + j; *bad (host
