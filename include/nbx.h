@@ -204,8 +204,8 @@ nbx_status nbx_accel(nbx_ctx* ctx, double* ax, double* ay, double* az);
  * (16 MiB, held by each GPU it runs on until the process ends), sized for at
  * most NBX_NOALLOC_MAX_BODIES bodies and NBX_NOALLOC_MAX_NODES tree nodes.
  * Runs on the calling thread's current device and the given stream (null:
- * the null stream); synchronises that stream once for the node counts and
- * returns after the results are written.  Calls on one device share the
+ * the null stream); waits on that stream once and returns after the results
+ * are written.  Calls on one device share the
  * array and are serialised by a lock.  The call itself allocates no memory
  * and is not capturable (it waits on the stream).  Errors: NBX_ERR_ARG (null
  * pointer, n < 0 or above the maximum, theta < 0), NBX_ERR_NOMEM (the tree

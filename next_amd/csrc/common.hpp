@@ -65,6 +65,7 @@ struct DevScalars {
   // which the tree kernels of the run do nothing.
   int32_t abort_flags;
   int32_t level_off[kMaxDepthSlots];
+  unsigned long long over_depths;       // depths with nodes that end beyond their units (units.hpp)
   int32_t step_count;                   // next entry of the dt log of a captured run
   uint32_t ndesc;                       // descents of nearly sorted keys (patch_sort_u64), cleared per build
 };

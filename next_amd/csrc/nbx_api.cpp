@@ -61,6 +61,7 @@ struct nbx_ctx {
   DBuf lcp, cnt_s;
   DBuf nodes, heads;          // reference-mode node records and their walk heads
   DBuf level_list, end_list;  // internal nodes by depth, and their skip targets
+  DBuf over;                  // small systems: per depth and unit, the node that ends beyond the unit
   DBuf scratch, dts, lvl_part;
   DBuf pnodes, paux, pot, epart, eout;     // physics-mode tree, moments, potential, energy
   DBuf dacc, dpart;           // forces of the diagnostic passes (potential, direct sum), partial direct sums
@@ -213,7 +214,7 @@ void each_buf(nbx_ctx* c, F f) {
   for (auto& w : c->st) for (auto& b : w) f(b);
   for (DBuf* a : {c->acc, c->key, c->idx, c->key2, c->amag})
     for (int k = 0; k < (a == c->acc ? 3 : 2); ++k) f(a[k]);
-  for (DBuf* b : {&c->lcp, &c->cnt_s, &c->nodes, &c->heads, &c->level_list, &c->end_list, &c->scratch, &c->dts,
+  for (DBuf* b : {&c->lcp, &c->cnt_s, &c->nodes, &c->heads, &c->level_list, &c->end_list, &c->over, &c->scratch, &c->dts,
                   &c->lvl_part, &c->pnodes, &c->paux, &c->pot, &c->dacc, &c->dpart, &c->epart, &c->eout, &c->s_root, &c->s_dt,
                   &c->s_v2, &c->s_soff, &c->s_sroot, &c->s_send, &c->groups, &c->boxes, &c->box_off, &c->box_part,
                   &c->tgroups, &c->gmarks, &c->snap_amag})
@@ -271,6 +272,7 @@ nbx_status ensure_particles(nbx_ctx* c, int64_t n, int64_t keep_n) {
     NBXCHK(ensure(c, c->lcp, (size_t)cap * 4));
     NBXCHK(ensure(c, c->cnt_s, (size_t)cap * 4));
     NBXCHK(ensure(c, c->lvl_part, (size_t)lcp_part_words(cap) * 4));
+    NBXCHK(ensure(c, c->over, (size_t)unit_count(std::min(cap, kUnitsMax)) * kMaxLevels * 4));
     NBXCHK(ensure(c, c->scratch, std::max(sort_scratch_words(cap), scan_scratch_words(cap)) * 4));
     c->cap = cap;
   }
@@ -352,6 +354,13 @@ int sys_bits(int nsys) {
   int b = 0;
   while ((1 << b) < nsys) ++b;
   return b;
+}
+
+// The unit pass's view of the layout (the buffers the last build filled).
+UnitArgs unit_args(nbx_ctx* c) {
+  return UnitArgs{c->n, unit_count(c->n), kUnitSpan, P<int32_t>(c->lcp), P<uint32_t>(c->cnt_s),
+                  P<uint32_t>(c->lvl_part), P<int32_t>(c->level_list), P<uint32_t>(c->end_list), c->sc,
+                  P<int32_t>(c->over)};
 }
 
 // Bounding boxes, keys, sort by key and then system, gather of the state
@@ -563,8 +572,11 @@ nbx_status build_post(nbx_ctx* c, const uint64_t* skey) {
     NBXCHK(ref_layout(c, c->spec_emit && total + 1 <= (int64_t)c->spec_nodes && m <= (int64_t)c->spec_int));
     record(c, EV_BUILD);
     RefNode* nodes = P<RefNode>(c->nodes);
-    launch_upward_all(c->hsc->level_count, P<int32_t>(c->level_list), P<uint32_t>(c->end_list), nodes,
-                      P<WalkHead>(c->heads), c->cfg.theta, St.sys, sy.root, s);
+    if (n <= kUnitsMax)
+      launch_upward_units(unit_args(c), nodes, P<WalkHead>(c->heads), c->cfg.theta, St.sys, sy, s);
+    else
+      launch_upward_all(c->hsc->level_count, P<int32_t>(c->level_list), P<uint32_t>(c->end_list), nodes,
+                        P<WalkHead>(c->heads), c->cfg.theta, St.sys, sy.root, s);
   }
   record(c, EV_UPWARD);
   c->tree_valid = true;
@@ -822,11 +834,15 @@ void build_bounded(nbx_ctx* c) {
     RefNode* nodes = P<RefNode>(c->nodes);
     launch_emit(n, P<int32_t>(c->lcp), P<uint32_t>(c->cnt_s), P<uint32_t>(c->lvl_part), St, sy, c->sc, nodes,
                 P<WalkHead>(c->heads), P<int32_t>(c->level_list), P<uint32_t>(c->end_list), cap_rec, cap_lst, s);
-    launch_upward_tail(c->b_dmax + 1, P<int32_t>(c->level_list), P<uint32_t>(c->end_list), nodes,
-                       P<WalkHead>(c->heads), c->cfg.theta, St.sys, sy.root, c->sc, s);
-    for (int d = c->b_dmax; d >= 0; --d)
-      launch_upward_level(c->b_grid_up[d], d, P<int32_t>(c->level_list), P<uint32_t>(c->end_list), nodes,
-                          P<WalkHead>(c->heads), c->cfg.theta, St.sys, sy.root, c->sc, s);
+    if (n <= kUnitsMax) {
+      launch_upward_units(unit_args(c), nodes, P<WalkHead>(c->heads), c->cfg.theta, St.sys, sy, s);
+    } else {
+      launch_upward_tail(c->b_dmax + 1, P<int32_t>(c->level_list), P<uint32_t>(c->end_list), nodes,
+                         P<WalkHead>(c->heads), c->cfg.theta, St.sys, sy.root, c->sc, s);
+      for (int d = c->b_dmax; d >= 0; --d)
+        launch_upward_level(c->b_grid_up[d], d, P<int32_t>(c->level_list), P<uint32_t>(c->end_list), nodes,
+                            P<WalkHead>(c->heads), c->cfg.theta, St.sys, sy.root, c->sc, s);
+    }
   }
   c->skey = skey;
   c->skey2 = P<uint64_t>(c->key2[0]);

@@ -42,7 +42,7 @@ constexpr size_t align256(size_t b) { return (b + 255) & ~size_t(255); }
 // kNaNodes nodes.
 struct Layout {
   size_t sc, st[2][10], acc[3], key[2], idx, key2, lcp, cnt_s, part, scanscr, nodes, heads, level_list, end_list;
-  size_t root, dt, v2, soff, sroot, send, groups, boxes, box_off, box_part, total;
+  size_t root, dt, v2, soff, sroot, send, over, groups, boxes, box_off, box_part, total;
 };
 
 constexpr Layout make_layout() {
@@ -70,6 +70,7 @@ constexpr Layout make_layout() {
   L.soff = take(2 * 4);
   L.sroot = take(4);
   L.send = take(4);
+  L.over = take((size_t)unit_count(kNaBodies) * kMaxLevels * 4);
   L.groups = take((size_t)kNaGroups * sizeof(Group));
   L.boxes = take((size_t)kNaBoxes * sizeof(BoxBlock));
   L.box_off = take(2 * 4);
@@ -101,7 +102,7 @@ __global__ __launch_bounds__(kBlock) void k_na_setup(int64_t n, const double* __
                                                      const double* __restrict__ y, const double* __restrict__ z,
                                                      const double* __restrict__ m, const int32_t* __restrict__ type,
                                                      StateArrays st, Group* groups, BoxBlock* boxes,
-                                                     int32_t* box_off, int32_t* soff, int32_t width) {
+                                                     int32_t* box_off, int32_t* soff, int32_t width, DevScalars* sc) {
   const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
   if (i < n) {
     st.x[i] = x[i]; st.y[i] = y[i]; st.z[i] = z[i];
@@ -118,16 +119,17 @@ __global__ __launch_bounds__(kBlock) void k_na_setup(int64_t n, const double* __
     const int32_t b = (int32_t)(i * kBoxSpan);
     boxes[i] = BoxBlock{0, b, (int32_t)std::min<int64_t>(b + kBoxSpan, n), 0};
   }
-  if (i == 0) { box_off[0] = 0; box_off[1] = (int32_t)nb; soff[0] = 0; soff[1] = (int32_t)n; }
+  if (i == 0) { sc->abort_flags = 0; box_off[0] = 0; box_off[1] = (int32_t)nb; soff[0] = 0; soff[1] = (int32_t)n; }
 }
 
 // Accelerations from key order back to the caller's order.
 __global__ __launch_bounds__(kBlock) void k_na_scatter(int64_t n, const int32_t* __restrict__ id,
                                                        const double* __restrict__ a0, const double* __restrict__ a1,
                                                        const double* __restrict__ a2, double* __restrict__ ax,
-                                                       double* __restrict__ ay, double* __restrict__ az) {
+                                                       double* __restrict__ ay, double* __restrict__ az,
+                                                       const DevScalars* __restrict__ sc) {
   const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-  if (i >= n) return;
+  if (i >= n || sc->abort_flags) return;                   // no forces: the caller's arrays stay as they are
   const int32_t o = id[i];
   ax[o] = a0[i]; ay[o] = a1[i]; az[o] = a2[i];
 }
@@ -181,11 +183,9 @@ nbx_status accel_in_arena(const Arena& A, int64_t n, const double* x, const doub
   const int64_t nb = (n + kBoxSpan - 1) / kBoxSpan;
   hipLaunchKernelGGL(k_na_setup, dim3((unsigned)div_up(n, kBlock)), dim3(kBlock), 0, s,
                      n, x, y, z, m, type, St, A.at<Group>(kLayout.groups), A.at<BoxBlock>(kLayout.boxes),
-                     A.at<int32_t>(kLayout.box_off), A.at<int32_t>(kLayout.soff), walk_width(n, theta));
+                     A.at<int32_t>(kLayout.box_off), A.at<int32_t>(kLayout.soff), walk_width(n, theta), sc);
   launch_bbox(St, A.at<BoxBlock>(kLayout.boxes), (int)nb, A.at<int32_t>(kLayout.box_off),
-              A.at<double>(kLayout.box_part), sy, nullptr, s);
-  launch_fill_scalars(sc, 1 | 4 | 8, s);
-  launch_set_run(sc, 0, s);                                // no abort flag: the walk runs
+              A.at<double>(kLayout.box_part), sy, sc, s);    // (clears the build's counts too)
   uint64_t* key[2] = {A.at<uint64_t>(kLayout.key[0]), A.at<uint64_t>(kLayout.key[1])};
   uint64_t* key2 = A.at<uint64_t>(kLayout.key2);
   launch_keys(n, St, sy, key[0], A.at<uint32_t>(kLayout.idx), sc, s);
@@ -201,16 +201,10 @@ nbx_status accel_in_arena(const Arena& A, int64_t n, const double* x, const doub
   launch_fix_runs(n, St, sy, skey, key2, nullptr, 0, s);
   launch_lcp_count(n, skey, key2, St.sys, lcp, cnt_s, part, sc, s);
   scan_u32(cnt_s, cnt_s, n, tot_nodes, scr, s);
-  DevScalars h;
-  {
-    const nbx_status r = read_scalars(sc, &h, s);
-    if (r != NBX_OK) return r;
-  }
-  if (h.err & 1) return NBX_ERR_NONFINITE;
-  if (h.coincident > 0) return NBX_ERR_DEPTH;
-  const int64_t total = (uint32_t)h.total_nodes;
-  const int64_t mi = internal_count(h);
-  if (total > kNaNodes || mi > kNaNodes) return NBX_ERR_NOMEM;   // the tree does not fit the array
+  // The launches below are sized by n alone, and every kernel from here on
+  // does nothing (the layout: nothing beyond the array) if the tree does not
+  // fit or a position is not finite; the scalars are read once, at the end.
+  launch_check(sc, kNaNodes + 1, kNaNodes, kMaxLevels, s);
   launch_sys_roots(sy, cnt_s, sc, s);
   RefNode* nodes = A.at<RefNode>(kLayout.nodes);
   WalkHead* heads = A.at<WalkHead>(kLayout.heads);
@@ -218,14 +212,23 @@ nbx_status accel_in_arena(const Arena& A, int64_t n, const double* x, const doub
   uint32_t* end_list = A.at<uint32_t>(kLayout.end_list);
   launch_emit(n, lcp, cnt_s, part, St, sy, sc, nodes, heads, level_list, end_list, (uint32_t)(kNaNodes + 1),
               (uint32_t)kNaNodes, s);
-  launch_upward_all(h.level_count, level_list, end_list, nodes, heads, theta, St.sys, sy.root, s);
+  launch_upward_units(UnitArgs{n, unit_count(n), kUnitSpan, lcp, cnt_s, part, level_list, end_list, sc,
+                               A.at<int32_t>(kLayout.over)},
+                      nodes, heads, theta, St.sys, sy, s);
   double* acc[3] = {A.at<double>(kLayout.acc[0]), A.at<double>(kLayout.acc[1]), A.at<double>(kLayout.acc[2])};
-  launch_walk(A.at<Group>(kLayout.groups), div_up(n, walk_width(n, theta)), nodes, heads, St, sy, theta, acc[0], acc[1], acc[2], sc,
-              false, false, s);
+  launch_walk(A.at<Group>(kLayout.groups), div_up(n, walk_width(n, theta)), nodes, heads, St, sy, theta, acc[0],
+              acc[1], acc[2], sc, false, false, s);
   hipLaunchKernelGGL(k_na_scatter, dim3((unsigned)div_up(n, kBlock)), dim3(kBlock), 0, s, n, St.id, acc[0], acc[1],
-                     acc[2], ax, ay, az);
+                     acc[2], ax, ay, az, sc);
   NA_HIP(hipGetLastError());
-  NA_HIP(hipStreamSynchronize(s));
+  DevScalars h;
+  {
+    const nbx_status r = read_scalars(sc, &h, s);
+    if (r != NBX_OK) return r;
+  }
+  if (h.err & 1) return NBX_ERR_NONFINITE;
+  if (h.coincident > 0) return NBX_ERR_DEPTH;
+  if (h.abort_flags) return NBX_ERR_NOMEM;                 // the tree does not fit the array
   return NBX_OK;
 }
 

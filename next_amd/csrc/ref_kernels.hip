@@ -13,7 +13,8 @@
 //         octree.h:69-87 in depth-first preorder (children 0..7), built from
 //         the rule "an internal node exists for every digit prefix shared by
 //         two or more bodies", with skip pointers for stackless traversal
-//   upward pass, one launch per depth, deepest first (octree.h:92-127)
+//   upward pass, deepest first, one launch per depth or, in small systems,
+//         within units of bodies (octree.h:92-127)
 //   walk: one wave per group of consecutive targets; the group decides once
 //         what all its targets decide alike, each target walks the rest with
 //         its own acceptance test (octree.h:133-179), so every target
@@ -22,6 +23,7 @@
 #include "layout.hpp"
 #include "prims.hpp"
 #include "ref_kernels.hpp"
+#include "units.hpp"
 
 #include <algorithm>
 #include <climits>
@@ -60,7 +62,7 @@ __global__ __launch_bounds__(kBlock) void k_fill_scalars(DevScalars* sc, int wha
   const int t = threadIdx.x;
   if (what & 1) {
     if (t < kMaxDepthSlots) sc->level_count[t] = 0;
-    if (t == 0) { sc->collisions = 0; sc->coincident = 0; sc->max_leaf_depth = 0; sc->ndesc = 0; }
+    if (t == 0) { sc->collisions = 0; sc->coincident = 0; sc->max_leaf_depth = 0; sc->ndesc = 0; sc->over_depths = 0ull; }
   }
   if ((what & 4) && t == 0) sc->err = 0;
   if ((what & 8) && t == 0) { sc->n_pp = 0ull; sc->n_pc = 0ull; sc->n_open = 0ull; sc->n_iter = 0ull; sc->n_eval = 0ull; }
@@ -112,6 +114,7 @@ __global__ __launch_bounds__(kWave) void k_bbox_final(const double* __restrict__
     clear->level_count[t] = 0;
     if (t == 0) {
       clear->collisions = 0; clear->coincident = 0; clear->max_leaf_depth = 0; clear->err = 0; clear->ndesc = 0;
+      clear->over_depths = 0ull;
     }
   }
   if (s >= sy.nsys) return;
@@ -587,22 +590,46 @@ __global__ __launch_bounds__(kWave) void k_check(DevScalars* sc, int64_t cap_rec
 // (all of it but the padding) and its walk head.  end: the preorder index after its
 // subtree (its skip pointer, from the list of skip targets); the first body
 // comes from the first child, the half-width from the system's root.
-__device__ __forceinline__ void upward_node(int32_t id, int32_t end, int d, RefNode* __restrict__ nodes,
-                                            WalkHead* __restrict__ heads, double inv_theta,
-                                            const int32_t* __restrict__ sys, const double* __restrict__ root) {
+//
+// The unit's nodes keep mass, centre and first body in LDS (36 bytes each).
+constexpr int kUnitNodes = 2048;
+struct UnitMoments {
+  double m[kUnitNodes], x[kUnitNodes], y[kUnitNodes], z[kUnitNodes];
+  int32_t first[kUnitNodes];
+};
+
+__device__ __forceinline__ void upward_node(const UnitView& v, UnitMoments* lm, int32_t id, int32_t end, int d,
+                                            RefNode* __restrict__ nodes, WalkHead* __restrict__ heads,
+                                            double inv_theta, double half, const int32_t* __restrict__ sys,
+                                            const double* __restrict__ root) {
   // One walk of the child chain (at most 8; the bound also keeps a malformed
   // chain finite) gathers each child's mass and centre into registers; a
   // slot past the last child keeps mass 0, which both sums skip.
   double cmv[8], cxv[8], cyv[8], czv[8];
-  int32_t c = id + 1, first = 0;
+  int32_t first = 0;
+  if (v.lds) {
+    int c = v.slot(id) + 1;
+    const int e = v.slot(end);
+    first = lm->first[c];
 #pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    cmv[j] = 0.0; cxv[j] = 0.0; cyv[j] = 0.0; czv[j] = 0.0;
-    if (c < end) {
-      const RefNode& ch = nodes[c];
-      cmv[j] = ch.m; cxv[j] = ch.cx; cyv[j] = ch.cy; czv[j] = ch.cz;
-      if (j == 0) first = ch.first;
-      c = ch.skip;
+    for (int j = 0; j < 8; ++j) {
+      cmv[j] = 0.0; cxv[j] = 0.0; cyv[j] = 0.0; czv[j] = 0.0;
+      if (c < e) {
+        cmv[j] = lm->m[c]; cxv[j] = lm->x[c]; cyv[j] = lm->y[c]; czv[j] = lm->z[c];
+        c = v.skips[c];
+      }
+    }
+  } else {
+    int32_t c = id + 1;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      cmv[j] = 0.0; cxv[j] = 0.0; cyv[j] = 0.0; czv[j] = 0.0;
+      if (c < end) {
+        const RefNode& ch = nodes[c];
+        cmv[j] = ch.m; cxv[j] = ch.cx; cyv[j] = ch.cy; czv[j] = ch.cz;
+        if (j == 0) first = ch.first;
+        c = ch.skip;
+      }
     }
   }
   double M = 0.0, sx = 0.0, sy = 0.0, sz = 0.0;
@@ -617,7 +644,7 @@ __device__ __forceinline__ void upward_node(int32_t id, int32_t end, int d, RefN
   }
   double cx = sx, cy = sy, cz = sz;
   if (M > 0.0) { cx = sx / M; cy = sy / M; cz = sz / M; }
-  const double size = ldexp(root[4 * sys[first] + 3], -d);
+  const double size = ldexp(sys ? root[4 * sys[first] + 3] : half, -d);
   double qxx = 0, qyy = 0, qzz = 0, qxy = 0, qxz = 0, qyz = 0;
   const double soft = size * size * 0.01;
 #pragma unroll
@@ -633,22 +660,20 @@ __device__ __forceinline__ void upward_node(int32_t id, int32_t end, int d, RefN
     qxz = qxz + mc * (3.0 * rx * rz);
     qyz = qyz + mc * (3.0 * ry * rz);
   }
-  RefNode p;
-  p.cx = cx; p.cy = cy; p.cz = cz; p.m = M;
-  p.skip = end;
-  p.body = -1;
-  p.depth = d;
-  p.first = first;
-  p.size = size;
-  const double cm = cbrt(M);
-  p.esum = size * 0.015 + cm * 0.002;
-  p.dmk = 2.0 * size / dm_power(M, cm);
-  p.qxx = qxx; p.qyy = qyy; p.qzz = qzz; p.qxy = qxy; p.qxz = qxz; p.qyz = qyz;
+  if (v.lds) {
+    const int k = v.slot(id);
+    lm->m[k] = M; lm->x[k] = cx; lm->y[k] = cy; lm->z[k] = cz;
+    lm->first[k] = first;
+  }
+  const double cb = cbrt(M);
   RefNode& out = nodes[id];                  // the record but its padding
-  out.cx = p.cx; out.cy = p.cy; out.cz = p.cz; out.m = p.m;
-  out.skip = p.skip; out.body = p.body; out.depth = p.depth; out.first = p.first;
-  out.size = p.size; out.esum = p.esum; out.dmk = p.dmk;
-  out.qxx = p.qxx; out.qyy = p.qyy; out.qzz = p.qzz; out.qxy = p.qxy; out.qxz = p.qxz; out.qyz = p.qyz;
+  out.cx = cx; out.cy = cy; out.cz = cz;
+  out.dmk = 2.0 * size / dm_power(M, cb);
+  out.m = M;
+  out.esum = size * 0.015 + cb * 0.002;
+  out.skip = end; out.body = -1; out.depth = d; out.first = first;
+  out.qxx = qxx; out.qyy = qyy; out.qzz = qzz; out.qxy = qxy; out.qxz = qxz; out.qyz = qyz;
+  out.size = size;
   // Upper edge of the opening test's band for r^2 (NEXT tests r^2 + 1e-20,
   // so the 1e-20 is taken off the edge); NaN, and every decision exact, where
   // (size/theta)^2 <= 1e-16, where the 1e-20 would eat the band's margin.
@@ -667,7 +692,8 @@ __global__ __launch_bounds__(kBlock) void k_upward(const int32_t* __restrict__ l
                                                    const double* __restrict__ root) {
   const int64_t k = (int64_t)blockIdx.x * kBlock + threadIdx.x;
   if (k >= cnt) return;
-  upward_node(level_list[beg + k], (int32_t)end_list[beg + k], d, nodes, heads, inv_theta, sys, root);
+  upward_node(UnitView{}, nullptr, level_list[beg + k], (int32_t)end_list[beg + k], d, nodes, heads, inv_theta, 0.0,
+              sys, root);
 }
 
 // Depths d_lo .. 41 of a build whose counts stay on the device, deepest
@@ -686,7 +712,8 @@ __global__ __launch_bounds__(kBlock) void k_upward_tail(int d_lo, const int32_t*
     const int64_t beg = sc->level_off[d], cnt = sc->level_count[d];
     if (cnt == 0) continue;
     for (int64_t k = threadIdx.x; k < cnt; k += kBlock)
-      upward_node(level_list[beg + k], (int32_t)end_list[beg + k], d, nodes, heads, inv_theta, sys, root);
+      upward_node(UnitView{}, nullptr, level_list[beg + k], (int32_t)end_list[beg + k], d, nodes, heads, inv_theta, 0.0,
+              sys, root);
     __syncthreads();
   }
 }
@@ -703,7 +730,36 @@ __global__ __launch_bounds__(kBlock) void k_upward_level(int d, const int32_t* _
   if (sc->abort_flags) return;
   const int64_t beg = sc->level_off[d], cnt = sc->level_count[d];
   for (int64_t k = (int64_t)blockIdx.x * kBlock + threadIdx.x; k < cnt; k += (int64_t)gridDim.x * kBlock)
-    upward_node(level_list[beg + k], (int32_t)end_list[beg + k], d, nodes, heads, inv_theta, sys, root);
+    upward_node(UnitView{}, nullptr, level_list[beg + k], (int32_t)end_list[beg + k], d, nodes, heads, inv_theta, 0.0,
+              sys, root);
+}
+
+__global__ __launch_bounds__(kBlock) void k_upward_unit(UnitArgs a, RefNode* __restrict__ nodes,
+                                                        WalkHead* __restrict__ heads, double inv_theta,
+                                                        const int32_t* __restrict__ sys,
+                                                        const double* __restrict__ root) {
+  __shared__ UnitMoments lm;
+  const double half = root[3];
+  upward_unit<1, kUnitNodes>(
+      a,
+      [&](const UnitView& v, int32_t k) {
+        const RefNode& nd = nodes[k];
+        const int s = v.slot(k);
+        lm.m[s] = nd.m; lm.x[s] = nd.cx; lm.y[s] = nd.cy; lm.z[s] = nd.cz;
+        lm.first[s] = nd.first;
+      },
+      [&](const UnitView& v, int32_t id, int32_t end, int d, int) {
+        upward_node(v, &lm, id, end, d, nodes, heads, inv_theta, half, sys, root);
+      });
+}
+
+__global__ __launch_bounds__(kOverBlock) void k_upward_over(UnitArgs a, SysArrays sy, RefNode* __restrict__ nodes,
+                                                            WalkHead* __restrict__ heads, double inv_theta,
+                                                            const int32_t* __restrict__ sys) {
+  const double half = sy.root[3];
+  upward_over<1>(a, sy, [&](const UnitView& v, int32_t id, int32_t end, int d, int) {
+    upward_node(v, nullptr, id, end, d, nodes, heads, inv_theta, half, sys, sy.root);
+  });
 }
 
 // Blocks are dealt to the 8 XCDs round-robin; remap so that each XCD walks
@@ -1340,6 +1396,16 @@ void launch_upward_all(const int32_t* counts, const int32_t* level_list, const u
     off -= counts[d];
     launch_upward(level_list, end_list, off, counts[d], d, nodes, heads, theta, sys, root, s);
   }
+}
+void launch_upward_units(const UnitArgs& a, RefNode* nodes, WalkHead* heads, double theta, const int32_t* sys,
+                   const SysArrays& sy, hipStream_t s) {
+  if (a.n <= 0) return;
+  if (sy.nsys == 1) sys = nullptr;                         // one root
+  hipLaunchKernelGGL(k_upward_unit, dim3((unsigned)a.units), dim3(kBlock), 0, s, a, nodes, heads, 1.0 / theta, sys,
+                     sy.root);
+  if (a.units > 1)
+    hipLaunchKernelGGL(k_upward_over, dim3((unsigned)sy.nsys), dim3(kOverBlock), 0, s, a, sy, nodes, heads,
+                       1.0 / theta, sys);
 }
 void launch_walk(const Group* groups, int64_t ngroups, const RefNode* nodes, const WalkHead* heads,
                  const StateArrays& st,

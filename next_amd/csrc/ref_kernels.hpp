@@ -101,6 +101,28 @@ void launch_upward(const int32_t* level_list, const uint32_t* end_list, int64_t 
 // measured slower.)
 void launch_upward_all(const int32_t* counts, const int32_t* level_list, const uint32_t* end_list, RefNode* nodes,
                        WalkHead* heads, double theta, const int32_t* sys, const double* root, hipStream_t s);
+// The same for a build of at most kUnitsMax bodies in two launches whose sizes
+// need no counts on the host (units.hpp).  What it reads of the layout: the
+// lcp and node offsets of the bodies, the scanned per-block counts of
+// k_lcp_count, the per-depth node list and its skip targets; over holds
+// kMaxLevels entries per unit; sys: the bodies' systems (after
+// launch_sys_roots).
+struct UnitArgs {
+  int64_t n;
+  int32_t units, span;
+  const int32_t* lcp;
+  const uint32_t* pre_off;
+  const uint32_t* part;
+  const int32_t* level_list;
+  const uint32_t* end_list;
+  DevScalars* sc;
+  int32_t* over;
+};
+constexpr int64_t kUnitsMax = 262144;
+constexpr int32_t kUnitSpan = 768;   // bodies per unit: about 1,150 nodes
+constexpr int32_t unit_count(int64_t n) { return n >= 2 * kUnitSpan ? (int32_t)(n / kUnitSpan) : 1; }
+void launch_upward_units(const UnitArgs& a, RefNode* nodes, WalkHead* heads, double theta, const int32_t* sys,
+                         const SysArrays& sy, hipStream_t s);
 void launch_fill_u32(int64_t n, uint32_t* a, uint32_t v, hipStream_t s);
 // Keys and body arrays (amag may be null) in ascending order of the keys,
 // equal keys in their previous order: sort and gather in one launch, for
