@@ -604,19 +604,17 @@ __global__ __launch_bounds__(kPhysBlock) void k_phys_walk(const Group* __restric
 
 // FP64 direct sum.  One target per lane, 64 consecutive bodies per wave; the
 // sources are wave-uniform, so they come in by scalar loads and cost no LDS,
-// no barrier and no vector load.  blockIdx.y takes one of `splits` equal parts
-// of every system's sources, so that a small system fills the chip too; the
-// parts are summed in order by k_direct_sum.  A pair issues 18 FP64
-// instructions and v_rsq_f64 (one Newton step: a few ulp), so the sum is bound
-// by FP64 issue: 65,537 bodies 18.1 -> 3.3 ms per call against one target per thread
-// with sources staged in LDS, a correctly rounded square root and divide per
-// pair and 257 workgroups.
+// no barrier and no vector load.  Every system's sources are split over the
+// waves of a workgroup, whose sums meet in LDS, and over blockIdx.y
+// (k_direct_sum), so that a small system fills the chip too.  A pair issues 18
+// FP64 instructions and v_rsq_f64 (one Newton step: a few ulp), so the sum is
+// bound by FP64 issue: 65,537 bodies 18.1 -> 3.3 ms per call against one
+// target per thread with sources staged in LDS, a correctly rounded square
+// root and divide per pair and 257 workgroups.
 //
 // Only bodies of the target's own system act on it: a wave whose targets lie
 // in several systems takes them one after another.  The lanes' own bodies are
 // among 64 sources only; the rest of the loop does not test for the self pair.
-constexpr int kDirectWaves = 4;    // waves per workgroup, each with its own 64 targets
-
 struct DirectSum { double x, y, z, p; };
 
 // Sources [j, end).  SELF: some of them are targets of the wave (body i of
@@ -645,14 +643,15 @@ __device__ __forceinline__ void direct_range(const StateArrays& st, int64_t j, i
   }
 }
 
-template <bool ZERO>
-__global__ __launch_bounds__(kDirectWaves* kWave) void k_direct64(int64_t n, StateArrays st, SysArrays sy, double e2,
-                                                                  int splits, double* __restrict__ ax,
-                                                                  double* __restrict__ ay, double* __restrict__ az,
-                                                                  double* __restrict__ pot) {
+// The W waves of a workgroup have the same 64 targets and a part of the
+// sources each.
+template <bool ZERO, int W>
+__global__ __launch_bounds__(W* kWave) void k_direct64(int64_t n, StateArrays st, SysArrays sy, double e2,
+                                                       double* __restrict__ ax, double* __restrict__ ay,
+                                                       double* __restrict__ az, double* __restrict__ pot) {
+  __shared__ double part[W - 1][4][kWave];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-  const int64_t i0 = ((int64_t)blockIdx.x * kDirectWaves + wave) * kWave;
-  if (i0 >= n) return;
+  const int64_t i0 = (int64_t)blockIdx.x * kWave;
   const int64_t i1 = i0 + kWave < n ? i0 + kWave : n;        // targets [i0, i1)
   const int64_t i = i0 + lane_id();
   const bool valid = i < n;
@@ -660,10 +659,11 @@ __global__ __launch_bounds__(kDirectWaves* kWave) void k_direct64(int64_t n, Sta
   const double px = st.x[ii], py = st.y[ii], pz = st.z[ii];
   const int32_t me = st.sys[ii];
   const int32_t s0 = __builtin_amdgcn_readfirstlane(st.sys[i0]), s1 = __builtin_amdgcn_readfirstlane(st.sys[i1 - 1]);
+  const int q = blockIdx.y * W + wave, parts = gridDim.y * W;
   DirectSum a{0.0, 0.0, 0.0, 0.0};
   for (int32_t s = s0; s <= s1; ++s) {
     const int64_t lo = sy.soff[s], cnt = sy.soff[s + 1] - lo;
-    const int64_t b = lo + cnt * blockIdx.y / splits, e = lo + cnt * (blockIdx.y + 1) / splits;
+    const int64_t b = lo + cnt * q / parts, e = lo + cnt * (q + 1) / parts;
     if (me == s) {
       const int64_t c0 = i0 < b ? b : i0 < e ? i0 : e, c1 = i1 < b ? b : i1 < e ? i1 : e;   // own targets in [b, e)
       direct_range<false, ZERO>(st, b, c0, i, px, py, pz, e2, a);
@@ -671,10 +671,25 @@ __global__ __launch_bounds__(kDirectWaves* kWave) void k_direct64(int64_t n, Sta
       direct_range<false, ZERO>(st, c1, e, i, px, py, pz, e2, a);
     }
   }
-  if (!valid) return;
-  const int64_t at = (splits > 1 ? (int64_t)blockIdx.y * 4 * n : 0) + i;   // parts: x y z p, n each
-  if (splits > 1) { ax[at] = a.x; ax[at + n] = a.y; ax[at + 2 * n] = a.z; ax[at + 3 * n] = a.p; }
-  else { ax[i] = a.x; ay[i] = a.y; az[i] = a.z; if (pot) pot[i] = a.p; }
+  if (wave > 0) {
+    double(*const p)[kWave] = part[wave - 1];
+    p[0][lane_id()] = a.x; p[1][lane_id()] = a.y; p[2][lane_id()] = a.z; p[3][lane_id()] = a.p;
+  }
+  __syncthreads();
+  if (wave > 0 || !valid) return;
+  for (int w = 0; w < W - 1; ++w) {
+    a.x += part[w][0][lane_id()];
+    a.y += part[w][1][lane_id()];
+    a.z += part[w][2][lane_id()];
+    a.p += part[w][3][lane_id()];
+  }
+  if (gridDim.y > 1) {                                       // halves: x y z p, n each
+    const int64_t at = (int64_t)blockIdx.y * 4 * n + i;
+    ax[at] = a.x; ax[at + n] = a.y; ax[at + 2 * n] = a.z; ax[at + 3 * n] = a.p;
+  } else {
+    ax[i] = a.x; ay[i] = a.y; az[i] = a.z;
+    if (pot) pot[i] = a.p;
+  }
 }
 
 __global__ __launch_bounds__(kBlock) void k_direct_sum(int64_t n, int splits, const double* __restrict__ part,
@@ -838,25 +853,35 @@ void launch_phys_walk(const Group* groups, int64_t grid_groups, const PhysNode* 
                               th2, s);
 }
 
-// Parts of the sources: enough for 8 waves on each of the 1,024 SIMDs, of 64
-// sources or more.
+// Waves per workgroup and halves of the sources: 8 waves on each of the 1,024
+// SIMDs from 65,536 bodies on, at least 64 sources a wave below.  Workgroups
+// of 16 waves serve where 4 would leave SIMDs with fewer than 4 waves; above,
+// 2 resident ones per CU would leave the last round nearly empty.  No more
+// than two halves: their sums are 64 bytes per body.
+static int direct_waves(int64_t n) { return n <= 32768 ? 16 : 4; }
+
 int direct_splits(int64_t n) {
-  const int64_t waves = div_up(std::max<int64_t>(n, 1), kWave);
-  return (int)std::max<int64_t>(1, std::min<int64_t>({8192 / waves, waves, 64}));
+  const int64_t groups = div_up(std::max<int64_t>(n, 1), kWave);
+  const int w = direct_waves(n);
+  return groups * w < 8192 && groups >= 2 * w ? 2 : 1;
+}
+
+template <bool ZERO, int W>
+static void direct_go(int64_t n, int splits, const StateArrays& st, const SysArrays& sy, double e2, double* ax,
+                      double* ay, double* az, double* pot, hipStream_t s) {
+  hipLaunchKernelGGL((k_direct64<ZERO, W>), dim3(grid_of(n, kWave), (unsigned)splits), dim3(W * kWave), 0, s, n, st,
+                     sy, e2, ax, ay, az, pot);
 }
 
 void launch_direct64(int64_t n, const StateArrays& st, const SysArrays& sy, double eps, double* part, double* ax,
                      double* ay, double* az, double* pot, hipStream_t s) {
   if (n <= 0) return;
   const int splits = direct_splits(n);
-  const dim3 grid(grid_of(n, kDirectWaves * kWave), (unsigned)splits);
   double* const ox = splits > 1 ? part : ax;
-  if (eps * eps > 0.0)
-    hipLaunchKernelGGL(k_direct64<false>, grid, dim3(kDirectWaves * kWave), 0, s, n, st, sy, eps * eps, splits, ox, ay,
-                       az, pot);
-  else
-    hipLaunchKernelGGL(k_direct64<true>, grid, dim3(kDirectWaves * kWave), 0, s, n, st, sy, eps * eps, splits, ox, ay,
-                       az, pot);
+  const double e2 = eps * eps;
+  auto* const go = direct_waves(n) == 16 ? (e2 > 0.0 ? &direct_go<false, 16> : &direct_go<true, 16>)
+                                         : (e2 > 0.0 ? &direct_go<false, 4> : &direct_go<true, 4>);
+  go(n, splits, st, sy, e2, ox, ay, az, pot, s);
   if (splits > 1)
     hipLaunchKernelGGL(k_direct_sum, dim3(grid_of(n, kBlock)), dim3(kBlock), 0, s, n, splits, part, ax, ay, az, pot);
 }

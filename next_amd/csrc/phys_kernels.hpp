@@ -89,8 +89,8 @@ void launch_phys_walk(const Group* groups, int64_t grid_groups, const PhysNode* 
                       DevScalars* sc, bool kick, bool count, bool fp64, const float* amag, double alpha,
                       double theta, int list, hipStream_t s);
 // FP64 direct sum with Plummer softening over all pairs of each system (G = 1).
-// part: room for direct_splits(n) * 4 * n partial sums when that is more than
-// one part (at most 17 MB).
+// part: room for direct_splits(n) * 4 * n partial sums when that is two parts
+// (fewer than 131,072 bodies).
 int direct_splits(int64_t n);
 void launch_direct64(int64_t n, const StateArrays& st, const SysArrays& sy, double eps, double* part, double* ax,
                      double* ay, double* az, double* pot, hipStream_t s);

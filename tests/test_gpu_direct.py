@@ -1,10 +1,10 @@
 """The FP64 direct sum at the sizes where its split changes (64 targets per
-wave; the sources in up to 64 parts of at least 64, one part from 524,288
-bodies on), for single systems and batches whose systems share waves, against
-the oracle's direct sum.  Tolerance: sums of n terms in different orders, each
-term a few ulp: relative to the sum of the terms' magnitudes the difference is
-below n 2^-53 by a wide margin; 1e-12 of the largest acceleration and
-potential.
+workgroup; the sources over 16 waves up to 32,768 bodies and over 4 above, and
+in two halves below 131,008 bodies, one where a half would be too short), for
+single systems and batches whose systems share waves, against the oracle's
+direct sum.  Tolerance: sums of n terms in different orders, each term a few
+ulp: relative to the sum of the terms' magnitudes the difference is below
+n 2^-53 by a wide margin; 1e-12 of the largest acceleration and potential.
 """
 import numpy as np
 import pytest
@@ -22,7 +22,8 @@ def check(a, pot, p, eps, tg):
     assert np.max(np.abs(pot[tg] - pd)) <= 1e-12 * max(np.max(np.abs(pd)), 1e-300)
 
 
-@pytest.mark.parametrize("n", [1, 2, 63, 64, 65, 129, 4095, 4097, 8193, 65537, 524287, 524289])
+@pytest.mark.parametrize("n", [1, 2, 63, 64, 65, 129, 4095, 4097, 8193, 32768, 32769, 65537, 131008, 131009,
+                               524287, 524289])
 def test_sizes(n):
     p = ic.plummer(n, seed=n, virial=None)
     with Engine(mode=MODE_PHYSICS, precision=PREC_FP64, eps=0.01) as e:
