@@ -38,6 +38,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <cstddef>
 
 namespace nbx {
 namespace {
@@ -129,6 +130,41 @@ __global__ __launch_bounds__(kBlock) void k_phys_pair_dev(const int32_t* __restr
     pn[level_list[k]].skip = (int32_t)end_list[k];
 }
 
+// Eight lanes work on one node of the upward pass, a lane per child: a node's
+// children (192 bytes each) come in at once and their terms are formed side
+// by side; a sum runs over the children in order in one lane, the terms passed
+// through LDS.  One thread per node waits for its children one after another
+// and keeps 5 waves per SIMD at most: the pass's launches over all depths took
+// 850 us at 4,194,304 bodies, 255 us at 2^20 and 317 us at 96 systems of
+// 1.49 M bodies; now 593, 183 and 238 us.  (Units of bodies as in units.hpp,
+// two launches in all: 154 us at 16,384 bodies against 95, 183 against 103 at
+// 65,536, 244 at the 96 systems.)
+constexpr int kNodeLanes = 8;
+constexpr int kNodeTerms = 6;      // sums over the children exchanged at once
+typedef double NodeXch[kNodeTerms * kNodeLanes];
+
+__device__ __forceinline__ void wave_order() {   // LDS traffic of one wave keeps its order; so must the compiler
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Sum q over the node's children in order, in lane q < Q; v[q] is this lane's
+// (this child's) term.
+template <int Q>
+__device__ __forceinline__ double sum_children(double* xch, int c, const double (&v)[Q]) {
+  static_assert(Q <= kNodeTerms, "exchange buffer");
+  wave_order();
+#pragma unroll
+  for (int q = 0; q < Q; ++q) xch[q * kNodeLanes + c] = v[q];
+  wave_order();
+  double s = 0.0;
+  const double* row = xch + (c < Q ? c : 0) * kNodeLanes;
+#pragma unroll
+  for (int j = 0; j < kNodeLanes; ++j) s = s + row[j];
+  return s;
+}
+
 // Internal nodes of one depth from their children (FP64), and the walk
 // groups this node packs: a node of more than G bodies packs its children of
 // at most G bodies into groups, consecutive siblings together while the sum
@@ -136,99 +172,112 @@ __global__ __launch_bounds__(kBlock) void k_phys_pair_dev(const int32_t* __restr
 // Every body lands in exactly one group and a group's bodies lie inside one
 // node, so groups are compact in space where runs of G consecutive Morton
 // keys are not (such a run can straddle two distant cells).
-__device__ __forceinline__ void phys_upward_node(int32_t id, bool root_level, PhysNode* __restrict__ pn,
-                                                 PhysAux* __restrict__ aux, double inv_theta, int G,
-                                                 int32_t* __restrict__ gcnt, uint32_t* __restrict__ gmark) {
+// Called by the eight lanes of a node together; c: the lane's child.
+__device__ __forceinline__ void phys_upward_node(double* xch, int32_t id, bool root_level, int c,
+                                                 PhysNode* __restrict__ pn, PhysAux* __restrict__ aux,
+                                                 double inv_theta, int G, int32_t* __restrict__ gcnt,
+                                                 uint32_t* __restrict__ gmark) {
   const int32_t end = pn[id].skip;
+  const int lead = lane_id() - c;
   const int32_t first = pn[id].first;
-  // One walk of the child chain (at most 8 children) records the child
-  // indices (-1: no child) and sizes and sums mass and mass moment; the
-  // second pass reads the same (now cached) records again, which keeps the
-  // kernel's registers, and so its occupancy, where a latency-bound pass
-  // needs them.
-  int32_t chv[8], cnv[8];
-  double M = 0, sx = 0, sy = 0, sz = 0;
-  int32_t count = 0;
-  int32_t c = id + 1;
+  int32_t ci = -1;                                           // this lane's child
+  {
+    int32_t p = id + 1;
 #pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    chv[j] = -1; cnv[j] = 0;
-    if (c < end) {
-      const PhysNode& ch = pn[c];
-      chv[j] = c;
-      cnv[j] = ch.count;
-      const double cm = ch.count == 1 ? leaf_mass(ch) : aux[c].m;
-      M += cm;
-      sx += ch.cx * cm; sy += ch.cy * cm; sz += ch.cz * cm;
-      count += ch.count;
-      c = ch.skip;
-    }
-  }
-  double cx, cy, cz;
-  if (M > 0) { cx = sx / M; cy = sy / M; cz = sz / M; }
-  else { cx = pn[id + 1].cx; cy = pn[id + 1].cy; cz = pn[id + 1].cz; }
-  double q[6] = {0, 0, 0, 0, 0, 0};
-  double bsum = 0;
-  double lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
-#pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    if (chv[j] < 0) continue;
-    const PhysNode& ch = pn[chv[j]];
-    const double px = ch.cx, py = ch.cy, pz = ch.cz;
-    const double rx = px - cx, ry = py - cy, rz = pz - cz;
-    const double r2 = rx * rx + ry * ry + rz * rz;
-    double b = sqrt(r2);
-    double mc;
-    if (cnv[j] == 1) {                                     // a body: a point
-      mc = leaf_mass(ch);
-      lo[0] = fmin(lo[0], px); hi[0] = fmax(hi[0], px);
-      lo[1] = fmin(lo[1], py); hi[1] = fmax(hi[1], py);
-      lo[2] = fmin(lo[2], pz); hi[2] = fmax(hi[2], pz);
-    } else {                                               // a cell: its moments and box
-      const PhysAux& a = aux[chv[j]];
-      mc = a.m;
-      for (int t = 0; t < 6; ++t) q[t] += a.q[t];
-      b += a.bmax;
-      for (int d = 0; d < 3; ++d) {
-        lo[d] = fmin(lo[d], a.lo[d]);
-        hi[d] = fmax(hi[d], a.hi[d]);
+    for (int j = 0; j < kNodeLanes; ++j) {
+      if (p < end) {
+        if (j == c) ci = p;
+        p = pn[p].skip;
       }
     }
-    q[0] += mc * (3 * rx * rx - r2);
-    q[1] += mc * (3 * ry * ry - r2);
-    q[2] += mc * (3 * rz * rz - r2);
-    q[3] += mc * 3 * rx * ry;
-    q[4] += mc * 3 * rx * rz;
-    q[5] += mc * 3 * ry * rz;
-    if (b > bsum) bsum = b;
+  }
+  // a body (a point) or a cell with its moments and box
+  int32_t cn = 0;
+  double px = 0, py = 0, pz = 0, cm = 0, bc = 0;
+  double cq[6] = {0, 0, 0, 0, 0, 0};
+  double lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
+  if (ci >= 0) {
+    const PhysNode& ch = pn[ci];
+    cn = ch.count;
+    px = ch.cx; py = ch.cy; pz = ch.cz;
+    if (cn == 1) {
+      cm = leaf_mass(ch);
+      lo[0] = hi[0] = px; lo[1] = hi[1] = py; lo[2] = hi[2] = pz;
+    } else {
+      const PhysAux& a = aux[ci];
+      cm = a.m;
+      bc = a.bmax;
+      for (int t = 0; t < 6; ++t) cq[t] = a.q[t];
+      for (int k = 0; k < 3; ++k) { lo[k] = a.lo[k]; hi[k] = a.hi[k]; }
+    }
+  }
+  const double sums = sum_children<4>(xch, c, {cm, px * cm, py * cm, pz * cm});
+  const double M = __shfl(sums, lead, kWave);
+  // lanes 1 to 3: x, y, z (of the first child where there is no mass)
+  const double x0 = __shfl(px, lead, kWave), y0 = __shfl(py, lead, kWave), z0 = __shfl(pz, lead, kWave);
+  const double com = M > 0 ? sums / M : c == 1 ? x0 : c == 2 ? y0 : z0;
+  const double cx = __shfl(com, lead + 1, kWave), cy = __shfl(com, lead + 2, kWave), cz = __shfl(com, lead + 3, kWave);
+  // (no child: 0, whose square times no mass is 0 at any distance of the centre)
+  const double rx = ci >= 0 ? px - cx : 0.0, ry = ci >= 0 ? py - cy : 0.0, rz = ci >= 0 ? pz - cz : 0.0;
+  const double r2 = rx * rx + ry * ry + rz * rz;
+  double bsum = ci >= 0 ? sqrt(r2) + bc : 0.0;
+  const double quad =
+      sum_children<6>(xch, c, {cq[0] + cm * (3 * rx * rx - r2), cq[1] + cm * (3 * ry * ry - r2),
+                               cq[2] + cm * (3 * rz * rz - r2), cq[3] + cm * 3 * rx * ry, cq[4] + cm * 3 * rx * rz,
+                               cq[5] + cm * 3 * ry * rz});
+  int32_t count = cn;
+#pragma unroll
+  for (int o = 1; o < kNodeLanes; o <<= 1) {
+    count += __shfl_xor(count, o, kWave);
+    bsum = fmax(bsum, __shfl_xor(bsum, o, kWave));
+    for (int k = 0; k < 3; ++k) {
+      lo[k] = fmin(lo[k], __shfl_xor(lo[k], o, kWave));
+      hi[k] = fmax(hi[k], __shfl_xor(hi[k], o, kWave));
+    }
   }
   // bmax: the farthest corner of the bodies' box from the centre of mass,
   // or the children's bound if that is smaller.
   const double ex = fmax(cx - lo[0], hi[0] - cx), ey = fmax(cy - lo[1], hi[1] - cy), ez = fmax(cz - lo[2], hi[2] - cz);
   double bmax = sqrt(ex * ex + ey * ey + ez * ez);
   if (bsum < bmax) bmax = bsum;
-  PhysNode nd;
-  nd.cx = cx; nd.cy = cy; nd.cz = cz;
-  nd.m = (float)M;
-  nd.count = count;
   // Cells of very few bodies cost more as a multipole than as bodies.
   const double rc = bmax * inv_theta;
-  nd.rc2 = count < 4 ? INFINITY : (float)(rc * rc * (1.0 + 1e-6));
-  nd.qxx = (float)q[0]; nd.qyy = (float)q[1];
-  nd.qxy = (float)q[3]; nd.qxz = (float)q[4]; nd.qyz = (float)q[5];
-  nd.skip = end;
-  nd.first = first;
-  pn[id] = nd;
+  const float rc2 = count < 4 ? INFINITY : (float)(rc * rc * (1.0 + 1e-6));
+  // The record in one store and the moments in two, 8 bytes a lane.
+  static_assert(offsetof(PhysNode, cx) == 0 && offsetof(PhysNode, m) == 24 && offsetof(PhysNode, rc2) == 28 &&
+                    offsetof(PhysNode, qxx) == 32 && offsetof(PhysNode, qxy) == 40 && offsetof(PhysNode, qyz) == 48 &&
+                    offsetof(PhysNode, skip) == 52 && offsetof(PhysNode, first) == 56 && offsetof(PhysAux, q) == 16 &&
+                    offsetof(PhysAux, lo) == 64,
+                "stored by lane");
+  const float qf = (float)quad;
+  const float qxx = __shfl(qf, lead, kWave), qyy = __shfl(qf, lead + 1, kWave), qxy = __shfl(qf, lead + 3, kWave),
+              qxz = __shfl(qf, lead + 4, kWave), qyz = __shfl(qf, lead + 5, kWave);
+  const uint32_t wlo = c == 0   ? __float_as_uint((float)M)
+                       : c == 4 ? __float_as_uint(qxx)
+                       : c == 5 ? __float_as_uint(qxy)
+                       : c == 6 ? __float_as_uint(qyz)
+                                : (uint32_t)first;
+  const uint32_t whi = c == 0   ? __float_as_uint(rc2)
+                       : c == 4 ? __float_as_uint(qyy)
+                       : c == 5 ? __float_as_uint(qxz)
+                       : c == 6 ? (uint32_t)end
+                                : (uint32_t)count;
+  const double word = __longlong_as_double((long long)((uint64_t)wlo | ((uint64_t)whi << 32)));
+  const bool is_com = c >= 1 && c <= 3;
+  reinterpret_cast<double*>(pn + id)[is_com ? c - 1 : c == 0 ? 3 : c] = is_com ? com : word;
+  double* const ax = reinterpret_cast<double*>(aux + id);
+  ax[c < 6 ? 2 + c : c - 6] = c < 6 ? quad : c == 6 ? M : bmax;
+  if (c < 6) ax[8 + c] = c == 0 ? lo[0] : c == 1 ? lo[1] : c == 2 ? lo[2] : c == 3 ? hi[0] : c == 4 ? hi[1] : hi[2];
   // walk groups
   if (count > G) {
     int32_t run_first = 0, run = 0, f = first;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const int32_t cc = cnv[j];
-      const int32_t cf = f;                                // children's bodies follow one another
+    for (int j = 0; j < kNodeLanes; ++j) {
+      const int32_t cc = __shfl(cn, lead + j, kWave);
+      const int32_t cf = f;                                  // children's bodies follow one another
       f += cc;
-      if (cc == 0) continue;
-      if (cc > G) {                                        // packs its own children
+      if (c != 0 || cc == 0) continue;
+      if (cc > G) {                                          // packs its own children
         if (run > 0) mark_group(run_first, run, gcnt, gmark);
         run = 0;
         continue;
@@ -238,53 +287,53 @@ __device__ __forceinline__ void phys_upward_node(int32_t id, bool root_level, Ph
       run += cc;
     }
     if (run > 0) mark_group(run_first, run, gcnt, gmark);
-  } else if (root_level) {
+  } else if (root_level && c == 0) {
     mark_group(first, count, gcnt, gmark);
   }
-  PhysAux a;
-  a.m = M;
-  a.bmax = bmax;
-  for (int j = 0; j < 6; ++j) a.q[j] = q[j];
-  for (int d = 0; d < 3; ++d) { a.lo[d] = lo[d]; a.hi[d] = hi[d]; }
-  a.pad[0] = a.pad[1] = 0.0;
-  aux[id] = a;
 }
 
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5)))
+__global__ __launch_bounds__(kBlock)
 void k_phys_upward(const int32_t* __restrict__ level_list, int64_t beg, int64_t cnt, bool root_level,
                    PhysNode* __restrict__ pn, PhysAux* __restrict__ aux, double inv_theta, int G,
                    int32_t* __restrict__ gcnt, uint32_t* __restrict__ gmark) {
-  const int64_t k = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+  __shared__ NodeXch xch[kBlock / kNodeLanes];
+  const int64_t k = ((int64_t)blockIdx.x * kBlock + threadIdx.x) / kNodeLanes;
   if (k >= cnt) return;
-  phys_upward_node(level_list[beg + k], root_level, pn, aux, inv_theta, G, gcnt, gmark);
+  phys_upward_node(xch[threadIdx.x / kNodeLanes], level_list[beg + k], root_level, threadIdx.x % kNodeLanes, pn, aux,
+                   inv_theta, G, gcnt, gmark);
 }
 
 // Depths d_lo .. 41 of a build whose counts stay on the device in one
 // workgroup, deepest first, a barrier between depths (see k_upward_tail).
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5)))
+__global__ __launch_bounds__(kBlock)
 void k_phys_upward_tail(int d_lo, const int32_t* __restrict__ level_list, PhysNode* __restrict__ pn,
                         PhysAux* __restrict__ aux, double inv_theta, int G, int32_t* __restrict__ gcnt,
                         uint32_t* __restrict__ gmark, const DevScalars* __restrict__ sc) {
+  __shared__ NodeXch xch[kBlock / kNodeLanes];
   if (sc->abort_flags) return;
   for (int d = kMaxLevels - 1; d >= d_lo; --d) {
     const int64_t beg = sc->level_off[d], cnt = sc->level_count[d];
     if (cnt == 0) continue;
-    for (int64_t k = threadIdx.x; k < cnt; k += kBlock)
-      phys_upward_node(level_list[beg + k], d == 0, pn, aux, inv_theta, G, gcnt, gmark);
+    for (int64_t k = threadIdx.x / kNodeLanes; k < cnt; k += kBlock / kNodeLanes)
+      phys_upward_node(xch[threadIdx.x / kNodeLanes], level_list[beg + k], d == 0, threadIdx.x % kNodeLanes, pn, aux,
+                       inv_theta, G, gcnt, gmark);
     __syncthreads();
   }
 }
 
 // Depth d of a build whose counts stay on the device (k_check): fixed grid
 // striding over the depth's extent in the node list.
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5)))
+__global__ __launch_bounds__(kBlock)
 void k_phys_upward_level(int d, const int32_t* __restrict__ level_list, PhysNode* __restrict__ pn,
                          PhysAux* __restrict__ aux, double inv_theta, int G, int32_t* __restrict__ gcnt,
                          uint32_t* __restrict__ gmark, const DevScalars* __restrict__ sc) {
+  __shared__ NodeXch xch[kBlock / kNodeLanes];
   if (sc->abort_flags) return;
   const int64_t beg = sc->level_off[d], cnt = sc->level_count[d];
-  for (int64_t k = (int64_t)blockIdx.x * kBlock + threadIdx.x; k < cnt; k += (int64_t)gridDim.x * kBlock)
-    phys_upward_node(level_list[beg + k], d == 0, pn, aux, inv_theta, G, gcnt, gmark);
+  for (int64_t k = ((int64_t)blockIdx.x * kBlock + threadIdx.x) / kNodeLanes; k < cnt;
+       k += (int64_t)gridDim.x * (kBlock / kNodeLanes))
+    phys_upward_node(xch[threadIdx.x / kNodeLanes], level_list[beg + k], d == 0, threadIdx.x % kNodeLanes, pn, aux,
+                     inv_theta, G, gcnt, gmark);
 }
 
 template <typename T>
@@ -819,14 +868,14 @@ void launch_phys_upward_tail(int d_lo, const int32_t* level_list, PhysNode* pn, 
 
 void launch_phys_upward_level(unsigned grid, int d, const int32_t* level_list, PhysNode* pn, void* aux, double theta,
                               int group_size, int32_t* gcnt, uint32_t* gmark, const DevScalars* sc, hipStream_t s) {
-  hipLaunchKernelGGL(k_phys_upward_level, dim3(grid), dim3(kBlock), 0, s, d, level_list, pn,
+  hipLaunchKernelGGL(k_phys_upward_level, dim3(grid * kNodeLanes), dim3(kBlock), 0, s, d, level_list, pn,
                      reinterpret_cast<PhysAux*>(aux), 1.0 / theta, group_size, gcnt, gmark, sc);
 }
 
 void launch_phys_upward(const int32_t* level_list, int64_t beg, int64_t cnt, int depth, PhysNode* pn, void* aux,
                         double theta, int group_size, int32_t* gcnt, uint32_t* gmark, hipStream_t s) {
   if (cnt > 0)
-    hipLaunchKernelGGL(k_phys_upward, dim3(grid_of(cnt, kBlock)), dim3(kBlock), 0, s, level_list, beg, cnt,
+    hipLaunchKernelGGL(k_phys_upward, dim3(grid_of(cnt, kBlock / kNodeLanes)), dim3(kBlock), 0, s, level_list, beg, cnt,
                        depth == 0, pn, reinterpret_cast<PhysAux*>(aux), 1.0 / theta, group_size, gcnt, gmark);
 }
 
