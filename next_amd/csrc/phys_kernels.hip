@@ -39,6 +39,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstddef>
+#include <cstdint>
 
 namespace nbx {
 namespace {
@@ -373,8 +374,105 @@ __device__ __forceinline__ double rsq<double>(double x) { return rsqrt(x); }
 // overflow.  All decisions are made in lockstep by one wave and compacted in
 // lane order, so the lists, and every sum, come out in the same order on
 // every run.
-template <typename T, int LIST, bool KICK, bool POT, bool COUNT>
-__global__ __launch_bounds__(kPhysBlock) void k_phys_walk(const Group* __restrict__ groups,
+template <typename T, int LIST>
+struct CellList {
+  V4<T> a[LIST];   // relative centre of mass, mass
+  V4<T> b[LIST];   // qxx qyy qxy qxz
+  V2<T> q[LIST];   // qyz qzz
+};
+template <typename T, int LIST>
+struct BodyList {
+  V4<T> p[LIST];   // relative position, mass
+};
+
+// What a lane needs of its target to evaluate list entries.
+template <typename T>
+struct WalkTarget {
+  T x, y, z, e2;   // relative to the group's centre; softening squared
+  int width, parts, part;
+};
+
+// The sum over the n entries of a list for the wave's targets, every product
+// fused into the sum it feeds: a = m d / r^3 + 2.5 (d.Q.d) d / r^7 - Q d / r^5
+// and phi = -m / r - 0.5 (d.Q.d) / r^5, d from the target to the cell.
+template <bool POT, typename T, int LIST>
+__device__ __forceinline__ void sum_cells(const CellList<T, LIST>& L, int n, const WalkTarget<T>& t, T& fx, T& fy,
+                                          T& fz, T& fp) {
+  auto term = [&](int k) {
+    const V4<T> a = L.a[k];
+    const V4<T> b = L.b[k];
+    const V2<T> q = L.q[k];
+    const T dx = a.x - t.x, dy = a.y - t.y, dz = a.z - t.z;
+    const T r2 = fma(dz, dz, fma(dy, dy, fma(dx, dx, t.e2)));
+    const T ri = rsq<T>(r2);
+    const T ri2 = ri * ri;
+    const T ri3 = ri2 * ri;
+    const T ri5 = ri3 * ri2;
+    const T qdx = fma(b.w, dz, fma(b.z, dy, b.x * dx));
+    const T qdy = fma(q.x, dz, fma(b.y, dy, b.z * dx));
+    const T qdz = fma(q.y, dz, fma(q.x, dy, b.w * dx));
+    const T dqd = fma(dz, qdz, fma(dy, qdy, dx * qdx));
+    const T u = dqd * ri5;
+    const T s = fma((T)2.5 * ri2, u, a.w * ri3);
+    fx = fma(-ri5, qdx, fma(s, dx, fx));
+    fy = fma(-ri5, qdy, fma(s, dy, fy));
+    fz = fma(-ri5, qdz, fma(s, dz, fz));
+    if (POT) fp = fma((T)-0.5, u, fma(-a.w, ri, fp));
+  };
+  // A group of more than 32 targets has one lane per target, and every lane
+  // takes every entry: the loop is wave-uniform (scalar control, one LDS
+  // address for all lanes).
+  if (t.parts == 1) {
+#pragma unroll 2
+    for (int k = 0; k < n; ++k) term(k);
+  } else {
+    for (int k = t.part; k < n; k += t.parts) term(k);
+    combine_parts(fx, fy, fz, fp, t.width);
+  }
+}
+
+template <bool POT, typename T, int LIST>
+__device__ __forceinline__ void sum_bodies(const BodyList<T, LIST>& L, int n, const WalkTarget<T>& t, T& fx, T& fy,
+                                           T& fz, T& fp) {
+  auto term = [&](int k) {
+    const V4<T> b = L.p[k];
+    const T dx = b.x - t.x, dy = b.y - t.y, dz = b.z - t.z;
+    const T r2 = fma(dz, dz, fma(dy, dy, fma(dx, dx, t.e2)));
+    const T ri = rsq<T>(r2);
+    const T mri = b.w * ri;
+    const T mr3 = mri * (ri * ri);
+    fx = fma(mr3, dx, fx);
+    fy = fma(mr3, dy, fy);
+    fz = fma(mr3, dz, fz);
+    if (POT) fp -= mri;
+  };
+  if (t.parts == 1) {
+#pragma unroll 2
+    for (int k = 0; k < n; ++k) term(k);
+  } else {
+    for (int k = t.part; k < n; k += t.parts) term(k);
+    combine_parts(fx, fy, fz, fp, t.width);
+  }
+}
+
+// Counters in LDS that waves of a workgroup wait on.
+__device__ __forceinline__ int lds_get(const int* p) {
+  return __builtin_amdgcn_readfirstlane(__hip_atomic_load(p, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP));
+}
+__device__ __forceinline__ void lds_put(int* p, int v) {   // after all the wave's LDS accesses before it
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+  if (lane_id() == 0) __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
+// EVAL > 0: the workgroup has EVAL more waves.  The first wave walks and hands
+// every full list over as a job; job j is summed by wave 1 + j % EVAL, and the
+// sums are added to the totals (LDS) in the order of the jobs, so the result is
+// that of one wave, bit for bit.  A buffer is filled again when the job that
+// held it has been added.  Every wait ends: the walk waits for jobs handed over
+// before, a job only for the ones before it, and the waves beyond the last job
+// for the walk's end.
+template <typename T, int LIST, bool KICK, bool POT, bool COUNT, int EVAL>
+__global__ __launch_bounds__(kPhysBlock * (1 + EVAL)) void k_phys_walk(const Group* __restrict__ groups,
                                                           const PhysNode* __restrict__ pn, StateArrays st,
                                                           SysArrays sy, double eps, int nleaf,
                                                           double* __restrict__ ax, double* __restrict__ ay,
@@ -385,12 +483,19 @@ __global__ __launch_bounds__(kPhysBlock) void k_phys_walk(const Group* __restric
   __shared__ int32_t stk_e[kPhysStack];
   __shared__ int32_t bfirst[kWave];      // buckets of the current step: first body,
   __shared__ int32_t bstart[kWave];      //   offset in the step's flattened body list
-  __shared__ V4<T> ca[LIST];             // cell: relative centre of mass, mass
-  __shared__ V4<T> cb[LIST];             // cell: qxx qyy qxy qxz
-  __shared__ V2<T> cq[LIST];             // cell: qyz qzz
-  __shared__ V4<T> pl[LIST];             // body: relative position, mass
+  // (Four buffers of 5 + 2 KB leave a CU 5 workgroups, as their registers do;
+  // FP64's three of 10 + 4 KB, 3.)
+  constexpr int kBufs = !EVAL ? 1 : sizeof(T) == 4 ? 4 : 3, kSums = POT ? 4 : 3;
+  constexpr int kJobs = 8;                            // at most 2 kBufs jobs are out
+  static_assert(2 * kBufs <= kJobs && kBufs <= 8, "job ring");
+  __shared__ CellList<T, LIST> cells[kBufs];
+  __shared__ BodyList<T, LIST> bodies[kBufs];
+  __shared__ int job_at[EVAL ? kJobs : 1];            // job j: entries, buffer, kind at j % kJobs
+  __shared__ int buf_job[EVAL ? 2 * kBufs : 1];       // last job that held a buffer (cells, bodies)
+  __shared__ int handed, added, last;                 // jobs handed over, added; how many there are in the end
+  __shared__ double total[EVAL ? kSums : 1][kWave];
 
-  const int lane = threadIdx.x;
+  const int lane = lane_id(), wave = EVAL ? __builtin_amdgcn_readfirstlane(threadIdx.x / kWave) : 0;
   // The group count comes from the device (the compaction that wrote it ran
   // earlier on this stream), so the host need not read it back first; the
   // grid (a multiple of 8) is sized from a bound.  Blocks are dealt to the 8
@@ -416,7 +521,7 @@ __global__ __launch_bounds__(kPhysBlock) void k_phys_walk(const Group* __restric
     const int64_t ii = slot < g.count ? i : g.first;
     const double px = st.x[ii], py = st.y[ii], pz = st.z[ii];
     const uint64_t ltmask = lanemask_lt();
-    const int32_t root = sy.sroot[g.sys], total = sy.send[g.sys];   // this system's tree
+    const int32_t root = sy.sroot[g.sys], tree_end = sy.send[g.sys];   // this system's tree
 
     // group bounding box
     double lo[3] = {px, py, pz}, hi[3] = {px, py, pz};
@@ -433,8 +538,7 @@ __global__ __launch_bounds__(kPhysBlock) void k_phys_walk(const Group* __restric
     const float hx = (float)(0.5 * (hi[0] - lo[0])) * (1.0f + 1e-6f);
     const float hy = (float)(0.5 * (hi[1] - lo[1])) * (1.0f + 1e-6f);
     const float hz = (float)(0.5 * (hi[2] - lo[2])) * (1.0f + 1e-6f);
-    const T tx = (T)(px - gcx), ty = (T)(py - gcy), tz = (T)(pz - gcz);
-    const T e2 = (T)(eps * eps);
+    const WalkTarget<T> tg{(T)(px - gcx), (T)(py - gcy), (T)(pz - gcz), (T)(eps * eps), width, parts, part};
     // Relative criterion (amag != null): a cell that passes the geometric test
     // is accepted only if its first neglected (octupole) term, ~ m bmax^3 / d^5,
     // is at most alpha times the smallest previous |a| of the group:
@@ -447,84 +551,83 @@ __global__ __launch_bounds__(kPhysBlock) void k_phys_walk(const Group* __restric
       arel = rel2 * am * am;
     }
 
+    if (EVAL) {
+      if (wave == 0) {
+        if (lane < 2 * kBufs) buf_job[lane] = -1;
+        if (lane == 0) { handed = 0; added = 0; last = INT32_MAX; }
+        for (int k = 0; k < kSums; ++k) total[k][lane] = 0.0;
+      }
+      __syncthreads();
+      if (wave > 0) {
+        for (int j = wave - 1;; j += EVAL) {
+          bool none = false;
+          while (lds_get(&handed) <= j) {
+            none = lds_get(&last) <= j;
+            if (none) break;
+            __builtin_amdgcn_s_sleep(1);
+          }
+          if (none) break;
+          const int job = __builtin_amdgcn_readfirstlane(job_at[j % kJobs]);
+          const int buf = job >> 1 & 7, cnt = job >> 4;
+          T fx = 0, fy = 0, fz = 0, fp = 0;
+          if (job & 1) sum_bodies<POT>(bodies[buf], cnt, tg, fx, fy, fz, fp);
+          else sum_cells<POT>(cells[buf], cnt, tg, fx, fy, fz, fp);
+          while (lds_get(&added) != j) __builtin_amdgcn_s_sleep(1);
+          total[0][lane] += (double)fx; total[1][lane] += (double)fy; total[2][lane] += (double)fz;
+          if (POT) total[kSums - 1][lane] += (double)fp;
+          lds_put(&added, j + 1);
+        }
+        __syncthreads();                                   // the group's end
+        continue;
+      }
+    }
+
     double Ax = 0, Ay = 0, Az = 0, P = 0;
     uint32_t ncell_tot = 0, npart_tot = 0, niter = 0, nopen = 0;
-    int nc = 0, np = 0;
+    int nc = 0, np = 0, cbuf = 0, bbuf = 0, jobs = 0;
 
-    // The terms of list entry k added to the running sums, every product
-    // fused into the sum it feeds: a = m d / r^3 + 2.5 (d.Q.d) d / r^7 - Q d / r^5
-    // and phi = -m / r - 0.5 (d.Q.d) / r^5, d from the target to the cell.
-    auto cell_term = [&](int k, T& fx, T& fy, T& fz, T& fp) {
-      const V4<T> a = ca[k];
-      const V4<T> b = cb[k];
-      const V2<T> q = cq[k];
-      const T dx = a.x - tx, dy = a.y - ty, dz = a.z - tz;
-      const T r2 = fma(dz, dz, fma(dy, dy, fma(dx, dx, e2)));
-      const T ri = rsq<T>(r2);
-      const T ri2 = ri * ri;
-      const T ri3 = ri2 * ri;
-      const T ri5 = ri3 * ri2;
-      const T qdx = fma(b.w, dz, fma(b.z, dy, b.x * dx));
-      const T qdy = fma(q.x, dz, fma(b.y, dy, b.z * dx));
-      const T qdz = fma(q.y, dz, fma(q.x, dy, b.w * dx));
-      const T dqd = fma(dz, qdz, fma(dy, qdy, dx * qdx));
-      const T u = dqd * ri5;
-      const T s = fma((T)2.5 * ri2, u, a.w * ri3);
-      fx = fma(-ri5, qdx, fma(s, dx, fx));
-      fy = fma(-ri5, qdy, fma(s, dy, fy));
-      fz = fma(-ri5, qdz, fma(s, dz, fz));
-      if (POT) fp = fma((T)-0.5, u, fma(-a.w, ri, fp));
-    };
-    auto body_term = [&](int k, T& fx, T& fy, T& fz, T& fp) {
-      const V4<T> b = pl[k];
-      const T dx = b.x - tx, dy = b.y - ty, dz = b.z - tz;
-      const T r2 = fma(dz, dz, fma(dy, dy, fma(dx, dx, e2)));
-      const T ri = rsq<T>(r2);
-      const T mri = b.w * ri;
-      const T mr3 = mri * (ri * ri);
-      fx = fma(mr3, dx, fx);
-      fy = fma(mr3, dy, fy);
-      fz = fma(mr3, dz, fz);
-      if (POT) fp -= mri;
-    };
-    // A group of more than 32 targets has one lane per target, and every
-    // lane takes every entry: the loop is wave-uniform (scalar control, one
-    // LDS address for all lanes).
-    auto flush_cells = [&]() {
-      __syncthreads();
-      T fx = 0, fy = 0, fz = 0, fp = 0;
-      if (parts == 1) {
-#pragma unroll 2
-        for (int k = 0; k < nc; ++k) cell_term(k, fx, fy, fz, fp);
-      } else {
-        for (int k = part; k < nc; k += parts) cell_term(k, fx, fy, fz, fp);
-        combine_parts(fx, fy, fz, fp, width);
+    auto hand_over = [&](int kind, int& buf, int cnt) {
+      if (lane == 0) {
+        job_at[jobs % kJobs] = kind | buf << 1 | cnt << 4;
+        buf_job[kind * kBufs + buf] = jobs;
       }
-      Ax += (double)fx; Ay += (double)fy; Az += (double)fz;
-      if (POT) P += (double)fp;
+      lds_put(&handed, ++jobs);
+      buf = buf + 1 < kBufs ? buf + 1 : 0;
+      wave_order();
+      const int before = __builtin_amdgcn_readfirstlane(buf_job[kind * kBufs + buf]);
+      while (lds_get(&added) <= before) __builtin_amdgcn_s_sleep(1);
+    };
+    auto flush_cells = [&]() {
+      wave_order();
+      if (EVAL) {
+        hand_over(0, cbuf, nc);
+      } else {
+        T fx = 0, fy = 0, fz = 0, fp = 0;
+        sum_cells<POT>(cells[0], nc, tg, fx, fy, fz, fp);
+        Ax += (double)fx; Ay += (double)fy; Az += (double)fz;
+        if (POT) P += (double)fp;
+      }
       if (COUNT) ncell_tot += nc;
-      __syncthreads();
+      wave_order();
       nc = 0;
     };
     auto flush_parts = [&]() {
-      __syncthreads();
-      T fx = 0, fy = 0, fz = 0, fp = 0;
-      if (parts == 1) {
-#pragma unroll 2
-        for (int k = 0; k < np; ++k) body_term(k, fx, fy, fz, fp);
+      wave_order();
+      if (EVAL) {
+        hand_over(1, bbuf, np);
       } else {
-        for (int k = part; k < np; k += parts) body_term(k, fx, fy, fz, fp);
-        combine_parts(fx, fy, fz, fp, width);
+        T fx = 0, fy = 0, fz = 0, fp = 0;
+        sum_bodies<POT>(bodies[0], np, tg, fx, fy, fz, fp);
+        Ax += (double)fx; Ay += (double)fy; Az += (double)fz;
+        if (POT) P += (double)fp;
       }
-      Ax += (double)fx; Ay += (double)fy; Az += (double)fz;
-      if (POT) P += (double)fp;
       if (COUNT) npart_tot += np;
-      __syncthreads();
+      wave_order();
       np = 0;
     };
 
-    int32_t cur = lane == 0 ? root : total;                  // this lane's range [cur, end)
-    int32_t end = total;
+    int32_t cur = lane == 0 ? root : tree_end;                  // this lane's range [cur, end)
+    int32_t end = tree_end;
     int sp = 0;                                              // donated ranges on the stack
     for (;;) {
       // idle lanes take ranges from the top of the stack
@@ -549,7 +652,7 @@ __global__ __launch_bounds__(kPhysBlock) void k_phys_walk(const Group* __restric
         ncx = nd.cx; ncy = nd.cy; ncz = nd.cz;
         const float rx = (float)(ncx - gcx), ry = (float)(ncy - gcy), rz = (float)(ncz - gcz);
         const float dx = fmaxf(fabsf(rx) - hx, 0.f), dy = fmaxf(fabsf(ry) - hy, 0.f), dz = fmaxf(fabsf(rz) - hz, 0.f);
-        const float d2 = dx * dx + dy * dy + dz * dz;
+        const float d2 = fmaf(dz, dz, fmaf(dx, dx, dy * dy));
         cnt = nd.count;
         first = nd.first;
         nskip = nd.skip > cur ? nd.skip : cur + 1;           // skip > cur by construction
@@ -571,9 +674,10 @@ __global__ __launch_bounds__(kPhysBlock) void k_phys_walk(const Group* __restric
       if (acc) {
         const int pos = nc + (int)__popcll(am & ltmask);
         const PhysNode& nd = pn[cur];
-        ca[pos] = V4<T>{(T)(ncx - gcx), (T)(ncy - gcy), (T)(ncz - gcz), (T)nd.m};
-        cb[pos] = V4<T>{(T)nd.qxx, (T)nd.qyy, (T)nd.qxy, (T)nd.qxz};
-        cq[pos] = V2<T>{(T)nd.qyz, (T)(-((double)nd.qxx + (double)nd.qyy))};
+        CellList<T, LIST>& L = cells[EVAL ? cbuf : 0];
+        L.a[pos] = V4<T>{(T)(ncx - gcx), (T)(ncy - gcy), (T)(ncz - gcz), (T)nd.m};
+        L.b[pos] = V4<T>{(T)nd.qxx, (T)nd.qyy, (T)nd.qxy, (T)nd.qxz};
+        L.q[pos] = V2<T>{(T)nd.qyz, (T)(-((double)nd.qxx + (double)nd.qyy))};
       }
       nc += (int)__popcll(am);
       // opened nodes hand [skip, end) to the stack while it has room
@@ -598,7 +702,7 @@ __global__ __launch_bounds__(kPhysBlock) void k_phys_walk(const Group* __restric
         bfirst[j] = first;
         bstart[j] = (int)(bincl - cb_n);
       }
-      __syncthreads();
+      wave_order();
       for (int base = 0; base < nbody; base += kWave) {
         if (np > LIST - kWave) flush_parts();
         const int t = base + lane;
@@ -609,14 +713,21 @@ __global__ __launch_bounds__(kPhysBlock) void k_phys_walk(const Group* __restric
             if (bstart[mid] <= t) lo_j = mid; else hi_j = mid - 1;
           }
           const int32_t b = bfirst[lo_j] + (t - bstart[lo_j]);
-          pl[np + lane] = V4<T>{(T)(st.x[b] - gcx), (T)(st.y[b] - gcy), (T)(st.z[b] - gcz), (T)st.m[b]};
+          bodies[EVAL ? bbuf : 0].p[np + lane] = V4<T>{(T)(st.x[b] - gcx), (T)(st.y[b] - gcy), (T)(st.z[b] - gcz), (T)st.m[b]};
         }
         np += nbody - base < kWave ? nbody - base : kWave;
       }
-      __syncthreads();
+      wave_order();
     }
     if (nc) flush_cells();
     if (np) flush_parts();
+    if (EVAL) {
+      lds_put(&last, jobs);
+      while (lds_get(&added) < jobs) __builtin_amdgcn_s_sleep(1);
+      Ax = total[0][lane]; Ay = total[1][lane]; Az = total[2][lane];
+      if (POT) P = total[kSums - 1][lane];
+      __syncthreads();                                     // the group's end
+    }
 
     double v2 = 0.0;
     if (valid) {
@@ -647,7 +758,7 @@ __global__ __launch_bounds__(kPhysBlock) void k_phys_walk(const Group* __restric
       atomicAdd(&sc->n_open, (unsigned long long)nopen);
       atomicAdd(&sc->n_iter, (unsigned long long)niter);
     }
-    __syncthreads();                                       // the next group reuses the LDS lists
+    wave_order();                                          // the next group reuses the LDS lists
   }
 }
 
@@ -791,20 +902,44 @@ __global__ __launch_bounds__(kBlock) void k_energy_final(const double* __restric
   for (int k = 0; k < 5; ++k) out[5 * s + k] = t[k];
 }
 
+// Workgroups of 4 waves for launches of at most kSplitGroups groups (10 waves
+// per SIMD of the walk alone, more than its registers allow; the bound that
+// stands in for a count the host does not have yet is a quarter above it), the
+// default list size.  Few groups leave most SIMDs with one wave at most, and a wave's time
+// is then its evaluation's latency (about 2/3) plus its walk's.  Walk of a
+// single system, one wave per group against 1 + 3 waves (FP32 / FP64):
+//      2,000 bodies,     55 groups    132 ->  70 us     167 ->   77 us
+//     16,384            378           584 -> 205        771 ->  319
+//     65,536          1,476           381 -> 211        561 ->  417
+//    200,000          4,424           573 -> 484      1,074 -> 1,066
+//    327,680 (20)     7,549           842 -> 652      1,528 -> 1,370
+//    524,288         11,522         1,200 -> 1,193    2,562 -> 2,730
+//  4,194,304                        9,010 -> 9,930
+// Two evaluating waves: 275 us (FP32, 16,384 bodies), five or seven: 208.
+constexpr int kWalkEval = 3;
+constexpr unsigned kSplitGroups = 10240;
+
 template <typename T, int LIST>
 void walk_dispatch(unsigned nb, const Group* groups, const PhysNode* pn, const StateArrays& st, const SysArrays& sy,
                    double eps, int nleaf, double* ax, double* ay, double* az, double* pot, DevScalars* sc, bool kick,
                    bool count, const float* amag, float rel2, float th2, hipStream_t s) {
-#define NBX_PW(K, P, C)                                                                                          \
-  hipLaunchKernelGGL((k_phys_walk<T, LIST, K, P, C>), dim3(nb), dim3(kPhysBlock), 0, s, groups, pn, st, sy, eps, \
-                     nleaf, ax, ay, az, pot, sc, amag, rel2, th2)
-  const bool p = pot != nullptr;
+#define NBX_PW(K, P, C, E)                                                                                      \
+  hipLaunchKernelGGL((k_phys_walk<T, LIST, K, P, C, E>), dim3(nb), dim3(kPhysBlock * (1 + (E))), 0, s, groups, \
+                     pn, st, sy, eps, nleaf, ax, ay, az, pot, sc, amag, rel2, th2)
+  constexpr int kSplit = LIST == 128 ? kWalkEval : 0;
+  const bool p = pot != nullptr, split = kSplit > 0 && !count && nb <= kSplitGroups;
   if (kick) {
-    if (count) NBX_PW(true, false, true); else NBX_PW(true, false, false);
+    if (count) NBX_PW(true, false, true, 0);
+    else if (split) NBX_PW(true, false, false, kSplit);
+    else NBX_PW(true, false, false, 0);
   } else if (p) {
-    if (count) NBX_PW(false, true, true); else NBX_PW(false, true, false);
+    if (count) NBX_PW(false, true, true, 0);
+    else if (split) NBX_PW(false, true, false, kSplit);
+    else NBX_PW(false, true, false, 0);
   } else {
-    if (count) NBX_PW(false, false, true); else NBX_PW(false, false, false);
+    if (count) NBX_PW(false, false, true, 0);
+    else if (split) NBX_PW(false, false, false, kSplit);
+    else NBX_PW(false, false, false, 0);
   }
 #undef NBX_PW
 }
