@@ -20,9 +20,14 @@
 
 #include <algorithm>
 #include <chrono>
+#include <condition_variable>
 #include <cstdio>
 #include <cstring>
+#include <mutex>
+#include <new>
 #include <string>
+#include <system_error>
+#include <thread>
 #include <vector>
 
 #include "common.hpp"
@@ -44,6 +49,11 @@ struct DBuf {
 enum { EV_START, EV_KICK, EV_KEYS, EV_SORT, EV_BUILD, EV_UPWARD, EV_WALK0, EV_WALK, EV_COUNT };
 constexpr int kStateArrays = 10;   // x y z vx vy vz m type id sys
 constexpr int64_t kOutChunk = 65536;   // bodies per chunk of a download (3 MB of six arrays)
+// Bodies from which two more threads help with the copies.  Downloads of the
+// six arrays, alone / with two / with five helpers: 200,000 bodies 0.34 / 0.34 /
+// 0.37 ms, 366,000 0.67 / 0.52 / 0.54, 2^20 3.6 / 2.2 / 2.1, 4,194,304 13.7 /
+// 7.6 / 6.6.
+constexpr int64_t kOutTeam = 262144;
 
 }  // namespace
 
@@ -1017,6 +1027,80 @@ nbx_status fetch(nbx_ctx* c, const void* dev, size_t bytes, const void** staged)
   return NBX_OK;
 }
 
+// Threads that help one download copy its chunks into the caller's arrays,
+// each a part of the chunk's values (array after array, so that a thread
+// mostly writes pages of its own: fresh ones are zeroed as they are touched,
+// which is half of the time).  Fewer, or none, where threads cannot be started.
+class CopyTeam {
+ public:
+  explicit CopyTeam(int helpers) {
+    try {
+      threads_.reserve((size_t)helpers);
+      for (int t = 1; t <= helpers; ++t) {
+        threads_.emplace_back([this, t] { help(t); });
+        ++started_;
+      }
+    } catch (const std::system_error&) {
+    } catch (const std::bad_alloc&) {
+    }
+  }
+  CopyTeam(const CopyTeam&) = delete;
+  CopyTeam& operator=(const CopyTeam&) = delete;
+  ~CopyTeam() {
+    {
+      std::lock_guard<std::mutex> lk(mu_);
+      stop_ = true;
+    }
+    go_.notify_all();
+    for (std::thread& t : threads_) t.join();
+  }
+  // dst[q][j0 + i] = from[q len + i] for q < m, i < len
+  void copy(const double* from, double* const* dst, int m, int64_t j0, int64_t len) {
+    {
+      std::lock_guard<std::mutex> lk(mu_);
+      from_ = from; dst_ = dst; m_ = m; j0_ = j0; len_ = len; parts_ = started_ + 1;
+      left_ = started_;
+      ++round_;
+    }
+    go_.notify_all();
+    part(0);
+    std::unique_lock<std::mutex> lk(mu_);
+    done_.wait(lk, [this] { return left_ == 0; });
+  }
+
+ private:
+  void part(int t) {
+    const int64_t n = m_ * len_, e = n * (t + 1) / parts_;
+    for (int64_t b = n * t / parts_; b < e;) {
+      const int64_t q = b / len_, i = b - q * len_, cnt = std::min(len_ - i, e - b);
+      std::memcpy(dst_[q] + j0_ + i, from_ + b, (size_t)cnt * 8);
+      b += cnt;
+    }
+  }
+  void help(int t) {
+    uint64_t seen = 0;
+    std::unique_lock<std::mutex> lk(mu_);
+    for (;;) {
+      go_.wait(lk, [&] { return stop_ || round_ != seen; });
+      if (stop_) return;
+      seen = round_;
+      lk.unlock();
+      part(t);
+      lk.lock();
+      if (--left_ == 0) done_.notify_one();
+    }
+  }
+  std::mutex mu_;
+  std::condition_variable go_, done_;
+  std::vector<std::thread> threads_;
+  int started_ = 0, left_ = 0, parts_ = 1, m_ = 0;
+  bool stop_ = false;
+  uint64_t round_ = 0;
+  const double* from_ = nullptr;
+  double* const* dst_ = nullptr;
+  int64_t j0_ = 0, len_ = 0;
+};
+
 // Copy bodies [off, off + cnt) of key-order device arrays out, each at its
 // upload index minus `base` (a null `outs` entry is skipped).  The upload
 // indices of those slots must be a permutation of [base, base + cnt); anything
@@ -1046,6 +1130,7 @@ nbx_status copy_out(nbx_ctx* c, int64_t off, int64_t cnt, int64_t base, const do
   *bad = 0;
   uint32_t* inv = P<uint32_t>(c->idx[0]);                  // sort scratch, free between steps
   launch_out_index(cnt, id, (int32_t)base, inv, bad, c->stream);
+  CopyTeam team(cnt >= kOutTeam ? std::min(m, 3) - 1 : 0);
   const int64_t nchunks = div_up(cnt, chunk);
   for (int64_t k = 0; k <= nchunks; ++k) {
     if (k < nchunks) {
@@ -1061,7 +1146,7 @@ nbx_status copy_out(nbx_ctx* c, int64_t off, int64_t cnt, int64_t base, const do
         return fail(c, NBX_ERR_STATE, "body indices on the device are not a permutation");
       }
       const double* from = reinterpret_cast<const double*>(stage + ((k - 1) & 1) * half);
-      for (int q = 0; q < m; ++q) std::memcpy(dst[q] + j0, from + q * len, (size_t)len * 8);
+      team.copy(from, dst, m, j0, len);
     }
   }
   return NBX_OK;

@@ -1,4 +1,5 @@
-"""Downloads around the chunk size: the state comes back in upload order,
+"""Downloads around the chunk size, and around the size from which further
+threads help (four chunks): the state comes back in upload order,
 bit for bit, after the engine has put the bodies into key order, for single
 systems, systems of a batch (offset slots) and skipped arrays."""
 import ctypes as C
@@ -23,7 +24,8 @@ def columns(p):
     return np.stack([p.x, p.y, p.z, p.vx, p.vy, p.vz])
 
 
-@pytest.mark.parametrize("n", [1, 2, 255, CHUNK - 1, CHUNK, CHUNK + 1, 2 * CHUNK, 3 * CHUNK + 5])
+@pytest.mark.parametrize("n", [1, 2, 255, CHUNK - 1, CHUNK, CHUNK + 1, 2 * CHUNK, 3 * CHUNK + 5, 4 * CHUNK - 1,
+                               4 * CHUNK, 4 * CHUNK + 1, 7 * CHUNK + 3])
 def test_upload_order(n):
     p = bodies(n, n)
     with Engine(theta=0.9) as e:
