@@ -12,7 +12,8 @@ from next_amd.nbx import MODE_PHYSICS, PREC_MIXED, Engine, lib
 
 pytestmark = pytest.mark.gpu
 
-CHUNK = 65536
+CHUNK = 65536                           # from four chunks on; below, chunks of SMALL bodies
+SMALL = 16384
 
 
 def bodies(n, seed):
@@ -24,8 +25,8 @@ def columns(p):
     return np.stack([p.x, p.y, p.z, p.vx, p.vy, p.vz])
 
 
-@pytest.mark.parametrize("n", [1, 2, 255, CHUNK - 1, CHUNK, CHUNK + 1, 2 * CHUNK, 3 * CHUNK + 5, 4 * CHUNK - 1,
-                               4 * CHUNK, 4 * CHUNK + 1, 7 * CHUNK + 3])
+@pytest.mark.parametrize("n", [1, 2, 255, SMALL - 1, SMALL, SMALL + 1, CHUNK - 1, CHUNK, CHUNK + 1, 2 * CHUNK,
+                               3 * CHUNK + 5, 4 * CHUNK - 1, 4 * CHUNK, 4 * CHUNK + 1, 7 * CHUNK + 3])
 def test_upload_order(n):
     p = bodies(n, n)
     with Engine(theta=0.9) as e:
