@@ -39,7 +39,7 @@ sys.path.insert(0, ROOT)
 from next_amd import ic  # noqa: E402
 
 FP64_PEAK_TFLOPS = 78.6   # MI355X FP64 vector (and matrix) peak
-FP32_PEAK_TFLOPS = 157.3  # MI355X FP32 vector peak (packed FP32; unpacked issue gives half)
+FP32_PEAK_TFLOPS = 157.3  # MI355X FP32 vector peak
 HBM_PEAK_GBS = 8000.0
 FLOPS_PP, FLOPS_PC = 19, 55
 # The physics walk is counted by the same convention (FMA = 2, rsqrt = 1,

@@ -34,8 +34,8 @@ __host__ __device__ inline double leaf_mass(const PhysNode& nd) {
   return m;
 }
 
-constexpr int kPhysBlock = 64;      // one wave = one group of targets
-// Per-wave LDS (7.4 KB with these sizes) bounds the walk's occupancy at
+constexpr int kPhysBlock = 64;      // one wave = one group of targets (further waves: k_phys_walk)
+// Per-wave LDS (7.9 KB with these sizes) bounds the walk's occupancy at
 // about 5 waves per SIMD; a 256-entry stack and body list (11 KB) allowed 3.
 // Entries of the per-wave LDS lists (accepted cells, bodies of accepted
 // buckets) a walk collects before it evaluates them: a walk setting

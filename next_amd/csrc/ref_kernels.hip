@@ -740,7 +740,7 @@ __global__ __launch_bounds__(kBlock) void k_upward_unit(UnitArgs a, RefNode* __r
                                                         const double* __restrict__ root) {
   __shared__ UnitMoments lm;
   const double half = root[3];
-  upward_unit<1, kUnitNodes>(
+  upward_unit<kUnitNodes>(
       a,
       [&](const UnitView& v, int32_t k) {
         const RefNode& nd = nodes[k];
@@ -748,7 +748,7 @@ __global__ __launch_bounds__(kBlock) void k_upward_unit(UnitArgs a, RefNode* __r
         lm.m[s] = nd.m; lm.x[s] = nd.cx; lm.y[s] = nd.cy; lm.z[s] = nd.cz;
         lm.first[s] = nd.first;
       },
-      [&](const UnitView& v, int32_t id, int32_t end, int d, int) {
+      [&](const UnitView& v, int32_t id, int32_t end, int d) {
         upward_node(v, &lm, id, end, d, nodes, heads, inv_theta, half, sys, root);
       });
 }
@@ -757,7 +757,7 @@ __global__ __launch_bounds__(kOverBlock) void k_upward_over(UnitArgs a, SysArray
                                                             WalkHead* __restrict__ heads, double inv_theta,
                                                             const int32_t* __restrict__ sys) {
   const double half = sy.root[3];
-  upward_over<1>(a, sy, [&](const UnitView& v, int32_t id, int32_t end, int d, int) {
+  upward_over(a, sy, [&](const UnitView& v, int32_t id, int32_t end, int d) {
     upward_node(v, nullptr, id, end, d, nodes, heads, inv_theta, half, sys, sy.root);
   });
 }
@@ -882,7 +882,6 @@ __device__ __forceinline__ void walk_common(const int32_t* list, int n, int part
                                             const RefNode* __restrict__ nodes, uint32_t zoff, double px, double py,
                                             double pz, double mip, Sum3& a) {
   if (parts == 1) {
-#pragma unroll 2
     for (int k = 0; k < n; ++k) {
       const int32_t e = __builtin_amdgcn_readfirstlane(list[k]);
       const RefNode& nd = node_at(nodes, (uint32_t)e << 7);

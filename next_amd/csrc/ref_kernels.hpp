@@ -152,17 +152,25 @@ void launch_out_gather(int64_t j0, int64_t len, int64_t cnt, const uint32_t* inv
 // than 64 puts 64 / width lanes on each target).  It depends on the system
 // alone, so a system's sums are the same alone and in a batch.  Narrow
 // groups give a small system enough waves and short ones; wide groups share
-// more of the traversal.  Measured walk times (us, theta 0.5, Plummer), width
-// 64 / 32 / 16 / 8: n = 1,000 150 / 92 / 69 / 54; 4,000 182 / 118 / 82 / 67;
-// 16,000 196 / 148 / 108 / 92 (64 such systems in one batch 1,519 / 1,665 /
-// 1,832 / 2,358, so 16 there); 64,000 242 / 188 / 177 / 232; 128,000 299 / 294
-// / 319 / 387; 256,000 516 / 536 / 588 / 732; 2^20 (cold sphere) 1,359 / 1,403
-// / 1,636 / 2,256.  At theta 0.3 each target's own walk is long and 16 is
-// fastest or within 3 % of it from 32,000 bodies on (256,000: 1,981 / 1,719 /
-// 1,611 / 1,612).
+// more of the traversal, which is what a batch of many systems needs, the more
+// so the larger theta.  The lines lie where the narrower groups would make
+// such a batch slower than one union traversal per 64 targets was ("u").
+// Walk (us, Plummer spheres), width u / 8 / 16 / 32 / 64:
+//   theta  n        alone                          batch
+//   0.3    2,000    502 /  97 / 140 / 223 / 397    512: 3,283 / 3,295 / 3,111 / 3,262 / 3,543
+//   0.3    16,384   981 / 212 / 239 / 410 / 565     64: 5,595 / 4,946 / 4,868 / 5,201 / 5,561
+//   0.4    2,000    343 /  76 / 107 / 134 / 231    512: 2,143 / 2,506 / 2,068 / 2,012 / 2,077
+//   0.5    1,000    237 /  56 /  72 / 103 / 152    512:   786 /   902 /   705 /   644 /   675
+//   0.5    2,000    270 /  84 /  81 / 120 / 181    512: 1,585 / 2,115 / 1,632 / 1,423 / 1,404
+//   0.5    16,384   369 /  93 / 117 / 141 / 205     64: 2,047 / 2,579 / 2,016 / 1,724 / 1,557
+//   0.5    65,536   426 / 217 / 171 / 185 / 252     16: 2,196 / 2,810 / 2,127 / 1,833 / 1,562
+//   0.5    100,000  490 / 326 / 276 / 248 / 262     12: 2,538 / 3,368 / 2,533 / 2,182 / 1,742
+//   0.5    200,000  677 / 611 / 491 / 461 / 410
+//   0.7    16,384   201 /  69 /  75 / 100 / 131     64: 1,267 / 2,030 / 1,435 / 1,112 /   825
+//   0.7    65,536   238 / 173 / 122 / 126 / 170     16: 1,354 / 2,189 / 1,518 / 1,170 /   810
 inline int32_t walk_width(int64_t n, double theta) {
-  if (n <= 4096) return 8;
-  if (n <= 98304 || theta < 0.4) return 16;
+  if (theta <= 0.32 && n <= 4096) return 8;
+  if (theta < 0.4 || (theta <= 0.55 && n <= 98304)) return 16;
   return n <= 196608 ? 32 : 64;
 }
 void launch_walk(const Group* groups, int64_t ngroups, const RefNode* nodes, const WalkHead* heads,

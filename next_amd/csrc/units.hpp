@@ -67,14 +67,12 @@ struct UnitView {
 // The body of a unit kernel (kBlock threads, one unit per block).
 // load(view, k): called once for every node k of the unit, in parallel, when
 // the unit fits LDS (a leaf's data; an internal node's are written by node).
-// node(view, id, end, depth, lane): one internal node, computed by LANES
-// threads (lane 0 .. LANES - 1).
+// node(view, id, end, depth): one internal node.
 // NODES: nodes of a unit whose lists LDS holds (a unit of up to 1.5 span bodies
 // has about 1.5 nodes per body); with more (clumps that share many digits) the
 // lists and records are read from memory.
-template <int LANES, int NODES, class Load, class Node>
+template <int NODES, class Load, class Node>
 __device__ __forceinline__ void upward_unit(const UnitArgs& a, Load load, Node node) {
-  constexpr int kNodes = kBlock / LANES;
   __shared__ unsigned long long red[kBlock / kWave];
   __shared__ int32_t seg[2][kMaxDepthSlots];       // this unit's part of each depth's list
   __shared__ uint32_t off[kMaxDepthSlots];         // nodes of smaller depth
@@ -139,11 +137,11 @@ __device__ __forceinline__ void upward_unit(const UnitArgs& a, Load load, Node n
     for (int d = kMaxLevels - 1; d >= 0; --d) {
       const int32_t cnt = seg[1][d] - seg[0][d];
       if (cnt == 0) continue;                                // (uniform)
-      for (int32_t k = t / LANES; k < cnt; k += kNodes) {
+      for (int32_t k = t; k < cnt; k += kBlock) {
         const uint32_t e = list[at[d] + k], id = e & 0xffffu, end = e >> 16;
         if (end == (uint32_t)NODES) continue;
-        node(view, (int32_t)(p0 + id), (int32_t)(p0 + end), d, t % LANES);
-        if (t % LANES == 0) skips[id] = (uint16_t)end;
+        node(view, (int32_t)(p0 + id), (int32_t)(p0 + end), d);
+        skips[id] = (uint16_t)end;
       }
       __syncthreads();
     }
@@ -151,10 +149,10 @@ __device__ __forceinline__ void upward_unit(const UnitArgs& a, Load load, Node n
     for (int d = kMaxLevels - 1; d >= 0; --d) {
       const int32_t b = seg[0][d], e = seg[1][d];
       if (b == e) continue;
-      for (int32_t k = b + t / LANES; k < e; k += kNodes) {
+      for (int32_t k = b + t; k < e; k += kBlock) {
         const uint32_t end = a.end_list[k];
         if (end > p1) over[d] = k;
-        else node(view, a.level_list[k], (int32_t)end, d, t % LANES);
+        else node(view, a.level_list[k], (int32_t)end, d);
       }
       __syncthreads();
     }
@@ -170,11 +168,10 @@ __device__ __forceinline__ void upward_unit(const UnitArgs& a, Load load, Node n
 
 // The nodes that end beyond their units, depth by depth: one workgroup of
 // kOverBlock threads per system (a system's nodes are its own).  The depth
-// mask is cleared by the next build's (or refit's) first kernel.
+// mask is cleared by the next build's first kernel.
 constexpr int kOverBlock = 1024;
-template <int LANES, class Node>
+template <class Node>
 __device__ __forceinline__ void upward_over(const UnitArgs& a, const SysArrays& sy, Node node) {
-  constexpr int kNodes = kOverBlock / LANES;
   __shared__ int32_t list[kOverBlock];
   __shared__ int32_t count;
   if (a.sc->abort_flags) return;
@@ -198,8 +195,8 @@ __device__ __forceinline__ void upward_over(const UnitArgs& a, const SysArrays& 
         if (id >= root && id < end) list[atomicAdd(&count, 1)] = k;
       }
       __syncthreads();
-      for (int32_t j = t / LANES; j < count; j += kNodes)
-        node(view, a.level_list[list[j]], (int32_t)a.end_list[list[j]], d, t % LANES);
+      for (int32_t j = t; j < count; j += kOverBlock)
+        node(view, a.level_list[list[j]], (int32_t)a.end_list[list[j]], d);
       __syncthreads();
     }
   }

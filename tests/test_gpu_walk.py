@@ -1,8 +1,9 @@
 """The reference-mode walk at the sizes where its group width changes.
 
 The walk puts 64 / width lanes on each target of a group of `width` bodies;
-the width follows the system's size (8 up to 4,096 bodies, 16 up to 98,304,
-32 up to 196,608, then 64; 16 for larger systems below theta 0.4).
+the width follows the system's size and theta (8 up to 4,096 bodies and theta
+0.32, 16 below theta 0.4 and up to 98,304 bodies and theta 0.55, else 32 up to
+196,608 bodies, then 64).
 Accelerations against the oracle's walk (octree.h:133-179) at the edges of
 those ranges and of a group, with dark-matter targets (octree.h:146-148).
 Tolerance: the accelerations' own, median <= 1e-12 and 99th percentile <=
@@ -40,7 +41,8 @@ def test_small(n, theta):
 
 
 @pytest.mark.parametrize("n,theta", [(4096, 0.5), (4097, 0.5), (98304, 0.39), (98305, 0.4), (98305, 0.39),
-                                     (196608, 0.5), (196609, 0.5), (196609, 0.39)])
+                                     (196608, 0.5), (196609, 0.5), (196609, 0.39), (4096, 0.32), (4097, 0.32),
+                                     (4096, 0.33), (98304, 0.55), (98304, 0.56), (196609, 0.56)])
 def test_width_edges(n, theta):
     check(ic.plummer(n, seed=3, virial=None, type_fraction_dm=0.1), theta, f"n={n} theta={theta}")
 
