@@ -294,16 +294,33 @@ nbx_status ensure_particles(nbx_ctx* c, int64_t n, int64_t keep_n) {
 }
 
 // Reference mode's walk groups: runs of walk_width bodies of one system each.
+// Each of the 8 XCDs walks an eighth of the table; where widths differ, empty
+// groups fill its parts up so that they hold equal numbers of bodies (equal
+// numbers of groups gave the XCDs of the large systems twice the work).
 std::vector<Group> ref_groups(const nbx_ctx* c) {
   std::vector<Group> groups;
+  bool mixed = false;
   int32_t at = 0;
   for (size_t s = 0; s < c->sys_n.size(); ++s) {
     const int32_t end = at + (int32_t)c->sys_n[s], width = walk_width(c->sys_n[s], c->cfg.theta);
+    mixed |= width != walk_width(c->sys_n[0], c->cfg.theta);
     for (int32_t b = at; b < end; b += width)
       groups.push_back(Group{b, std::min<int32_t>(width, end - b), (int32_t)s, 0});
     at = end;
   }
-  return groups;
+  if (!mixed) return groups;
+  constexpr int kXcds = 8;
+  size_t cut[kXcds + 1] = {}, part = 0;
+  for (int x = 1; x <= kXcds; ++x) {
+    size_t g = cut[x - 1];
+    while (g < groups.size() && (int64_t)groups[g].first * kXcds < (int64_t)at * x) ++g;
+    cut[x] = x == kXcds ? groups.size() : g;
+    part = std::max(part, cut[x] - cut[x - 1]);
+  }
+  std::vector<Group> table(kXcds * part, Group{0, 0, 0, 0});
+  for (int x = 0; x < kXcds; ++x)
+    std::copy(groups.begin() + cut[x], groups.begin() + cut[x + 1], table.begin() + x * part);
+  return table;
 }
 
 // The copy of `groups` is under way on return: the caller drains the stream

@@ -978,6 +978,7 @@ void k_walk(const Group* __restrict__ groups, int64_t ngroups, const RefNode* __
   if (gi >= ngroups || sc->abort_flags) return;            // past the end, or an aborted build
   const int lane = threadIdx.x;
   const Group g = groups[gi];
+  if (g.count == 0) return;                                // (fills an XCD's part of the table)
   int width = kWave;
   while (width > 1 && (width >> 1) >= g.count) width >>= 1;
   const int parts = kWave / width;

@@ -163,6 +163,7 @@ void launch_out_gather(int64_t j0, int64_t len, int64_t cnt, const uint32_t* inv
 //   0.5    1,000    237 /  56 /  72 / 103 / 152    512:   786 /   902 /   705 /   644 /   675
 //   0.5    2,000    270 /  84 /  81 / 120 / 181    512: 1,585 / 2,115 / 1,632 / 1,423 / 1,404
 //   0.5    16,384   369 /  93 / 117 / 141 / 205     64: 2,047 / 2,579 / 2,016 / 1,724 / 1,557
+//   0.5    32,768   386 / 127 / 130 / 162 / 215     64: 3,840 /     - / 4,175 / 3,490 /     -
 //   0.5    65,536   426 / 217 / 171 / 185 / 252     16: 2,196 / 2,810 / 2,127 / 1,833 / 1,562
 //   0.5    100,000  490 / 326 / 276 / 248 / 262     12: 2,538 / 3,368 / 2,533 / 2,182 / 1,742
 //   0.5    200,000  677 / 611 / 491 / 461 / 410
@@ -170,7 +171,7 @@ void launch_out_gather(int64_t j0, int64_t len, int64_t cnt, const uint32_t* inv
 //   0.7    65,536   238 / 173 / 122 / 126 / 170     16: 1,354 / 2,189 / 1,518 / 1,170 /   810
 inline int32_t walk_width(int64_t n, double theta) {
   if (theta <= 0.32 && n <= 4096) return 8;
-  if (theta < 0.4 || (theta <= 0.55 && n <= 98304)) return 16;
+  if (theta < 0.4 || n <= (theta < 0.45 ? 98304 : theta <= 0.55 ? 20480 : 0)) return 16;
   return n <= 196608 ? 32 : 64;
 }
 void launch_walk(const Group* groups, int64_t ngroups, const RefNode* nodes, const WalkHead* heads,

@@ -2,8 +2,8 @@
 
 The walk puts 64 / width lanes on each target of a group of `width` bodies;
 the width follows the system's size and theta (8 up to 4,096 bodies and theta
-0.32, 16 below theta 0.4 and up to 98,304 bodies and theta 0.55, else 32 up to
-196,608 bodies, then 64).
+0.32, 16 below theta 0.4, up to 98,304 bodies below 0.45 and up to 20,480 up to
+0.55, else 32 up to 196,608 bodies, then 64).
 Accelerations against the oracle's walk (octree.h:133-179) at the edges of
 those ranges and of a group, with dark-matter targets (octree.h:146-148).
 Tolerance: the accelerations' own, median <= 1e-12 and 99th percentile <=
@@ -42,7 +42,8 @@ def test_small(n, theta):
 
 @pytest.mark.parametrize("n,theta", [(4096, 0.5), (4097, 0.5), (98304, 0.39), (98305, 0.4), (98305, 0.39),
                                      (196608, 0.5), (196609, 0.5), (196609, 0.39), (4096, 0.32), (4097, 0.32),
-                                     (4096, 0.33), (98304, 0.55), (98304, 0.56), (196609, 0.56)])
+                                     (4096, 0.33), (98304, 0.44), (98304, 0.45), (20480, 0.5), (20481, 0.5),
+                                     (20480, 0.56), (196609, 0.56)])
 def test_width_edges(n, theta):
     check(ic.plummer(n, seed=3, virial=None, type_fraction_dm=0.1), theta, f"n={n} theta={theta}")
 
@@ -74,3 +75,19 @@ def test_theta_changes_the_width():
         with Engine(theta=theta) as f:
             f.upload(p)
             assert np.array_equal(got, f.accel())
+
+
+@pytest.mark.parametrize("sizes", [[1, 20481], [20481, 1, 1, 1], [20480, 20481], [5, 70, 30000, 3, 21000, 600], [25000] + [9] * 40])
+def test_batch_of_mixed_widths(sizes):
+    """The group table of a batch whose widths differ is cut by bodies: every
+    system gets its forces alone, bit for bit."""
+    ps = [ic.plummer(n, seed=k, virial=None, type_fraction_dm=0.2) for k, n in enumerate(sizes)]
+    with Engine(theta=0.5) as e:
+        e.upload_batch(ps)
+        a = e.accel()
+    at = 0
+    for p in ps:
+        with Engine(theta=0.5) as f:
+            f.upload(p)
+            assert np.array_equal(a[at:at + len(p)], f.accel())
+        at += len(p)
