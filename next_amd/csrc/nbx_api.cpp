@@ -11,7 +11,7 @@
 //   per-system root cube, keys, radix sort by key and then by system,
 //   state gather                                   tree of x_{n+1}
 //   lcp/counts, scans  -> host reads node counts (one small copy)
-//   node emit, depth sorts, skip pairing, upward pass per depth
+//   node layout, upward pass per depth (small systems: by units of bodies)
 //   walk over the group table + closing kick(a_{n+1}, dt/2) + max |v|^2
 //
 // Systems never share a tree node or a walk group, so each system's result
