@@ -299,6 +299,7 @@ nbx_status ensure_particles(nbx_ctx* c, int64_t n, int64_t keep_n) {
 // numbers of groups gave the XCDs of the large systems twice the work).
 std::vector<Group> ref_groups(const nbx_ctx* c) {
   std::vector<Group> groups;
+  groups.reserve((size_t)c->n / 16 + c->sys_n.size());
   bool mixed = false;
   int32_t at = 0;
   for (size_t s = 0; s < c->sys_n.size(); ++s) {
