@@ -23,10 +23,10 @@
 #include <condition_variable>
 #include <cstdio>
 #include <cstring>
+#include <exception>
 #include <mutex>
 #include <new>
 #include <string>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -1052,18 +1052,18 @@ nbx_status fetch(nbx_ctx* c, const void* dev, size_t bytes, const void** staged)
 // Threads that help one download copy its chunks into the caller's arrays,
 // each a part of the chunk's values (array after array, so that a thread
 // mostly writes pages of its own: fresh ones are zeroed as they are touched,
-// which is half of the time).  Fewer, or none, where threads cannot be started.
+// which is half of the time).  Fewer, or none, where threads cannot be started
+// or helpers <= 0.
 class CopyTeam {
  public:
   explicit CopyTeam(int helpers) {
     try {
-      threads_.reserve((size_t)helpers);
+      threads_.reserve((size_t)std::max(helpers, 0));
       for (int t = 1; t <= helpers; ++t) {
         threads_.emplace_back([this, t] { help(t); });
         ++started_;
       }
-    } catch (const std::system_error&) {
-    } catch (const std::bad_alloc&) {
+    } catch (const std::exception&) {                      // (no memory, no thread)
     }
   }
   CopyTeam(const CopyTeam&) = delete;
@@ -1152,7 +1152,7 @@ nbx_status copy_out(nbx_ctx* c, int64_t off, int64_t cnt, int64_t base, const do
   *bad = 0;
   uint32_t* inv = P<uint32_t>(c->idx[0]);                  // sort scratch, free between steps
   launch_out_index(cnt, id, (int32_t)base, inv, bad, c->stream);
-  CopyTeam team(cnt >= kOutTeam ? std::min(m, 3) - 1 : 0);
+  CopyTeam team(cnt >= kOutTeam ? std::min(m, 3) - 1 : 0);   // (every output null: -1, none)
   const int64_t nchunks = div_up(cnt, chunk);
   for (int64_t k = 0; k <= nchunks; ++k) {
     if (k < nchunks) {

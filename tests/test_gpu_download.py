@@ -61,3 +61,38 @@ def test_skipped_arrays():
         assert fn(e._h, None, y.ctypes.data, None, None, None, vz.ctypes.data) == 0
         assert np.array_equal(y, p.y) and np.array_equal(vz, p.vz)
         assert fn(e._h, None, None, None, None, None, None) == 0
+
+
+@pytest.mark.parametrize("n", [4 * CHUNK, 4 * CHUNK + 1])
+def test_skipped_arrays_with_helping_threads(n):
+    """From four chunks on: every output null (the documented way to skip
+    them), or one array only; then the system is removed without its state."""
+    p = bodies(n, n)
+    L = C.CDLL(lib()._name)
+    vp = C.c_void_p
+    L.nbx_download.argtypes = [vp] * 7
+    L.nbx_download_system.argtypes = [vp, C.c_int32] + [vp] * 6
+    L.nbx_remove_system.argtypes = [vp, C.c_int32] + [vp] * 6
+    with Engine(theta=0.9) as e:
+        e.upload(p)
+        e.accel()
+        assert L.nbx_download(e._h, *[None] * 6) == 0
+        assert L.nbx_download_system(e._h, 0, *[None] * 6) == 0
+        x, vy = np.full(n, -7.0), np.full(n, -7.0)
+        assert L.nbx_download(e._h, x.ctypes.data, *[None] * 5) == 0
+        assert L.nbx_download_system(e._h, 0, None, None, None, None, vy.ctypes.data, None) == 0
+        assert np.array_equal(x, p.x) and np.array_equal(vy, p.vy)
+        assert L.nbx_remove_system(e._h, 0, *[None] * 6) == 0
+        assert e.num_systems() == 0
+
+
+def test_direct_without_outputs():
+    n = 4 * CHUNK
+    L = C.CDLL(lib()._name)
+    L.nbx_direct.argtypes = [C.c_void_p] * 5
+    with Engine(eps=0.01) as e:
+        e.upload(bodies(n, 5))
+        pot = np.full(n, 7.0)
+        assert L.nbx_direct(e._h, *[None] * 4) == 0
+        assert L.nbx_direct(e._h, None, None, None, pot.ctypes.data) == 0
+        assert np.all(pot < 0.0)
