@@ -18,13 +18,18 @@ constexpr int kMaxDepthSlots = 64; // histogram slots for node depths
 constexpr int32_t kLinkZeroMass = 1 << 30;   // link flag: zero mass, skipped whole
 struct alignas(128) RefNode {
   double cx, cy, cz;       // centre of mass
-  double dmk;              // 2*size / m^0.333333333 (softening floor of a dark-matter target, octree.h:146-148)
+  int32_t skip;            // preorder index of the first node after this subtree
+  int32_t first;           // first body (sorted index) of the subtree
   double m;                // mass
   double esum;             // size*0.015 + cbrt(m)*0.002 (softening numerator)
-  int32_t skip;            // preorder index of the first node after this subtree
-  int32_t body;            // leaf: sorted body index; internal: -1
-  int32_t depth;
-  int32_t first;           // first body (sorted index) of the subtree
+  // Softening floor of a dark-matter target (octree.h:146-148), 2*size / m^0.333333333:
+  // dmk (1 + dmr), the double and what rounding took off it.  Side by side: one
+  // load (12 bytes apart, a step of 200,003 bodies at theta 0.3, a tenth of them
+  // dark matter, took 6.6 % more than without dmr; so 1 %).
+  double dmk;
+  float dmr;
+  int16_t depth;
+  int16_t leaf;            // 1: one body, `first`
   // internal nodes only
   double qxx, qyy, qzz, qxy, qxz, qyz;
   double size;             // half-width: root half-width * 2^-depth

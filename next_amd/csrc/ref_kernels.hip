@@ -160,16 +160,43 @@ __device__ __forceinline__ void key_digits(double px, double py, double pz, cons
   }
 }
 
-// m^0.333333333 (the exponent of octree.h:146) from cbrt(m): the exponents
-// differ by d = 3.3e-10, and m^-d = 1 - d ln m + (d ln m)^2 / 2 with
-// |d ln m| < 2.5e-7, so ln m is needed to about 1e-6 only.  Odd in m, and 0
-// at 0.
-__device__ __forceinline__ double dm_power(double m, double cbrt_m) {
-  if (m == 0.0) return 0.0;
+// m^0.333333333 (the exponent of octree.h:146) as p (1 + r), from cb =
+// cbrt(m), odd in m and 0 at 0.  A softening floor is the quotient of two of
+// these, rounded once, so both carry their rounding errors along: the floor is
+// within 1.6e-16 of the exact one for masses of 1e-307 to 1e210 (pow of the
+// mass ratio: 2.5e-16), and for equal masses it is the half-width's double as
+// pow(1) makes it.  In units of a power of eight, g = m / 8^k:
+//   g^(1/3) = c (1 + (g - c^3) / (3 g)), the residual formed exactly;
+//   the exponents differ by d = 1/3 - 0.333333333, and g^-d = 1 - t + t^2 / 2
+//   with t = d ln m < 2.5e-7, so an error of 1e-7 in ln m (log of the mantissa
+//   in FP32, the exponent's part in FP64) moves the power by 3e-17.
+struct DmPower {
+  double p;
+  float r;
+};
+
+__device__ __forceinline__ DmPower dm_power(double m, double cb) {
+  if (m == 0.0) return DmPower{0.0, 0.0f};
+  constexpr double kD = 3.3333332390602283e-10;             // 1/3 minus the double nearest 0.333333333
   int e;
-  const float f = (float)frexp(fabs(m), &e);
-  const double t = (1.0 / 3.0 - 0.333333333) * (double)(__logf(f) + 0.69314718f * (float)e);
-  return cbrt_m * ((1.0 - t) + 0.5 * t * t);
+  const double f = frexp(fabs(m), &e);
+  const int k = e / 3;
+  const double g = ldexp(f, e - 3 * k), c = ldexp(fabs(cb), -k);
+  const double c2 = c * c, e2 = __builtin_fma(c, c, -c2);
+  const double c3 = c2 * c, e3 = __builtin_fma(e2, c, __builtin_fma(c2, c, -c3));
+  const float rel = (float)((g - c3) - e3) * __builtin_amdgcn_rcpf(3.0f * (float)g);
+  const double t = kD * __builtin_fma(0.6931471805599453, (double)e, (double)__logf((float)f));
+  const double w = (double)rel - __builtin_fma(-0.5 * t, t, t);
+  const double p = __builtin_fma(c, w, c);
+  const double left = __builtin_fma(c, w, c - p);
+  return DmPower{copysign(ldexp(p, k), m), (float)left * __builtin_amdgcn_rcpf((float)p)};
+}
+
+// The dmk and dmr of a node of half-width `size` and mass power q.
+__device__ __forceinline__ void set_floor(RefNode& nd, double size, const DmPower& q) {
+  const double s2 = 2.0 * size, k = s2 / q.p;
+  nd.dmk = k;
+  nd.dmr = (float)(__builtin_fma(-k, q.p, s2) * __builtin_amdgcn_rcp(s2)) - q.r;
 }
 
 __device__ __forceinline__ void sys_root(const SysArrays& sy, int32_t s, double root[4]) {
@@ -545,19 +572,19 @@ __global__ __launch_bounds__(kBlock) void k_emit(int64_t n, const int32_t* __res
     const double m = st.m[i];
     const double size = ldexp(sy.root[4 * st.sys[i] + 3], -d);
     // Leaves carry no quadrupole; the walk never reads a leaf's Q fields
-    // (the first 80 bytes of the record are written, in one piece).
+    // (the first 64 bytes of the record are written, in one piece).
     const double px = st.x[i], py = st.y[i], pz = st.z[i];
     RefNode& nd = nodes[p];
     nd.cx = px; nd.cy = py; nd.cz = pz;
     nd.m = m;
     nd.skip = (int32_t)(p + 1);
-    nd.body = (int32_t)i;
-    nd.depth = d;
     nd.first = (int32_t)i;
+    nd.depth = (int16_t)d;
+    nd.leaf = 1;
     // softening.h:26-27: size*0.015 + cbrt(m)*0.002, summed before the taper
     const double cm = cbrt(m);
     nd.esum = size * 0.015 + cm * 0.002;
-    nd.dmk = 2.0 * size / dm_power(m, cm);
+    set_floor(nd, size, dm_power(m, cm));
     // a leaf is accepted whatever its distance: no threshold
     heads[p] = WalkHead{px, py, pz, 0.0f, m == 0.0 ? (int32_t)(p + 1) | kLinkZeroMass : ~(int32_t)i};
   }
@@ -668,10 +695,10 @@ __device__ __forceinline__ void upward_node(const UnitView& v, UnitMoments* lm, 
   const double cb = cbrt(M);
   RefNode& out = nodes[id];                  // the record but its padding
   out.cx = cx; out.cy = cy; out.cz = cz;
-  out.dmk = 2.0 * size / dm_power(M, cb);
+  set_floor(out, size, dm_power(M, cb));
   out.m = M;
   out.esum = size * 0.015 + cb * 0.002;
-  out.skip = end; out.body = -1; out.depth = d; out.first = first;
+  out.skip = end; out.first = first; out.depth = (int16_t)d; out.leaf = 0;
   out.qxx = qxx; out.qyy = qyy; out.qzz = qzz; out.qxy = qxy; out.qxz = qxz; out.qyz = qyz;
   out.size = size;
   // Upper edge of the opening test's band for r^2 (NEXT tests r^2 + 1e-20,
@@ -770,9 +797,10 @@ __device__ __forceinline__ int64_t xcd_block(int nb) {
   return (int64_t)(blockIdx.x % 8) * per + blockIdx.x / 8;
 }
 
-// Reciprocal square root and reciprocal with a relative error of a few
-// units in the last place: the v_rsq_f64 / v_rcp_f64 estimates refined by
-// one Newton step each (the residual formed with an FMA).  The walk's
+// Reciprocal square root and reciprocal: the v_rsq_f64 / v_rcp_f64 estimates
+// refined by one Newton step each (the residual formed with an FMA).  v_rsq_f64
+// is off by up to 5.2e-8, 1.1e-8 in the root mean square, so rsq_nr by up to
+// 4.2e-15, 3.5e-16 in the root mean square, 1.8e-16 too small on average.  The walk's
 // arguments are positive, finite and mid-range: r^2 + 1e-20, r^2 + eps^2
 // with eps >= 1e-4, and 1 + 10 dist >= 1.
 __device__ __forceinline__ double rsq_nr(double x) {
@@ -828,23 +856,23 @@ static_assert(kWalkCommon > kWave && kWalkMixed > kWave, "a wave step appends up
 struct Sum3 { double x, y, z; };
 
 // One accepted node on one target (octree.h:139-172, G = 1): products fused
-// into FMAs and the square roots and divides faithfully rounded (a few ulp
-// per interaction).  d: node minus target, r2 = |d|^2 as the opening test
-// forms it; dist = sqrt(r2 + 1e-20), eps from softening.h:26-36, dinv =
-// 1/sqrt(r2 + eps^2).  DM: some target is dark matter: its softening floor
-// (octree.h:146-148) is 2 size / (m/mi)^p = dmk mi^p, with mip = mi^p for
-// a dark-matter target and 0 otherwise.  QUAD: the quadrupole term
+// into FMAs and the square roots and divides as rsq_nr and rcp_nr give them.
+// d: node minus target, r2 = |d|^2 as the opening test forms it; dist =
+// sqrt(r2 + 1e-20), eps from softening.h:26-36, dinv = 1/sqrt(r2 + eps^2).
+// DM: some target is dark matter: its softening floor (octree.h:146-148) is
+// 2 size / (m/mi)^p, dmk (1 + dmr) times the target's mass power mip (dm_power;
+// 0 for a target that is not dark matter).  QUAD: the quadrupole term
 // 0.5 (2 (Q d) inv5 - 5 q inv7 d), q = d.Q.d, as (Q d) inv5 + d (-(2.5 q) inv7).
 template <bool DM, bool QUAD>
 __device__ __forceinline__ void interact(double dx, double dy, double dz, double r2, double m, double esum,
-                                         double dmk, double mip, double qxx, double qyy, double qzz, double qxy,
-                                         double qxz, double qyz, Sum3& a) {
+                                         double dmk, float dmr, const DmPower& mip, double qxx, double qyy,
+                                         double qzz, double qxy, double qxz, double qyz, Sum3& a) {
   const double r2e = r2 + 1e-20;
   const double dist = r2e * rsq_nr(r2e);
   double eps = esum * rcp_nr(__builtin_fma(dist, 10.0, 1.0));
   if (eps < 1e-4) eps = 1e-4;
   if (DM) {
-    const double alt = dmk * mip;
+    const double alt = __builtin_fma(dmk, mip.p, dmk * mip.p * (double)(dmr + mip.r));
     if (eps < alt) eps = alt;
   }
   const double dinv = rsq_nr(__builtin_fma(eps, eps, r2));
@@ -880,7 +908,7 @@ __device__ __forceinline__ const RefNode& node_at(const RefNode* nodes, uint32_t
 template <bool DM>
 __device__ __forceinline__ void walk_common(const int32_t* list, int n, int part, int parts,
                                             const RefNode* __restrict__ nodes, uint32_t zoff, double px, double py,
-                                            double pz, double mip, Sum3& a) {
+                                            double pz, const DmPower& mip, Sum3& a) {
   if (parts == 1) {
     for (int k = 0; k < n; ++k) {
       const int32_t e = __builtin_amdgcn_readfirstlane(list[k]);
@@ -888,10 +916,10 @@ __device__ __forceinline__ void walk_common(const int32_t* list, int n, int part
       const double dx = nd.cx - px, dy = nd.cy - py, dz = nd.cz - pz;
       const double r2 = __builtin_fma(dz, dz, __builtin_fma(dy, dy, dx * dx));
       if (e < 0)
-        interact<DM, false>(dx, dy, dz, r2, nd.m, nd.esum, nd.dmk, mip, 0, 0, 0, 0, 0, 0, a);
+        interact<DM, false>(dx, dy, dz, r2, nd.m, nd.esum, nd.dmk, nd.dmr, mip, 0, 0, 0, 0, 0, 0, a);
       else
-        interact<DM, true>(dx, dy, dz, r2, nd.m, nd.esum, nd.dmk, mip, nd.qxx, nd.qyy, nd.qzz, nd.qxy, nd.qxz,
-                           nd.qyz, a);
+        interact<DM, true>(dx, dy, dz, r2, nd.m, nd.esum, nd.dmk, nd.dmr, mip, nd.qxx, nd.qyy, nd.qzz, nd.qxy,
+                           nd.qxz, nd.qyz, a);
     }
   } else {
     for (int k = part; k < n; k += parts) {
@@ -901,8 +929,8 @@ __device__ __forceinline__ void walk_common(const int32_t* list, int n, int part
       const RefNode& qn = node_at(nodes, e < 0 ? zoff : off);
       const double dx = nd.cx - px, dy = nd.cy - py, dz = nd.cz - pz;
       const double r2 = __builtin_fma(dz, dz, __builtin_fma(dy, dy, dx * dx));
-      interact<DM, true>(dx, dy, dz, r2, nd.m, nd.esum, nd.dmk, mip, qn.qxx, qn.qyy, qn.qzz, qn.qxy, qn.qxz, qn.qyz,
-                         a);
+      interact<DM, true>(dx, dy, dz, r2, nd.m, nd.esum, nd.dmk, nd.dmr, mip, qn.qxx, qn.qyy, qn.qzz, qn.qxy, qn.qxz,
+                         qn.qyz, a);
     }
   }
 }
@@ -914,8 +942,9 @@ __device__ __forceinline__ void walk_common(const int32_t* list, int n, int part
 template <bool DM, bool COUNT>
 __device__ __forceinline__ void walk_mixed(const int32_t* list, int n, bool valid, int part, int parts, int32_t self,
                                            const RefNode* __restrict__ nodes, const WalkHead* __restrict__ heads,
-                                           uint32_t zoff, double theta, double px, double py, double pz, double mip,
-                                           Sum3& a, uint32_t& npp, uint32_t& npc, uint32_t& nop, uint32_t& nit) {
+                                           uint32_t zoff, double theta, double px, double py, double pz,
+                                           const DmPower& mip, Sum3& a, uint32_t& npp, uint32_t& npc, uint32_t& nop,
+                                           uint32_t& nit) {
   int k = part;
   bool live = valid && k < n;
   int32_t cur = live ? list[k] : 0, root = cur, end = 0;
@@ -959,8 +988,8 @@ __device__ __forceinline__ void walk_mixed(const int32_t* list, int n, bool vali
       const uint32_t off = (uint32_t)cur << 7;
       const RefNode& nd = node_at(nodes, off);
       const RefNode& qn = node_at(nodes, leaf ? zoff : off);
-      interact<DM, true>(dx, dy, dz, r2, nd.m, nd.esum, nd.dmk, mip, qn.qxx, qn.qyy, qn.qzz, qn.qxy, qn.qxz, qn.qyz,
-                         a);
+      interact<DM, true>(dx, dy, dz, r2, nd.m, nd.esum, nd.dmk, nd.dmr, mip, qn.qxx, qn.qyy, qn.qzz, qn.qxy, qn.qxz,
+                         qn.qyz, a);
     }
     cur = next;
     h = hn;
@@ -987,7 +1016,7 @@ void k_walk(const Group* __restrict__ groups, int64_t ngroups, const RefNode* __
   const int64_t i = g.first + (valid ? slot : 0);
   const double px = st.x[i], py = st.y[i], pz = st.z[i], pm = st.m[i];
   const bool dark = valid && st.type[i] == 1;
-  const double mip = dark ? dm_power(pm, cbrt(pm)) : 0.0;
+  const DmPower mip = dark ? dm_power(pm, cbrt(pm)) : DmPower{0.0, 0.0f};
   const bool any_dm = __ballot(dark) != 0;
   const int32_t self = ~(int32_t)i;                          // link of this target's own leaf
   const uint64_t ltmask = lanemask_lt();
@@ -1239,8 +1268,8 @@ __global__ __launch_bounds__(kBlock) void k_export(int64_t total, const RefNode*
   if (k >= total) return;
   const RefNode nd = nodes[k];
   depth[k] = nd.depth;
-  leaf[k] = nd.body >= 0 ? 1 : 0;
-  body[k] = nd.body >= 0 ? id[nd.body] : -1;
+  leaf[k] = nd.leaf;
+  body[k] = nd.leaf ? id[nd.first] : -1;
   double cx = sy.root[0], cy = sy.root[1], cz = sy.root[2], s = sy.root[3];
   for (int l = 0; l < nd.depth; ++l) {
     const uint32_t o = digit_at(key, key2, nd.first, l);
@@ -1252,13 +1281,13 @@ __global__ __launch_bounds__(kBlock) void k_export(int64_t total, const RefNode*
   }
   geo4[4 * k] = cx; geo4[4 * k + 1] = cy; geo4[4 * k + 2] = cz; geo4[4 * k + 3] = s;
   int32_t mask = 0;
-  if (nd.body < 0)
+  if (!nd.leaf)
     for (int32_t c = (int32_t)k + 1, it = 0; it < 8 && c < nd.skip; ++it, c = nodes[c].skip)
       mask |= 1 << digit_at(key, key2, nodes[c].first, nd.depth);
   cmask[k] = mask;
   mass[k] = nd.m;
   com3[3 * k] = nd.cx; com3[3 * k + 1] = nd.cy; com3[3 * k + 2] = nd.cz;
-  const bool lf = nd.body >= 0;
+  const bool lf = nd.leaf != 0;
   q6[6 * k] = lf ? 0.0 : nd.qxx; q6[6 * k + 1] = lf ? 0.0 : nd.qyy; q6[6 * k + 2] = lf ? 0.0 : nd.qzz;
   q6[6 * k + 3] = lf ? 0.0 : nd.qxy; q6[6 * k + 4] = lf ? 0.0 : nd.qxz; q6[6 * k + 5] = lf ? 0.0 : nd.qyz;
 }
