@@ -222,7 +222,10 @@ nbx_status nbx_accel_noalloc(void* stream, int64_t n, const double* x, const dou
 nbx_status nbx_potential(nbx_ctx* ctx, double* pot);
 
 /* FP64 direct sum over all pairs with Plummer softening cfg.eps (G = 1):
- * the force reference for either mode.  Any output may be null. */
+ * the force reference for either mode.  Any output may be null.  A system's
+ * results do not depend on the others in the context.  The context keeps the
+ * call's buffers (32 bytes per body, 96 below 131,009 bodies) like its others:
+ * nbx_device_bytes counts them, nbx_trim frees them. */
 nbx_status nbx_direct(nbx_ctx* ctx, double* ax, double* ay, double* az, double* pot);
 
 /* Energy and momentum of the current state, FP64 with a fixed reduction

@@ -774,7 +774,7 @@ __global__ __launch_bounds__(kPhysBlock * (1 + EVAL)) void k_phys_walk(const Gro
 // waves of a workgroup, whose sums meet in LDS, and over blockIdx.y
 // (k_direct_sum), so that a small system fills the chip too.  A pair issues 19
 // FP64 instructions and v_rsq_f64, so the sum is bound by FP64 issue: two sums
-// over 65,537 bodies (forces, then energies) with the download 6.67 ms, against
+// over 65,537 bodies (forces, then energies) with the download 6.8 ms, against
 // 36.1 of one target per thread with sources staged in LDS, a correctly rounded
 // square root and divide per pair and 257 workgroups.  v_rsq_f64 (5.2e-8 at
 // most) is refined by one step of third order, y (1 + h/2 + 3/8 h^2) with
@@ -784,6 +784,13 @@ __global__ __launch_bounds__(kPhysBlock * (1 + EVAL)) void k_phys_walk(const Gro
 // Only bodies of the target's own system act on it: a wave whose targets lie
 // in several systems takes them one after another.  The lanes' own bodies are
 // among 64 sources only; the rest of the loop does not test for the self pair.
+//
+// A system's sources are cut into kDirectChunks parts by the system's size
+// alone, each part is summed from zero, and the parts are added in a balanced
+// tree: a wave its consecutive parts, a workgroup its waves, k_direct_sum the
+// halves.  How many parts a wave takes follows from the size of the launch and
+// changes no bit, so a system's sums are the same alone and in a batch.
+constexpr int kDirectChunks = 32;
 struct DirectSum { double x, y, z, p; };
 
 // Sources [j, end).  SELF: some of them are targets of the wave (body i of
@@ -791,6 +798,7 @@ struct DirectSum { double x, y, z, p; };
 template <bool SELF, bool ZERO>
 __device__ __forceinline__ void direct_range(const StateArrays& st, int64_t j, int64_t end, int64_t i, double px,
                                              double py, double pz, double e2, DirectSum& a) {
+#pragma clang fp contract(off)   // the same roundings with and without SELF (a wave's neighbours decide which)
   typedef const __attribute__((address_space(4))) double* cptr;   // scalar loads
   const cptr X = (cptr)st.x, Y = (cptr)st.y, Z = (cptr)st.z, M = (cptr)st.m;
 #pragma unroll 4
@@ -813,13 +821,25 @@ __device__ __forceinline__ void direct_range(const StateArrays& st, int64_t j, i
   }
 }
 
-// The W waves of a workgroup have the same 64 targets and a part of the
-// sources each.
-template <bool ZERO, int W>
-__global__ __launch_bounds__(W* kWave) void k_direct64(int64_t n, StateArrays st, SysArrays sy, double e2,
-                                                       double* __restrict__ ax, double* __restrict__ ay,
-                                                       double* __restrict__ az, double* __restrict__ pot) {
-  __shared__ double part[W - 1][4][kWave];
+__device__ __forceinline__ DirectSum operator+(const DirectSum& a, const DirectSum& b) {
+  return DirectSum{a.x + b.x, a.y + b.y, a.z + b.z, a.p + b.p};
+}
+
+// Component q of waves [w, w + N) of a workgroup, added in a balanced tree.
+template <int N>
+__device__ __forceinline__ double sum_waves(const double (*part)[4][kWave], int w, int q) {
+  if constexpr (N == 1) return part[w][q][lane_id()];
+  else return sum_waves<N / 2>(part, w, q) + sum_waves<N / 2>(part, w + N / 2, q);
+}
+
+// The W waves of a workgroup have the same 64 targets and PER consecutive
+// parts of the sources each; blockIdx.y: which of the W PER parts.
+template <bool ZERO, int W, int PER>
+__global__ __launch_bounds__(W* kWave) __attribute__((amdgpu_waves_per_eu(PER < 8 ? 8 : 7)))
+void k_direct64(int64_t n, StateArrays st, SysArrays sy, double e2, double* __restrict__ ax, double* __restrict__ ay,
+                double* __restrict__ az, double* __restrict__ pot) {
+  static_assert(W >= 4 && (PER == 1 || PER == 2 || PER == 4 || PER == 8), "waves of the last sum, levels of the tree");
+  __shared__ double part[W][4][kWave];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int64_t i0 = (int64_t)blockIdx.x * kWave;
   const int64_t i1 = i0 + kWave < n ? i0 + kWave : n;        // targets [i0, i1)
@@ -829,47 +849,53 @@ __global__ __launch_bounds__(W* kWave) void k_direct64(int64_t n, StateArrays st
   const double px = st.x[ii], py = st.y[ii], pz = st.z[ii];
   const int32_t me = st.sys[ii];
   const int32_t s0 = __builtin_amdgcn_readfirstlane(st.sys[i0]), s1 = __builtin_amdgcn_readfirstlane(st.sys[i1 - 1]);
-  const int q = blockIdx.y * W + wave, parts = gridDim.y * W;
-  DirectSum a{0.0, 0.0, 0.0, 0.0};
+  const int c0 = ((int)blockIdx.y * W + wave) * PER;         // parts [c0, c0 + PER)
+  DirectSum total{0.0, 0.0, 0.0, 0.0};
   for (int32_t s = s0; s <= s1; ++s) {
-    const int64_t lo = sy.soff[s], cnt = sy.soff[s + 1] - lo;
-    const int64_t b = lo + cnt * q / parts, e = lo + cnt * (q + 1) / parts;
+    const int32_t lo = sy.soff[s], cnt = sy.soff[s + 1] - lo;   // (a context holds at most 2^25 bodies: cnt * 32 fits)
     if (me == s) {
-      const int64_t c0 = i0 < b ? b : i0 < e ? i0 : e, c1 = i1 < b ? b : i1 < e ? i1 : e;   // own targets in [b, e)
-      direct_range<false, ZERO>(st, b, c0, i, px, py, pz, e2, a);
-      direct_range<true, ZERO>(st, c0, c1, i, px, py, pz, e2, a);
-      direct_range<false, ZERO>(st, c1, e, i, px, py, pz, e2, a);
+      DirectSum l1{}, l2{}, l4{};                            // sums of 1, 2 and 4 parts that wait for their neighbours
+#pragma unroll 1
+      for (int k = 0; k < PER; ++k) {
+        // (wave-uniform, and told so: with one part the compiler lost track and loaded the sources by lane)
+        const int64_t b = __builtin_amdgcn_readfirstlane(lo + cnt * (c0 + k) / kDirectChunks),
+                      e = __builtin_amdgcn_readfirstlane(lo + cnt * (c0 + k + 1) / kDirectChunks);
+        const int64_t o0 = i0 < b ? b : i0 < e ? i0 : e, o1 = i1 < b ? b : i1 < e ? i1 : e;   // own targets in [b, e)
+        DirectSum a{0.0, 0.0, 0.0, 0.0};
+        direct_range<false, ZERO>(st, b, o0, i, px, py, pz, e2, a);
+        direct_range<true, ZERO>(st, o0, o1, i, px, py, pz, e2, a);
+        direct_range<false, ZERO>(st, o1, e, i, px, py, pz, e2, a);
+        if (PER > 1 && !(k & 1)) { l1 = a; continue; }
+        if (PER > 1) a = l1 + a;
+        if (PER > 2 && !(k & 2)) { l2 = a; continue; }
+        if (PER > 2) a = l2 + a;
+        if (PER > 4 && !(k & 4)) { l4 = a; continue; }
+        if (PER > 4) a = l4 + a;
+        total = a;
+      }
     }
   }
-  if (wave > 0) {
-    double(*const p)[kWave] = part[wave - 1];
-    p[0][lane_id()] = a.x; p[1][lane_id()] = a.y; p[2][lane_id()] = a.z; p[3][lane_id()] = a.p;
-  }
+  part[wave][0][lane_id()] = total.x; part[wave][1][lane_id()] = total.y;
+  part[wave][2][lane_id()] = total.z; part[wave][3][lane_id()] = total.p;
   __syncthreads();
-  if (wave > 0 || !valid) return;
-  for (int w = 0; w < W - 1; ++w) {
-    a.x += part[w][0][lane_id()];
-    a.y += part[w][1][lane_id()];
-    a.z += part[w][2][lane_id()];
-    a.p += part[w][3][lane_id()];
-  }
+  if (wave >= 4 || !valid) return;                           // a wave per component
+  const double v = sum_waves<W>(part, 0, wave);
   if (gridDim.y > 1) {                                       // halves: x y z p, n each
-    const int64_t at = (int64_t)blockIdx.y * 4 * n + i;
-    ax[at] = a.x; ax[at + n] = a.y; ax[at + 2 * n] = a.z; ax[at + 3 * n] = a.p;
+    ax[((int64_t)blockIdx.y * 4 + wave) * n + i] = v;
   } else {
-    ax[i] = a.x; ay[i] = a.y; az[i] = a.z;
-    if (pot) pot[i] = a.p;
+    double* const out = wave == 0 ? ax : wave == 1 ? ay : wave == 2 ? az : pot;
+    if (out) out[i] = v;
   }
 }
 
-__global__ __launch_bounds__(kBlock) void k_direct_sum(int64_t n, int splits, const double* __restrict__ part,
+// The two halves' sums.
+__global__ __launch_bounds__(kBlock) void k_direct_sum(int64_t n, const double* __restrict__ part,
                                                        double* __restrict__ ax, double* __restrict__ ay,
                                                        double* __restrict__ az, double* __restrict__ pot) {
   const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
   if (i >= n) return;
-  double v[4] = {0.0, 0.0, 0.0, 0.0};
-  for (int q = 0; q < splits; ++q)
-    for (int k = 0; k < 4; ++k) v[k] += part[((int64_t)q * 4 + k) * n + i];
+  double v[4];
+  for (int k = 0; k < 4; ++k) v[k] = part[k * n + i] + part[(4 + k) * n + i];
   ax[i] = v[0]; ay[i] = v[1]; az[i] = v[2];
   if (pot) pot[i] = v[3];
 }
@@ -1060,24 +1086,26 @@ int direct_splits(int64_t n) {
   return groups * w < 8192 && groups >= 2 * w ? 2 : 1;
 }
 
-template <bool ZERO, int W>
-static void direct_go(int64_t n, int splits, const StateArrays& st, const SysArrays& sy, double e2, double* ax,
-                      double* ay, double* az, double* pot, hipStream_t s) {
-  hipLaunchKernelGGL((k_direct64<ZERO, W>), dim3(grid_of(n, kWave), (unsigned)splits), dim3(W * kWave), 0, s, n, st,
-                     sy, e2, ax, ay, az, pot);
+template <bool ZERO, int W, int SPLITS>
+static void direct_go(int64_t n, const StateArrays& st, const SysArrays& sy, double e2, double* ax, double* ay,
+                      double* az, double* pot, hipStream_t s) {
+  hipLaunchKernelGGL((k_direct64<ZERO, W, kDirectChunks / (W * SPLITS)>), dim3(grid_of(n, kWave), SPLITS),
+                     dim3(W * kWave), 0, s, n, st, sy, e2, ax, ay, az, pot);
 }
 
 void launch_direct64(int64_t n, const StateArrays& st, const SysArrays& sy, double eps, double* part, double* ax,
                      double* ay, double* az, double* pot, hipStream_t s) {
   if (n <= 0) return;
-  const int splits = direct_splits(n);
-  double* const ox = splits > 1 ? part : ax;
+  const bool halves = direct_splits(n) == 2, wide = direct_waves(n) == 16;
+  double* const ox = halves ? part : ax;
   const double e2 = eps * eps;
-  auto* const go = direct_waves(n) == 16 ? (e2 > 0.0 ? &direct_go<false, 16> : &direct_go<true, 16>)
-                                         : (e2 > 0.0 ? &direct_go<false, 4> : &direct_go<true, 4>);
-  go(n, splits, st, sy, e2, ox, ay, az, pot, s);
-  if (splits > 1)
-    hipLaunchKernelGGL(k_direct_sum, dim3(grid_of(n, kBlock)), dim3(kBlock), 0, s, n, splits, part, ax, ay, az, pot);
+#define NBX_DS(Z)                                                                                         \
+  (wide ? (halves ? &direct_go<Z, 16, 2> : &direct_go<Z, 16, 1>) : (halves ? &direct_go<Z, 4, 2> : &direct_go<Z, 4, 1>))
+  auto* const go = e2 > 0.0 ? NBX_DS(false) : NBX_DS(true);
+#undef NBX_DS
+  go(n, st, sy, e2, ox, ay, az, pot, s);
+  if (halves)
+    hipLaunchKernelGGL(k_direct_sum, dim3(grid_of(n, kBlock)), dim3(kBlock), 0, s, n, part, ax, ay, az, pot);
 }
 
 void launch_energy(const StateArrays& st, const double* pot, const BoxBlock* blocks, int nblocks,

@@ -90,3 +90,22 @@ def test_one_pair_is_as_accurate_as_a_square_root_and_a_divide():
                     worst[1] = max(worst[1], float(abs(L(a[2 * k + i, q]) / (m * ri * ri * ri * d[q]) - 1)))
     print(f"pair: potential {worst[0] / u:.2f} u, force {worst[1] / u:.2f} u", flush=True)
     assert worst[0] <= 4.25 * u and worst[1] <= 13.75 * u
+
+
+@pytest.mark.parametrize("others", [[], [3], [1500], [40000], [140000, 7]])
+def test_alone_and_in_a_batch(others):
+    """How a launch splits the sources follows from its size (16 waves or 4, one
+    half or two); a system's forces, potentials and energies do not."""
+    ps = [ic.plummer(n, seed=n, virial=None) for n in (1, 2, 31, 33, 700, 1999)]
+    with Engine(mode=MODE_PHYSICS, precision=PREC_FP64, eps=0.01) as e:
+        e.upload_batch(ps + [ic.plummer(n, seed=n, virial=None) for n in others])
+        a, pot = e.direct()
+        energy = e.energy_systems(direct=True)
+    at = 0
+    for k, p in enumerate(ps):
+        with Engine(mode=MODE_PHYSICS, precision=PREC_FP64, eps=0.01) as f:
+            f.upload(p)
+            b, bpot = f.direct()
+            assert np.array_equal(a[at:at + len(p)], b) and np.array_equal(pot[at:at + len(p)], bpot), len(p)
+            assert np.array_equal(energy[k], f.energy_systems(direct=True)[0]), len(p)
+        at += len(p)
