@@ -84,6 +84,7 @@ struct nbx_ctx {
   DBuf s_root, s_dt, s_v2, s_soff, s_sroot, s_send;
   DBuf groups, boxes, box_off, box_part;   // groups: reference mode's walk groups
   int64_t ngroups = 0;
+  double groups_theta = 0.0;  // the theta their widths were chosen for
   DBuf tgroups;               // physics mode: walk groups packed from the tree
   DBuf gmarks;                // physics mode: per-body group counts and marks
   // Physics mode: the count of walk groups lives on the device
@@ -332,7 +333,28 @@ nbx_status put_groups(nbx_ctx* c, const std::vector<Group>& groups) {
     HIPCHK(c, hipMemcpyAsync(c->groups.p, groups.data(), groups.size() * sizeof(Group), hipMemcpyHostToDevice,
                              c->stream));
   c->ngroups = (int64_t)groups.size();
+  c->groups_theta = c->cfg.theta;
   return NBX_OK;
+}
+
+// The group width depends on theta: before a build, the table of the theta it
+// is for.  (nbx_set_theta only marks: it neither allocates nor waits.)
+nbx_status update_groups(nbx_ctx* c) {
+  if (c->physics || c->groups_theta == c->cfg.theta) return NBX_OK;
+  bool same = true;
+  for (const int64_t n : c->sys_n) same &= walk_width(n, c->groups_theta) == walk_width(n, c->cfg.theta);
+  if (same) {
+    c->groups_theta = c->cfg.theta;
+    return NBX_OK;
+  }
+  try {
+    const std::vector<Group> groups = ref_groups(c);
+    const nbx_status st = put_groups(c, groups);
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    return st;
+  } catch (const std::bad_alloc&) {
+    return fail(c, NBX_ERR_NOMEM, "no host memory for the walk groups");
+  }
 }
 
 // Host-built tables for the current systems: body offsets, walk groups,
@@ -650,6 +672,7 @@ nbx_status refit_tree(nbx_ctx* c) {
 // Tree of the current positions: per-system roots, keys, sort, gather,
 // layout, multipoles.
 nbx_status build_tree(nbx_ctx* c) {
+  NBXCHK(update_groups(c));
   const uint64_t* skey = nullptr;
   const bool patch = c->patch_ok && c->patch_wait == 0;
   if (c->patch_wait > 0) --c->patch_wait;
@@ -1413,12 +1436,6 @@ nbx_status nbx_set_theta(nbx_ctx* c, double theta) {
   c->cfg.theta = theta;
   c->acc_valid = false;
   ++c->gen;
-  if (!c->physics && !c->sys_n.empty()) {                  // the group width depends on theta
-    NBXCHK(check_ctx(c));
-    const std::vector<Group> groups = ref_groups(c);
-    NBXCHK(put_groups(c, groups));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-  }
   return NBX_OK;
 }
 

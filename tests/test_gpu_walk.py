@@ -77,6 +77,28 @@ def test_theta_changes_the_width():
             assert np.array_equal(got, f.accel())
 
 
+def test_setting_theta_allocates_nothing():
+    """nbx_set_theta marks; the next evaluation brings the group table up to
+    date, captured runs included."""
+    ps = [ic.plummer(n, seed=n, virial=None) for n in (200003, 5000)]
+    with Engine(theta=0.5, adaptive_dt=False) as e:
+        e.set_graph(1)
+        e.upload_batch(ps)
+        e.run(1e-4, 4)
+        held = e.device_bytes()
+        e.set_theta(0.35)               # four times as many groups for the first system
+        assert e.device_bytes() == held
+        e.run(1e-4, 4)
+        got = e.download()
+    with Engine(theta=0.5, adaptive_dt=False) as f:
+        f.upload_batch(ps)
+        for theta in (0.5, 0.35):
+            f.set_theta(theta)
+            for _ in range(4):
+                f.step(1e-4)
+        assert np.array_equal(got, f.download())
+
+
 @pytest.mark.parametrize("sizes", [[1, 20481], [20481, 1, 1, 1], [20480, 20481], [5, 70, 30000, 3, 21000, 600], [25000] + [9] * 40])
 def test_batch_of_mixed_widths(sizes):
     """The group table of a batch whose widths differ is cut by bodies: every
