@@ -312,8 +312,9 @@ nbx_status nbx_debug_tree(nbx_ctx* ctx, int32_t* depth, int32_t* leaf, int32_t* 
 /* The walk groups of the current positions, at most cap of them: first
  * body (an index into the leaf order of nbx_debug_tree's perm), body count
  * and system.  *ngroups receives the full count.  Reference mode: runs of
- * 64 consecutive bodies of a system; physics mode: groups packed from the
- * tree (at most group_size bodies inside one node). */
+ * consecutive bodies of a system, 8, 16, 32 or 64 by its size and theta;
+ * physics mode: groups packed from the tree (at most group_size bodies inside
+ * one node). */
 nbx_status nbx_debug_groups(nbx_ctx* ctx, int64_t cap, int32_t* first, int32_t* count, int32_t* sys,
                             int64_t* ngroups);
 

@@ -1831,31 +1831,20 @@ nbx_status nbx_debug_groups(nbx_ctx* c, int64_t cap, int32_t* first, int32_t* co
     NBXCHK(sync_scalars(c));
     c->ntgroups = c->hsc->tree_groups;
   }
-  if (!c->physics) {                                       // runs of 64 (the walk may split them)
-    int32_t at = 0;
-    for (size_t s = 0; s < c->sys_n.size(); ++s)
-      for (const int32_t end = at + (int32_t)c->sys_n[s]; at < end; at = std::min<int32_t>(at + kWave, end)) {
-        if (*ngroups < cap) {
-          first[*ngroups] = at;
-          count[*ngroups] = std::min<int32_t>(kWave, end - at);
-          sys[*ngroups] = (int32_t)s;
-        }
-        ++*ngroups;
-      }
-    return NBX_OK;
-  }
-  const int64_t ng = c->ntgroups;
-  const Group* dg = P<Group>(c->tgroups);
-  *ngroups = ng;
-  const int64_t k = std::min(ng, cap);
-  if (k == 0) return NBX_OK;
-  std::vector<Group> h((size_t)k);
-  HIPCHK(c, hipMemcpyAsync(h.data(), dg, (size_t)k * sizeof(Group), hipMemcpyDeviceToHost, c->stream));
+  const int64_t ng = c->physics ? c->ntgroups : c->ngroups;
+  if (ng == 0) return NBX_OK;
+  std::vector<Group> h((size_t)ng);
+  HIPCHK(c, hipMemcpyAsync(h.data(), (c->physics ? c->tgroups : c->groups).p, (size_t)ng * sizeof(Group),
+                           hipMemcpyDeviceToHost, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
-  for (int64_t j = 0; j < k; ++j) {
-    first[j] = h[(size_t)j].first;
-    count[j] = h[(size_t)j].count;
-    sys[j] = h[(size_t)j].sys;
+  for (const Group& g : h) {
+    if (g.count == 0) continue;                            // (fills an XCD's part of the reference table)
+    if (*ngroups < cap) {
+      first[*ngroups] = g.first;
+      count[*ngroups] = g.count;
+      sys[*ngroups] = g.sys;
+    }
+    ++*ngroups;
   }
   return NBX_OK;
 }

@@ -113,3 +113,26 @@ def test_batch_of_mixed_widths(sizes):
             f.upload(p)
             assert np.array_equal(a[at:at + len(p)], f.accel())
         at += len(p)
+
+
+@pytest.mark.parametrize("sizes", [[1], [1000], [20481], [1, 20481], [5, 70, 30000, 3, 21000, 600], [25000] + [9] * 40])
+def test_group_table(sizes):
+    """The groups the walk works through cover each body once, inside one
+    system, in runs of that system's width, before and after theta moves it."""
+    ps = [ic.plummer(n, seed=k, virial=None) for k, n in enumerate(sizes)]
+    with Engine(theta=0.5) as e:
+        e.upload_batch(ps)
+        for theta in (0.5, 0.3, 0.9):
+            e.set_theta(theta)
+            first, count, sys_ = e.debug_groups()
+            order = np.argsort(first)
+            assert np.array_equal(first[order], np.concatenate([[0], np.cumsum(count[order])[:-1]]))
+            assert count.sum() == sum(sizes)
+            at = 0
+            for s, n in enumerate(sizes):
+                c = count[sys_ == s]
+                assert c.sum() == n and np.all((first[sys_ == s] >= at) & (first[sys_ == s] + c <= at + n))
+                width = {(1000, 0.5): 16, (20481, 0.5): 32, (20481, 0.3): 16, (30000, 0.5): 32}.get((n, theta))
+                if width is not None:
+                    assert c.max() == width and np.sum(c < width) <= 1, (n, theta)
+                at += n
