@@ -412,7 +412,7 @@ int sys_bits(int nsys) {
 
 // The unit pass's view of the layout (the buffers the last build filled).
 UnitArgs unit_args(nbx_ctx* c) {
-  return UnitArgs{c->n, unit_count(c->n), kUnitSpan, P<int32_t>(c->lcp), P<uint32_t>(c->cnt_s),
+  return UnitArgs{c->n, unit_count(c->n), unit_span(c->n), P<int32_t>(c->lcp), P<uint32_t>(c->cnt_s),
                   P<uint32_t>(c->lvl_part), P<int32_t>(c->level_list), P<uint32_t>(c->end_list), c->sc,
                   P<int32_t>(c->over)};
 }

@@ -212,7 +212,7 @@ nbx_status accel_in_arena(const Arena& A, int64_t n, const double* x, const doub
   uint32_t* end_list = A.at<uint32_t>(kLayout.end_list);
   launch_emit(n, lcp, cnt_s, part, St, sy, sc, nodes, heads, level_list, end_list, (uint32_t)(kNaNodes + 1),
               (uint32_t)kNaNodes, s);
-  launch_upward_units(UnitArgs{n, unit_count(n), kUnitSpan, lcp, cnt_s, part, level_list, end_list, sc,
+  launch_upward_units(UnitArgs{n, unit_count(n), unit_span(n), lcp, cnt_s, part, level_list, end_list, sc,
                                A.at<int32_t>(kLayout.over)},
                       nodes, heads, theta, St.sys, sy, s);
   double* acc[3] = {A.at<double>(kLayout.acc[0]), A.at<double>(kLayout.acc[1]), A.at<double>(kLayout.acc[2])};

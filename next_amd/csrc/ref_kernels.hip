@@ -619,7 +619,10 @@ __global__ __launch_bounds__(kWave) void k_check(DevScalars* sc, int64_t cap_rec
 // comes from the first child, the half-width from the system's root.
 //
 // The unit's nodes keep mass, centre and first body in LDS (36 bytes each).
-constexpr int kUnitNodes = 2048;
+// 1,856 nodes (a unit of up to 1,152 bodies has about 1,700) so that two units
+// fit a CU; with 2,048 one did, and 512 systems of 500 bodies took 80 us instead
+// of 59, 262,144 bodies 98 instead of 80.
+constexpr int kUnitNodes = 1856;
 struct UnitMoments {
   double m[kUnitNodes], x[kUnitNodes], y[kUnitNodes], z[kUnitNodes];
   int32_t first[kUnitNodes];
@@ -766,6 +769,7 @@ __global__ __launch_bounds__(kBlock) void k_upward_unit(UnitArgs a, RefNode* __r
                                                         const int32_t* __restrict__ sys,
                                                         const double* __restrict__ root) {
   __shared__ UnitMoments lm;
+  static_assert(2 * (sizeof(UnitMoments) + unit_lds<kUnitNodes>()) <= 160 * 1024, "two units on a CU");
   const double half = root[3];
   upward_unit<kUnitNodes>(
       a,

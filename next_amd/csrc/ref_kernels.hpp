@@ -118,9 +118,14 @@ struct UnitArgs {
   DevScalars* sc;
   int32_t* over;
 };
-constexpr int64_t kUnitsMax = 262144;
 constexpr int32_t kUnitSpan = 768;   // bodies per unit: about 1,150 nodes
-constexpr int32_t unit_count(int64_t n) { return n >= 2 * kUnitSpan ? (int32_t)(n / kUnitSpan) : 1; }
+constexpr int64_t kUnitsMax = 512 * kUnitSpan;   // two units on each of 256 CUs
+// Units of n / units bodies, at most kUnitSpan, and up to half as many more where
+// the boundaries move to the smallest lcp (units.hpp): 1,152 bodies, which have
+// about 1,700 nodes.  (All of kUnitSpan but a longer last one left that with up
+// to 2,100 nodes, too many for LDS.)
+constexpr int32_t unit_count(int64_t n) { return n <= 1230 ? 1 : (int32_t)((n + kUnitSpan - 1) / kUnitSpan); }
+constexpr int32_t unit_span(int64_t n) { return (int32_t)(n / unit_count(n)); }
 void launch_upward_units(const UnitArgs& a, RefNode* nodes, WalkHead* heads, double theta, const int32_t* sys,
                          const SysArrays& sy, hipStream_t s);
 void launch_fill_u32(int64_t n, uint32_t* a, uint32_t v, hipStream_t s);

@@ -18,11 +18,12 @@
 // A launch per depth takes 5 to 6 us for every depth of up to some thousand
 // nodes (a dependent chain of list entry, up to 8 children one after another,
 // system and root, and 400 to 900 FP64 instructions), 10 to 20 depths a build.
-// Measured, whole upward pass: 16,384 bodies 77 -> 65 us, 50,021 89 -> 63,
-// 200,003 94 -> 82; forces of 1,000 bodies 30 us less per call, of 12,289 22.  Beyond that a
-// launch per depth is better (366,000 bodies in 40 systems 103 against 117,
-// 2^20 bodies 185 against 203 to 237 us): LDS holds two units per CU, and the
-// nodes that end beyond their units, one workgroup's work, grow with the units.
+// Measured, whole upward pass: 1,000 bodies 53 -> 34 us, 16,384 69 -> 59, 65,536
+// 88 -> 67, 262,144 96 -> 81, 366,000 107 -> 84, 128 systems of 2,000 76 -> 68.  A CU
+// holds two units (80 KB of LDS each at most), the chip 512: with more, a second
+// round of units costs what a launch per depth saves (512 systems of 1,000, 666
+// units: 114 against 96 us, 2^20 bodies 203 against 178), and the nodes that end
+// beyond their units, one workgroup's work, grow with the units.
 #pragma once
 
 #include <algorithm>
@@ -37,7 +38,7 @@ namespace nbx {
 // every thread of a kBlock-thread block; scratch: kBlock / kWave words.
 __device__ __forceinline__ int64_t unit_start(int64_t u, int32_t span, const int32_t* __restrict__ lcp,
                                               unsigned long long* scratch) {
-  const int64_t lo = u * span - span / 4;                    // u span + span / 4 <= n - 1: units = n / span
+  const int64_t lo = u * span - span / 4;                    // u span + span / 4 <= n - 1: units * span <= n
   unsigned long long best = ~0ull;
   for (int32_t k = threadIdx.x; k < span / 2; k += kBlock) {
     const unsigned long long v = ((unsigned long long)(uint32_t)(lcp[lo + k] + 1) << 32) | (uint32_t)k;
@@ -63,6 +64,12 @@ struct UnitView {
   uint16_t* skips;          // skip pointer, as a slot
   __device__ __forceinline__ int slot(int32_t k) const { return k - first; }
 };
+
+// LDS of upward_unit, its alignment included.
+template <int NODES>
+constexpr size_t unit_lds() {
+  return kBlock / kWave * 8 + 5 * kMaxDepthSlots * 4 + 2 * 4 + NODES * 6 + 8 * 16;
+}
 
 // The body of a unit kernel (kBlock threads, one unit per block).
 // load(view, k): called once for every node k of the unit, in parallel, when

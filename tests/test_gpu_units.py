@@ -1,8 +1,8 @@
-"""The upward pass in units of bodies (reference mode up to 262,144 bodies):
+"""The upward pass in units of bodies (reference mode up to 393,216 bodies):
 whole node tables against the oracle's, bit for bit, at the sizes where the
-number of units changes (768 bodies each, one unit below 1,536), with clumps
-whose chains of cells make a unit too large for LDS, with several systems in a
-context, and at both sides of the size where a launch per depth takes over.
+number of units changes (at most 768 bodies each, one unit up to 1,230), with
+clumps whose chains of cells make a unit too large for LDS, with several systems
+in a context, and at both sides of the size where a launch per depth takes over.
 """
 import numpy as np
 import pytest
@@ -42,6 +42,16 @@ def test_units_too_large_for_lds(n):
 
 @pytest.mark.parametrize("n", [262144, 262145])
 def test_both_sides_of_the_largest(n):
+    same_tables(ic.plummer(n, seed=2, virial=None))
+
+
+@pytest.mark.parametrize("n", [1230, 1231, 2305, 3073, 16385])
+def test_units_of_equal_length(n):
+    same_tables(ic.plummer(n, seed=n, virial=None))
+
+
+@pytest.mark.parametrize("n", [393216, 393217])
+def test_both_sides_of_512_units(n):
     same_tables(ic.plummer(n, seed=2, virial=None))
 
 
