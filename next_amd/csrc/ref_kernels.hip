@@ -1437,8 +1437,8 @@ void launch_upward_units(const UnitArgs& a, RefNode* nodes, WalkHead* heads, dou
   hipLaunchKernelGGL(k_upward_unit, dim3((unsigned)a.units), dim3(kBlock), 0, s, a, nodes, heads, 1.0 / theta, sys,
                      sy.root);
   if (a.units > 1)
-    hipLaunchKernelGGL(k_upward_over, dim3((unsigned)sy.nsys), dim3(kOverBlock), 0, s, a, sy, nodes, heads,
-                       1.0 / theta, sys);
+    hipLaunchKernelGGL(k_upward_over, dim3((unsigned)std::min(sy.nsys, kOverBlocks)), dim3(kOverBlock), 0, s, a, sy,
+                       nodes, heads, 1.0 / theta, sys);
 }
 void launch_walk(const Group* groups, int64_t ngroups, const RefNode* nodes, const WalkHead* heads,
                  const StateArrays& st,

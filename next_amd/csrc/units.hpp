@@ -173,38 +173,45 @@ __device__ __forceinline__ void upward_unit(const UnitArgs& a, Load load, Node n
   }
 }
 
-// The nodes that end beyond their units, depth by depth: one workgroup of
-// kOverBlock threads per system (a system's nodes are its own).  The depth
-// mask is cleared by the next build's first kernel.
-constexpr int kOverBlock = 1024;
+// The nodes that end beyond their units, depth by depth: a workgroup of
+// kOverBlock threads takes one system after another (a system's nodes are its
+// own).  A system of at most span / 2 bodies has none: where a unit ends inside
+// a system, the window its end was chosen from holds that system's bodies only.
+// At most kOverBlocks workgroups: one for each of 16,000 systems of 16 bodies
+// took 27 us to find nothing.  The depth mask is cleared by the next build's
+// first kernel.
+constexpr int kOverBlock = 1024, kOverBlocks = 512;
 template <class Node>
 __device__ __forceinline__ void upward_over(const UnitArgs& a, const SysArrays& sy, Node node) {
   __shared__ int32_t list[kOverBlock];
   __shared__ int32_t count;
   if (a.sc->abort_flags) return;
-  unsigned long long m = a.sc->over_depths;
+  const unsigned long long depths = a.sc->over_depths;
+  if (depths == 0) return;
   const int t = threadIdx.x;
-  const int s = blockIdx.x;
-  const int32_t root = sy.sroot[s], end = sy.send[s];
-  // units that can hold the system's bodies
-  const int32_t ub = (int32_t)std::max<int64_t>((int64_t)sy.soff[s] / a.span - 1, 0);
-  const int32_t ue = (int32_t)std::min<int64_t>((int64_t)sy.soff[s + 1] / a.span + 2, a.units);
   const UnitView view{0, false, nullptr};
-  while (m) {
-    const int d = 63 - __clzll((long long)m);
-    m &= ~(1ull << d);
-    for (int32_t u0 = ub; u0 < ue; u0 += kOverBlock) {
-      if (t == 0) count = 0;
-      __syncthreads();
-      const int32_t k = u0 + t < ue ? a.over[(int64_t)d * a.units + u0 + t] : -1;
-      if (k >= 0) {
-        const int32_t id = a.level_list[k];
-        if (id >= root && id < end) list[atomicAdd(&count, 1)] = k;
+  for (int32_t s = blockIdx.x; s < sy.nsys; s += gridDim.x) {
+    if (sy.soff[s + 1] - sy.soff[s] <= a.span / 2) continue;   // (uniform)
+    const int32_t root = sy.sroot[s], end = sy.send[s];
+    // units that can hold the system's bodies
+    const int32_t ub = (int32_t)std::max<int64_t>((int64_t)sy.soff[s] / a.span - 1, 0);
+    const int32_t ue = (int32_t)std::min<int64_t>((int64_t)sy.soff[s + 1] / a.span + 2, a.units);
+    for (unsigned long long m = depths; m;) {
+      const int d = 63 - __clzll((long long)m);
+      m &= ~(1ull << d);
+      for (int32_t u0 = ub; u0 < ue; u0 += kOverBlock) {
+        if (t == 0) count = 0;
+        __syncthreads();
+        const int32_t k = u0 + t < ue ? a.over[(int64_t)d * a.units + u0 + t] : -1;
+        if (k >= 0) {
+          const int32_t id = a.level_list[k];
+          if (id >= root && id < end) list[atomicAdd(&count, 1)] = k;
+        }
+        __syncthreads();
+        for (int32_t j = t; j < count; j += kOverBlock)
+          node(view, a.level_list[list[j]], (int32_t)a.end_list[list[j]], d);
+        __syncthreads();
       }
-      __syncthreads();
-      for (int32_t j = t; j < count; j += kOverBlock)
-        node(view, a.level_list[list[j]], (int32_t)a.end_list[list[j]], d);
-      __syncthreads();
     }
   }
 }

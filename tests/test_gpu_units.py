@@ -68,3 +68,21 @@ def test_systems_share_units():
             f.upload(p)
             f.run(1e-3, 2)
             assert np.array_equal(got[s], f.download()), s
+
+
+def test_more_systems_than_workgroups():
+    """Nodes beyond their units are worked off by at most 512 workgroups, and
+    systems of up to half a unit have none: systems on both sides of that, and
+    beyond the 512th, among many tiny ones."""
+    small, large = ic.plummer(2, seed=1, virial=None), [ic.plummer(n, seed=n, virial=None) for n in
+                                                       (3000, 383, 384, 385, 386, 5000, 770)]
+    ps = [large[5]] + [small] * 600 + large + [small] * 500 + [large[0]]
+    with Engine(theta=0.5) as e:
+        e.upload_batch(ps)
+        e.run(1e-3, 2)
+        got = {k: e.download_system(k) for k in [0, 1, 600, 1100, len(ps) - 1] + list(range(601, 608))}
+    for k, state in got.items():
+        with Engine(theta=0.5) as f:
+            f.upload(ps[k])
+            f.run(1e-3, 2)
+            assert np.array_equal(state, f.download()), k
