@@ -158,26 +158,45 @@ void launch_out_gather(int64_t j0, int64_t len, int64_t cnt, const uint32_t* inv
 // alone, so a system's sums are the same alone and in a batch.  Narrow
 // groups give a small system enough waves and short ones; wide groups share
 // more of the traversal, which is what a batch of many systems needs, the more
-// so the larger theta.  The lines lie where the narrower groups would make
-// such a batch slower than one union traversal per 64 targets was ("u").
+// so the larger theta, and what a large system needs too.  Up to 20,480 bodies
+// the lines lie where the narrower groups would make a batch of Plummer spheres
+// slower than one union traversal per 64 targets was ("u"); above, at the
+// fastest width.  64 bodies are one wave's work either way.
 // Walk (us, Plummer spheres), width u / 8 / 16 / 32 / 64:
-//   theta  n        alone                          batch
-//   0.3    2,000    502 /  97 / 140 / 223 / 397    512: 3,283 / 3,295 / 3,111 / 3,262 / 3,543
-//   0.3    16,384   981 / 212 / 239 / 410 / 565     64: 5,595 / 4,946 / 4,868 / 5,201 / 5,561
-//   0.4    2,000    343 /  76 / 107 / 134 / 231    512: 2,143 / 2,506 / 2,068 / 2,012 / 2,077
-//   0.5    1,000    237 /  56 /  72 / 103 / 152    512:   786 /   902 /   705 /   644 /   675
-//   0.5    2,000    270 /  84 /  81 / 120 / 181    512: 1,585 / 2,115 / 1,632 / 1,423 / 1,404
-//   0.5    16,384   369 /  93 / 117 / 141 / 205     64: 2,047 / 2,579 / 2,016 / 1,724 / 1,557
-//   0.5    32,768   386 / 127 / 130 / 162 / 215     64: 3,840 /     - / 4,175 / 3,490 /     -
-//   0.5    65,536   426 / 217 / 171 / 185 / 252     16: 2,196 / 2,810 / 2,127 / 1,833 / 1,562
-//   0.5    100,000  490 / 326 / 276 / 248 / 262     12: 2,538 / 3,368 / 2,533 / 2,182 / 1,742
-//   0.5    200,000  677 / 611 / 491 / 461 / 410
-//   0.7    16,384   201 /  69 /  75 / 100 / 131     64: 1,267 / 2,030 / 1,435 / 1,112 /   825
-//   0.7    65,536   238 / 173 / 122 / 126 / 170     16: 1,354 / 2,189 / 1,518 / 1,170 /   810
+//   theta  n        alone                              batch
+//   0.3    64        39 /  29 /  32 /  41 /  41      4,000:   103 /   250 /   174 /   140 /   110
+//   0.3    500      268 /  57 /  93 / 138 / 215        512:   475 /   573 /   505 /   512 /   542
+//   0.3    1,000    403 / 107 / 133 / 198 / 295        512: 1,399 / 1,319 / 1,211 / 1,295 / 1,434
+//   0.3    16,384   941 / 226 / 302 / 447 / 584         64: 5,600 / 4,926 / 4,816 / 5,194 / 5,504
+//   0.39   200,003 1,011 / 752 / 675 / 685 / 740
+//   0.35   2^20    5,155 / 5,032 / 4,372 / 4,160 / 3,750 (uniform 3,478 / 3,575 / 3,044 / 3,025 / 3,134)
+//   0.3    2^20    7,500 / 6,544 / 6,089 / 6,240 / 5,917 (uniform 4,953 / 4,457 / 4,162 / 4,438 / 4,851)
+//   0.39   2^22, uniform: 11,130 / 13,919 / 10,922 / 9,841 / 9,751
+//   0.4    2,000    358 /  70 /  91 / 137 / 224        512: 2,105 / 2,527 / 2,076 / 1,984 / 2,078
+//   0.44   100,000  592 / 338 / 303 / 285 / 302         10: 2,650 / 3,073 / 2,441 / 2,196 / 1,911
+//   0.5    1,000    246 /  57 /  70 / 103 / 152        512:   767 /   885 /   677 /   635 /   643
+//   0.5    2,000    270 /  57 /  78 / 112 / 162        512: 1,522 / 2,115 / 1,619 / 1,408 / 1,388
+//   0.5    16,384   343 /  84 / 108 / 173 / 195         64: 1,972 / 2,577 / 1,975 / 1,686 / 1,485
+//   0.5    32,768   378 / 117 / 121 / 200 / 232         32: 2,035 / 2,700 / 2,063 / 1,744 / 1,501
+//   0.5    65,536   441 / 218 / 165 / 185 / 248         16: 2,101 / 2,801 / 2,131 / 1,790 / 1,491
+//   0.5    100,000  458 / 305 / 258 / 233 / 265         10: 2,067 / 2,752 / 2,084 / 1,763 / 1,417
+//   0.5    200,003  631 / 583 / 449 / 432 / 417
+//   0.55   1,000    217 /  54 /  65 /  89 / 137        512:   667 /   833 /   623 /   567 /   575
+//   0.55   16,384   305 /  78 /  94 / 126 / 181         64: 1,683 / 2,388 / 1,779 / 1,466 / 1,203
+//   0.7    16,384   206 /  74 /  79 /  94 / 135         64: 1,210 / 2,021 / 1,419 / 1,115 /   782
+//   0.85   16,384   165 /  61 /  83 / 107 / 111         64:   940 / 1,779 / 1,216 /   926 /   639
+//   1.0    1,000    115 /  40 /  51 /  57 /  77        512:   330 /   621 /   429 /   327 /   285
+//   1.0    16,384   130 /  83 /  82 /  91 /  91         64:   757 / 1,583 / 1,066 /   779 /   539
+// Batches of uniform spheres, which have less to share, cross earlier: a step
+// of 64 of 16,384 bodies at theta 0.5 takes 1,783 us against 1,676, of 512 of
+// 2,000 1,479 against 1,315; alone the wider groups that would mend it cost
+// 35 to 65 us of a walk of 80 to 110.
 inline int32_t walk_width(int64_t n, double theta) {
-  if (theta <= 0.32 && n <= 4096) return 8;
-  if (theta < 0.4 || n <= (theta < 0.45 ? 98304 : theta <= 0.55 ? 20480 : 0)) return 16;
-  return n <= 196608 ? 32 : 64;
+  if (n <= 64) return 64;
+  if (theta <= 0.32 && n >= 896 && n <= 4096) return 8;
+  if (theta < 0.35) return 16;
+  if (n <= (theta < 0.4 ? 524288 : theta < 0.45 ? 98304 : theta <= 0.5 ? 20480 : theta <= 0.55 ? 1500 : 0)) return 16;
+  return n <= 1500 || (n <= 196608 && theta >= 0.4 && theta <= 0.8) ? 32 : 64;
 }
 void launch_walk(const Group* groups, int64_t ngroups, const RefNode* nodes, const WalkHead* heads,
                  const StateArrays& st,

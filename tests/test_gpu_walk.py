@@ -1,9 +1,10 @@
 """The reference-mode walk at the sizes where its group width changes.
 
 The walk puts 64 / width lanes on each target of a group of `width` bodies;
-the width follows the system's size and theta (8 up to 4,096 bodies and theta
-0.32, 16 below theta 0.4, up to 98,304 bodies below 0.45 and up to 20,480 up to
-0.55, else 32 up to 196,608 bodies, then 64).
+the width follows the system's size and theta (8 for 896 to 4,096 bodies up to
+theta 0.32; 16 below theta 0.35, up to 524,288 bodies below 0.4, 98,304 below
+0.45, 20,480 up to 0.5 and 1,500 up to 0.55; else 32 up to 1,500 bodies, and up
+to 196,608 between 0.4 and 0.8; else, and up to 64 bodies, 64).
 Accelerations against the oracle's walk (octree.h:133-179) at the edges of
 those ranges and of a group, with dark-matter targets (octree.h:146-148).
 Tolerance: the accelerations' own, median <= 1e-12 and 99th percentile <=
@@ -46,6 +47,18 @@ def test_small(n, theta):
                                      (20480, 0.56), (196609, 0.56)])
 def test_width_edges(n, theta):
     check(ic.plummer(n, seed=3, virial=None, type_fraction_dm=0.1), theta, f"n={n} theta={theta}")
+
+
+@pytest.mark.parametrize("n,theta,width", [(64, 0.3, 64), (65, 0.3, 16), (895, 0.32, 16), (896, 0.32, 8),
+                                           (1500, 0.55, 16), (1501, 0.55, 32), (1500, 0.56, 32), (1500, 0.95, 32),
+                                           (1501, 0.8, 32), (1501, 0.81, 64), (20480, 0.51, 32), (196608, 0.81, 64),
+                                           (524288, 0.35, 16), (524289, 0.35, 64), (524289, 0.34, 16)])
+def test_widths(n, theta, width):
+    p = ic.plummer(n, seed=8, virial=None, type_fraction_dm=0.1)
+    with Engine(theta=theta) as e:
+        e.upload(p)
+        assert e.debug_groups()[1].max() == min(n, width)
+    check(p, theta, f"n={n} theta={theta}")
 
 
 @pytest.mark.parametrize("lo,hi", [(-30, 30), (-3, 3), (200, 210), (-210, -200)])
