@@ -20,6 +20,8 @@
 //                     2- and 3-body closed forms; canonical-prefix rule
 //   orc_tree_accel    golden acc.f64 at theta 0.3/0.5/0.7; theta=0 equals
 //                     brute force with leaf softening; N=2 analytic
+//   orc_tree_accel_subset_ext   equality with orc_tree_accel_subset to the
+//                     rounding of its sums
 //   orc_adaptive_dt   closed-form clamps; golden dt sequence
 //   orc_step/orc_run  golden multi-step state and dt sequence
 //   orc_direct        Plummer-softened direct sum: two-body closed form and
@@ -231,6 +233,36 @@ void walk(const Tree& t, int id, int i, const double* x, const double* y, const 
     if (n.child[c] >= 0) walk(t, n.child[c], i, x, y, z, m, type, theta, ax, ay, az);
 }
 
+// The same walk with 64-bit mantissas: the opening decisions and the node
+// moments are the FP64 walk's, each interaction and the sums are not rounded
+// to FP64.
+void walk_ext(const Tree& t, int id, int i, const double* x, const double* y, const double* z,
+              const double* m, const int32_t* type, double theta, long double a[3]) {
+  using L = long double;
+  const Node& n = t.nodes[id];
+  if (n.m == 0) return;
+  if (n.leaf && n.body == i) return;
+  const double ex = n.cx - x[i], ey = n.cy - y[i], ez = n.cz - z[i];
+  if (!n.leaf && !((n.s / std::sqrt(ex * ex + ey * ey + ez * ez + 1e-20)) < theta)) {
+    for (int c = 0; c < 8; ++c)
+      if (n.child[c] >= 0) walk_ext(t, n.child[c], i, x, y, z, m, type, theta, a);
+    return;
+  }
+  const L d[3] = {(L)n.cx - x[i], (L)n.cy - y[i], (L)n.cz - z[i]};
+  const L r2 = d[0] * d[0] + d[1] * d[1] + d[2] * d[2];
+  L eps = ((L)n.s * 0.015 + std::cbrt((L)n.m) * 0.002) / (1 + 10 * std::sqrt(r2 + (L)1e-20));
+  if (eps < 1e-4) eps = 1e-4;
+  if (type[i] == 1) {
+    const L alt = 2 * (L)n.s / std::pow((L)n.m / m[i], (L)0.333333333);
+    if (eps < alt) eps = alt;
+  }
+  const L dinv = 1 / std::sqrt(r2 + eps * eps), inv3 = dinv * dinv * dinv, inv5 = inv3 * dinv * dinv;
+  const L qd[3] = {n.qxx * d[0] + n.qxy * d[1] + n.qxz * d[2], n.qxy * d[0] + n.qyy * d[1] + n.qyz * d[2],
+                   n.qxz * d[0] + n.qyz * d[1] + n.qzz * d[2]};
+  const L q = qd[0] * d[0] + qd[1] * d[1] + qd[2] * d[2];
+  for (int k = 0; k < 3; ++k) a[k] += d[k] * (n.m * inv3 - 2.5L * q * inv5 * dinv * dinv) + qd[k] * inv5;
+}
+
 void preorder(const Tree& t, int id, int depth, int64_t& k, int32_t* dep, int32_t* leaf,
               int32_t* body, int32_t* cmask, double* geo, double* mass, double* com, double* q,
               int32_t* perm, int64_t& pk) {
@@ -325,6 +357,22 @@ void orc_tree_accel_subset(const orc_tree* t, const double* x, const double* y, 
     double a0 = 0, a1 = 0, a2 = 0;
     walk(t->t, 0, (int)targets[k], x, y, z, m, type, theta, a0, a1, a2);
     ax[k] = a0; ay[k] = a1; az[k] = a2;
+  }
+}
+
+// The walk with 64-bit mantissas for a subset of targets: component c of target
+// k is hi[3 k + c] + lo[3 k + c].
+void orc_tree_accel_subset_ext(const orc_tree* t, const double* x, const double* y, const double* z,
+                               const double* m, const int32_t* type, double theta, int64_t nt,
+                               const int64_t* targets, double* hi, double* lo, int threads) {
+#pragma omp parallel for schedule(dynamic, 16) num_threads(threads)
+  for (int64_t k = 0; k < nt; ++k) {
+    long double a[3] = {0, 0, 0};
+    walk_ext(t->t, 0, (int)targets[k], x, y, z, m, type, theta, a);
+    for (int c = 0; c < 3; ++c) {
+      hi[3 * k + c] = (double)a[c];
+      lo[3 * k + c] = (double)(a[c] - hi[3 * k + c]);
+    }
   }
 }
 

@@ -41,6 +41,7 @@ def lib():
         L.orc_tree_accel_subset.argtypes = [C.c_void_p, f64p, f64p, f64p, f64p, i32p, C.c_double, C.c_int64,
                                             np.ctypeslib.ndpointer(np.int64, flags="C_CONTIGUOUS"), f64p, f64p,
                                             f64p, C.c_int]
+        L.orc_tree_accel_subset_ext.argtypes = L.orc_tree_accel_subset.argtypes[:9] + [f64p, f64p, C.c_int]
         L.orc_adaptive_dt.argtypes = [C.c_int64, f64p, f64p, f64p, C.c_double]
         L.orc_adaptive_dt.restype = C.c_double
         L.orc_step.argtypes = [C.c_int64] + [f64p] * 7 + [i32p, C.c_double, C.c_double, C.c_int]
@@ -126,6 +127,23 @@ def accel_subset(x, y, z, m, typ, theta, targets, threads=8):
     finally:
         L.orc_tree_free(h)
     return np.stack(out, axis=1)
+
+
+def accel_subset_ext(x, y, z, m, typ, theta, targets, threads=8):
+    """The same walk with 64-bit mantissas: (hi, lo), the accelerations being
+    their exact sum."""
+    L = lib()
+    x, y, z, m = (_c(a, np.float64) for a in (x, y, z, m))
+    tg = _c(targets, np.int64)
+    hi, lo = np.zeros((len(tg), 3)), np.zeros((len(tg), 3))
+    h = L.orc_tree_build(len(x), x, y, z, m)
+    try:
+        if L.orc_tree_error(h):
+            raise RuntimeError("oracle: coincident bodies (depth cap)")
+        L.orc_tree_accel_subset_ext(h, x, y, z, m, _c(typ, np.int32), theta, len(tg), tg, hi, lo, threads)
+    finally:
+        L.orc_tree_free(h)
+    return hi, lo
 
 
 def adaptive_dt(vx, vy, vz, base):

@@ -73,6 +73,26 @@ def test_dark_matter_masses(lo, hi):
     check(p, 0.5, f"masses 1e{lo}..1e{hi}")
 
 
+@pytest.mark.parametrize("n", [200003, 1 << 20])
+def test_sums_of_wide_groups(n):
+    """A lane that has a target to itself adds up to some thousand terms, the
+    distant nodes of the whole group first.  Against 64-bit mantissas, the median
+    error may exceed that of NEXT's own FP64 walk by 30 % (1/sqrt by a Newton
+    step where NEXT's is correctly rounded); in one running sum from far to near it
+    did by 46 %, summed list by list it does by 3 to 12."""
+    p = ic.uniform_sphere(n, seed=1)
+    with Engine(theta=0.5) as e:
+        e.upload(p)
+        a = e.accel()
+    tg = np.random.Generator(np.random.PCG64(1)).choice(n, 4096, False).astype(np.int64)
+    hi, lo = orc.accel_subset_ext(p.x, p.y, p.z, p.m, p.type, 0.5, tg)
+    scale = np.linalg.norm(hi, axis=1)
+    mine, nexts = (np.median(np.linalg.norm((v - hi) - lo, axis=1) / scale)
+                   for v in (a[tg], orc.accel_subset(p.x, p.y, p.z, p.m, p.type, 0.5, tg)))
+    print(f"n={n}: median error {mine:.2e}, NEXT's {nexts:.2e}", flush=True)
+    assert mine <= 1.3 * nexts
+
+
 def test_theta_changes_the_width():
     """A context whose theta moves across the width rule gives the forces of
     a fresh context at that theta."""

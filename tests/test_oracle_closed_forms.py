@@ -191,3 +191,16 @@ def test_direct_subset_equals_full_sum():
     tg = np.array([0, 5, 699, 123, 5], np.int64)
     b, pb = orc.direct_subset(p.x, p.y, p.z, p.m, 0.02, tg)
     assert np.array_equal(b, a[tg]) and np.array_equal(pb, pot[tg])
+
+
+@pytest.mark.parametrize("theta", [0.0, 0.5])
+def test_extended_walk_equals_the_walk(theta):
+    """Same terms, unrounded: some 1,000 of them of a few ulp each (1e-13 is
+    1,000 u), the low parts below an ulp of the high ones."""
+    p = ic.plummer(1500, seed=6, type_fraction_dm=0.3, virial=None)
+    tg = np.arange(0, 1500, 7, dtype=np.int64)
+    a = orc.accel_subset(p.x, p.y, p.z, p.m, p.type, theta, tg)
+    hi, lo = orc.accel_subset_ext(p.x, p.y, p.z, p.m, p.type, theta, tg)
+    scale = np.linalg.norm(hi, axis=1)
+    assert np.all(np.linalg.norm(a - hi, axis=1) <= 1e-13 * scale)
+    assert np.all(np.abs(lo) <= 2.0 ** -52 * np.abs(hi)) and np.any(lo != 0)
