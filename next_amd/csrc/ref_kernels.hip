@@ -1114,9 +1114,14 @@ void k_walk(const Group* __restrict__ groups, int64_t ngroups, const RefNode* __
         const double nz = fmax(fmax(lo[2] - h.cz, h.cz - hi[2]), 0.0), fz = fmax(h.cz - lo[2], hi[2] - h.cz);
         const double r2n = __builtin_fma(nz, nz, __builtin_fma(ny, ny, nx * nx));
         const double r2f = __builtin_fma(fz, fz, __builtin_fma(fy, fy, fx * fx));
-        const double e = (double)h.acc2;                     // NaN: mixed
+        const double e = (double)h.acc2;
         acc = r2n > e;
         opened = r2f < e * kBandLow;
+        if (e != e) {                                        // the band lies outside FP32's range
+          const double q = nodes[cur].size / theta, q2 = q * q;
+          acc = r2n + 1e-20 > q2 * (1.0 + 2e-6);
+          opened = r2f + 1e-20 < q2 * (1.0 - 2e-6);
+        }
         mix = !acc && !opened;
         donate = opened && skip < end;
       }

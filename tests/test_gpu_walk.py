@@ -16,7 +16,7 @@ import pytest
 
 import oracle_lib as orc
 from next_amd import ic
-from next_amd.nbx import Engine
+from next_amd.nbx import Engine, NbxError
 
 pytestmark = pytest.mark.gpu
 
@@ -59,6 +59,46 @@ def test_widths(n, theta, width):
         e.upload(p)
         assert e.debug_groups()[1].max() == min(n, width)
     check(p, theta, f"n={n} theta={theta}")
+
+
+@pytest.mark.parametrize("theta", [0.0, 0.05, 0.3, 0.7])
+@pytest.mark.parametrize("scale", [1e-12, 1e-9, 1e-7, 1e17, 1e18, 1e20, 1e60])
+def test_lengths_outside_fp32(scale, theta):
+    """Metres instead of scale lengths, say: the squares of lengths, against
+    which the opening test's band is kept, leave FP32's range."""
+    p = ic.plummer(1500, seed=12, virial=None, type_fraction_dm=0.2)
+    for a in (p.x, p.y, p.z):
+        a *= scale
+    check(p, theta, f"scale={scale} theta={theta}")
+
+
+@pytest.mark.parametrize("theta", [0.0, 0.5])
+def test_lengths_outside_fp32_in_a_batch(theta):
+    ps = []
+    for k, scale in enumerate((1.0, 1e20, 1e-9, 1e20, 1.0)):
+        p = ic.plummer(700 + k, seed=k, virial=None)
+        for a in (p.x, p.y, p.z):
+            a *= scale
+        ps.append(p)
+    with Engine(theta=theta) as e:
+        e.upload_batch(ps)
+        a = e.accel()
+    at = 0
+    for p in ps:
+        with Engine(theta=theta) as f:
+            f.upload(p)
+            assert np.array_equal(a[at:at + len(p)], f.accel())
+        at += len(p)
+
+
+@pytest.mark.parametrize("bad", [np.inf, -np.inf, np.nan])
+def test_positions_that_are_not_finite(bad):
+    p = ic.plummer(100, seed=1, virial=None)
+    p.y[57] = bad
+    with Engine(theta=0.5) as e:
+        e.upload(p)
+        with pytest.raises(NbxError):
+            e.accel()
 
 
 @pytest.mark.parametrize("lo,hi", [(-30, 30), (-3, 3), (200, 210), (-210, -200)])
