@@ -705,6 +705,14 @@ nbx_status build_tree(nbx_ctx* c) {
 // Grid of the physics walk: the group count if the host has it, else its bound.
 int64_t group_grid(const nbx_ctx* c) { return c->ntgroups >= 0 ? c->ntgroups : c->groups_bound; }
 
+// Whether the physics walk takes evaluating waves; by the last count the host
+// has where this build's is still on the device.
+bool split_walk(const nbx_ctx* c) {
+  return phys_walk_split(c->ntgroups >= 0 ? c->ntgroups : c->hsc->tree_groups,
+                         c->n / std::max<int64_t>((int64_t)c->sys_n.size(), 1), c->cfg.group_size, c->cfg.theta,
+                         c->cfg.precision == NBX_PREC_FP64);
+}
+
 nbx_status walk(nbx_ctx* c, bool kick) {
   const bool count = (c->prof & 2) != 0;
   if (count) launch_fill_scalars(c->sc, 8, c->stream);
@@ -712,7 +720,7 @@ nbx_status walk(nbx_ctx* c, bool kick) {
   if (c->physics)
     launch_phys_walk(P<Group>(c->tgroups), group_grid(c), P<PhysNode>(c->pnodes), view(c, c->cur), sysa(c), c->cfg.eps,
                      c->cfg.leaf_size, P<double>(c->acc[0]), P<double>(c->acc[1]), P<double>(c->acc[2]), nullptr,
-                     c->sc, kick, count, c->cfg.precision == NBX_PREC_FP64,
+                     c->sc, kick, count, c->cfg.precision == NBX_PREC_FP64, split_walk(c),
                      c->amag_live ? P<float>(c->amag[c->acur]) : nullptr, c->alpha, c->cfg.theta, c->walk_list,
                      c->stream);
   else
@@ -1684,7 +1692,8 @@ static nbx_status tree_potential(nbx_ctx* c) {
   double* da = P<double>(c->dacc);
   launch_phys_walk(P<Group>(c->tgroups), group_grid(c), P<PhysNode>(c->pnodes), view(c, c->cur), sysa(c), c->cfg.eps,
                    c->cfg.leaf_size, da, da + n, da + 2 * n, P<double>(c->pot), c->sc, false, false,
-                   c->cfg.precision == NBX_PREC_FP64, nullptr, 0.0, c->cfg.theta, c->walk_list, c->stream);
+                   c->cfg.precision == NBX_PREC_FP64, split_walk(c), nullptr, 0.0, c->cfg.theta, c->walk_list,
+                   c->stream);
   HIPCHK(c, hipGetLastError());
   return NBX_OK;
 }

@@ -938,32 +938,19 @@ __global__ __launch_bounds__(kBlock) void k_energy_final(const double* __restric
   for (int k = 0; k < 5; ++k) out[5 * s + k] = t[k];
 }
 
-// Workgroups of 4 waves for launches of at most kSplitGroups groups (10 waves
-// per SIMD of the walk alone, more than its registers allow; the bound that
-// stands in for a count the host does not have yet is a quarter above it), the
-// default list size.  Few groups leave most SIMDs with one wave at most, and a wave's time
-// is then its evaluation's latency (about 2/3) plus its walk's.  Walk of a
-// single system, one wave per group against 1 + 3 waves (FP32 / FP64):
-//      2,000 bodies,     55 groups    132 ->  70 us     167 ->   77 us
-//     16,384            378           584 -> 205        771 ->  319
-//     65,536          1,476           381 -> 211        561 ->  417
-//    200,000          4,424           573 -> 484      1,074 -> 1,066
-//    327,680 (20)     7,549           842 -> 652      1,528 -> 1,370
-//    524,288         11,522         1,200 -> 1,193    2,562 -> 2,730
-//  4,194,304                        9,010 -> 9,930
-// Two evaluating waves: 275 us (FP32, 16,384 bodies), five or seven: 208.
+// Evaluating waves of a split launch (phys_walk_split).  Two: 275 us (FP32,
+// 16,384 bodies) where three take 205; five or seven: 208.
 constexpr int kWalkEval = 3;
-constexpr unsigned kSplitGroups = 10240;
 
 template <typename T, int LIST>
 void walk_dispatch(unsigned nb, const Group* groups, const PhysNode* pn, const StateArrays& st, const SysArrays& sy,
                    double eps, int nleaf, double* ax, double* ay, double* az, double* pot, DevScalars* sc, bool kick,
-                   bool count, const float* amag, float rel2, float th2, hipStream_t s) {
+                   bool count, bool eval_waves, const float* amag, float rel2, float th2, hipStream_t s) {
 #define NBX_PW(K, P, C, E)                                                                                      \
   hipLaunchKernelGGL((k_phys_walk<T, LIST, K, P, C, E>), dim3(nb), dim3(kPhysBlock * (1 + (E))), 0, s, groups, \
                      pn, st, sy, eps, nleaf, ax, ay, az, pot, sc, amag, rel2, th2)
   constexpr int kSplit = LIST == 128 ? kWalkEval : 0;
-  const bool p = pot != nullptr, split = kSplit > 0 && !count && nb <= kSplitGroups;
+  const bool p = pot != nullptr, split = kSplit > 0 && !count && eval_waves;
   if (kick) {
     if (count) NBX_PW(true, false, true, 0);
     else if (split) NBX_PW(true, false, false, kSplit);
@@ -983,17 +970,17 @@ void walk_dispatch(unsigned nb, const Group* groups, const PhysNode* pn, const S
 template <typename T>
 void walk_dispatch_list(int list, unsigned nb, const Group* groups, const PhysNode* pn, const StateArrays& st,
                         const SysArrays& sy, double eps, int nleaf, double* ax, double* ay, double* az, double* pot,
-                        DevScalars* sc, bool kick, bool count, const float* amag, float rel2, float th2,
-                        hipStream_t s) {
+                        DevScalars* sc, bool kick, bool count, bool split, const float* amag, float rel2,
+                        float th2, hipStream_t s) {
   switch (list) {
-    case 96: walk_dispatch<T, 96>(nb, groups, pn, st, sy, eps, nleaf, ax, ay, az, pot, sc, kick, count, amag, rel2,
-                                  th2, s); break;
-    case 192: walk_dispatch<T, 192>(nb, groups, pn, st, sy, eps, nleaf, ax, ay, az, pot, sc, kick, count, amag,
-                                    rel2, th2, s); break;
-    case 256: walk_dispatch<T, 256>(nb, groups, pn, st, sy, eps, nleaf, ax, ay, az, pot, sc, kick, count, amag,
-                                    rel2, th2, s); break;
-    default: walk_dispatch<T, 128>(nb, groups, pn, st, sy, eps, nleaf, ax, ay, az, pot, sc, kick, count, amag,
-                                   rel2, th2, s); break;
+    case 96: walk_dispatch<T, 96>(nb, groups, pn, st, sy, eps, nleaf, ax, ay, az, pot, sc, kick, count, split,
+                                    amag, rel2, th2, s); break;
+    case 192: walk_dispatch<T, 192>(nb, groups, pn, st, sy, eps, nleaf, ax, ay, az, pot, sc, kick, count, split,
+                                    amag, rel2, th2, s); break;
+    case 256: walk_dispatch<T, 256>(nb, groups, pn, st, sy, eps, nleaf, ax, ay, az, pot, sc, kick, count, split,
+                                    amag, rel2, th2, s); break;
+    default: walk_dispatch<T, 128>(nb, groups, pn, st, sy, eps, nleaf, ax, ay, az, pot, sc, kick, count, split,
+                                    amag, rel2, th2, s); break;
   }
 }
 
@@ -1059,18 +1046,18 @@ void launch_group_compact(int64_t n, const int32_t* gcnt, uint32_t* gmark, const
 
 void launch_phys_walk(const Group* groups, int64_t grid_groups, const PhysNode* pn, const StateArrays& st,
                       const SysArrays& sy, double eps, int nleaf, double* ax, double* ay, double* az, double* pot,
-                      DevScalars* sc, bool kick, bool count, bool fp64, const float* amag, double alpha,
+                      DevScalars* sc, bool kick, bool count, bool fp64, bool split, const float* amag, double alpha,
                       double theta, int list, hipStream_t s) {
   if (grid_groups <= 0) return;
   const unsigned nb = (unsigned)(div_up(grid_groups, 8) * 8);
   const float rel2 = (float)(alpha * alpha), th2 = (float)(theta * theta);
   if (alpha <= 0.0) amag = nullptr;
   if (fp64)
-    walk_dispatch_list<double>(list, nb, groups, pn, st, sy, eps, nleaf, ax, ay, az, pot, sc, kick, count, amag, rel2,
-                               th2, s);
+    walk_dispatch_list<double>(list, nb, groups, pn, st, sy, eps, nleaf, ax, ay, az, pot, sc, kick, count, split, amag,
+                               rel2, th2, s);
   else
-    walk_dispatch_list<float>(list, nb, groups, pn, st, sy, eps, nleaf, ax, ay, az, pot, sc, kick, count, amag, rel2,
-                              th2, s);
+    walk_dispatch_list<float>(list, nb, groups, pn, st, sy, eps, nleaf, ax, ay, az, pot, sc, kick, count, split, amag,
+                              rel2, th2, s);
 }
 
 // Waves per workgroup and halves of the sources: 8 waves on each of the 1,024

@@ -84,10 +84,46 @@ void launch_group_compact(int64_t n, const int32_t* gcnt, uint32_t* gmark, const
 // the smallest |a| of the group and d the distance to the group's box.  The
 // kernel takes the group count from sc->tree_groups; grid_groups (> 0) only
 // sizes the grid, and a grid below the count walks the rest in more rounds.
+// split: three further waves per group (list size 128 and no counting only); the
+// bits are the same either way.
 void launch_phys_walk(const Group* groups, int64_t grid_groups, const PhysNode* pn, const StateArrays& st,
                       const SysArrays& sy, double eps, int nleaf, double* ax, double* ay, double* az, double* pot,
-                      DevScalars* sc, bool kick, bool count, bool fp64, const float* amag, double alpha,
+                      DevScalars* sc, bool kick, bool count, bool fp64, bool split, const float* amag, double alpha,
                       double theta, int list, hipStream_t s);
+// Whether a walk over about `groups` groups of systems of `mean` bodies on
+// average takes further waves.  Few groups leave most SIMDs with one wave at
+// most, and a wave's time is then its evaluation's latency (about 2/3) plus its
+// walk's: as long as all workgroups are resident at once (LDS: 5 on a CU in
+// FP32, 3 in FP64) the further waves pay unless a group's lists are hardly ever
+// full.  Beyond that they pay only where a group's work is long: large systems
+// and groups of more than 32 (a smaller group's lanes share the lists already).
+// Walk (us, Plummer spheres, theta 0.5), one wave per group / 1 + 3:
+//   systems x bodies, group size   groups      FP32            FP64
+//      1 x 2,000     64               60    125 /   67     158 /   77
+//      1 x 16,384    64              373    511 /  177     677 /  253
+//     30 x 1,000     64              990     99 /   68     117 /  119
+//   1000 x 64        64            1,000     26 /   30
+//      8 x 4,096     32            1,496    173 /  145     212 /  194
+//     30 x 1,000     32            1,800     89 /  117     108 /  164
+//    200 x 200       64            2,000     46 /   75      52 /  107
+//      4 x 16,384    32            2,936    435 /  277     542 /  423
+//      8 x 4,096     16            2,944    112 /  169     179 /  247
+//    100 x 1,000     64            3,300    117 /  171     226 /  273
+//     32 x 4,096     64            3,392    261 /  235     506 /  456
+//     64 x 2,000     64            3,840    190 /  202     369 /  381
+//   4000 x 64        64            4,000     34 /   94
+//      1 x 200,000   64            4,436    578 /  492   1,119 / 1,064  (theta 0.8: 282 / 285, 537 / 560)
+//     32 x 4,096     32            5,984    285 /  350     457 /  571
+//     20 x 16,384    64            7,460    799 /  645   1,482 / 1,382
+//      5 x 65,536    64            7,335    753 /  680   1,489 / 1,509  (theta 0.8: 392 / 418, 734 / 835)
+//    300 x 1,000     64            9,900    252 /  427     461 /  726
+inline bool phys_walk_split(int64_t groups, int64_t mean, int group_size, double theta, bool fp64) {
+  if (mean < 128) return false;
+  if (groups <= (fp64 ? 768 : 1280)) return true;
+  if (mean < 4096 || group_size <= 16) return false;
+  if (group_size <= 32) return groups <= 3072;
+  return groups <= (fp64 || theta > 0.6 ? 4608 : 8192);
+}
 // FP64 direct sum with Plummer softening over all pairs of each system (G = 1).
 // part: room for direct_splits(n) * 4 * n partial sums when that is two parts
 // (fewer than 131,072 bodies).

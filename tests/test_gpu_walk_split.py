@@ -1,7 +1,8 @@
-"""Physics-mode walk: launches of up to 10,240 groups have further waves that
-evaluate the lists, larger ones one wave per group.  Both add the same terms in
-the same order, so a system's results are the same bits alone (few groups) and
-beside a large system that takes the launch over that number.
+"""Physics-mode walk: launches of few groups (up to 1,280, or 768 in FP64, or some
+thousand of large systems; not systems below 128 bodies) have further waves that
+evaluate the lists, others one wave per group.  Both add the same terms in the
+same order, so a system's results are the same bits alone (few groups) and
+beside a large system that takes the launch over every such number.
 """
 import numpy as np
 import pytest
@@ -35,4 +36,24 @@ def test_same_bits_alone_and_beside_a_large_system(precision, alpha):
         few, alone = run([p], precision, alpha, 2)
         assert few < 10240 * 4 // 5 - 64
         assert np.array_equal(got[at:at + len(p)], alone), len(p)
+        at += len(p)
+
+
+@pytest.mark.parametrize("precision", [PREC_MIXED, PREC_FP64])
+@pytest.mark.parametrize("copies,group_size", [(1, 64), (60, 64), (1, 32), (60, 32), (60, 16)])
+def test_same_bits_in_batches_of_any_width(copies, group_size, precision):
+    """The choice follows the mean size of the systems, the number of groups and
+    their size: small systems alone, beside copies of themselves and beside one
+    that lifts the mean."""
+    ps = [ic.plummer(n, seed=n, virial=None) for n in (127, 128, 700, 4100)]
+    kw = dict(theta=0.5, eps=0.01, mode=MODE_PHYSICS, precision=precision, adaptive_dt=False, group_size=group_size)
+    with Engine(**kw) as e:
+        e.upload_batch(ps * copies + [ic.plummer(40000, seed=2, virial=None)])
+        a, pot = e.accel(), e.potential()
+    at = 0
+    for p in ps:
+        with Engine(**kw) as f:
+            f.upload(p)
+            assert np.array_equal(a[at:at + len(p)], f.accel()), len(p)
+            assert np.array_equal(pot[at:at + len(p)], f.potential()), len(p)
         at += len(p)
