@@ -81,6 +81,7 @@ struct nbx_ctx {
   DBuf dacc, dpart;           // forces of the diagnostic passes (potential, direct sum), partial direct sums
   // systems
   std::vector<int64_t> sys_n;              // bodies per system
+  int64_t sys_mean = 0;                    // mean over the bodies of their system's size
   DBuf s_root, s_dt, s_v2, s_soff, s_sroot, s_send;
   DBuf groups, boxes, box_off, box_part;   // groups: reference mode's walk groups
   int64_t ngroups = 0;
@@ -362,7 +363,12 @@ nbx_status update_groups(nbx_ctx* c) {
 nbx_status set_systems(nbx_ctx* c) {
   const int S = (int)c->sys_n.size();
   std::vector<int32_t> soff(S + 1, 0);
-  for (int s = 0; s < S; ++s) soff[s + 1] = soff[s] + (int32_t)c->sys_n[s];
+  double squares = 0.0;
+  for (int s = 0; s < S; ++s) {
+    soff[s + 1] = soff[s] + (int32_t)c->sys_n[s];
+    squares += (double)c->sys_n[s] * (double)c->sys_n[s];
+  }
+  c->sys_mean = S ? (int64_t)(squares / soff[S]) : 0;
   std::vector<BoxBlock> boxes;
   std::vector<int32_t> box_off(S + 1, 0);
   for (int s = 0; s < S; ++s) {
@@ -708,8 +714,7 @@ int64_t group_grid(const nbx_ctx* c) { return c->ntgroups >= 0 ? c->ntgroups : c
 // Whether the physics walk takes evaluating waves; by the last count the host
 // has where this build's is still on the device.
 bool split_walk(const nbx_ctx* c) {
-  return phys_walk_split(c->ntgroups >= 0 ? c->ntgroups : c->hsc->tree_groups,
-                         c->n / std::max<int64_t>((int64_t)c->sys_n.size(), 1), c->cfg.group_size, c->cfg.theta,
+  return phys_walk_split(c->ntgroups >= 0 ? c->ntgroups : c->hsc->tree_groups, c->sys_mean, c->cfg.group_size,
                          c->cfg.precision == NBX_PREC_FP64);
 }
 

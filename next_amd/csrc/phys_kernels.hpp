@@ -90,13 +90,14 @@ void launch_phys_walk(const Group* groups, int64_t grid_groups, const PhysNode* 
                       const SysArrays& sy, double eps, int nleaf, double* ax, double* ay, double* az, double* pot,
                       DevScalars* sc, bool kick, bool count, bool fp64, bool split, const float* amag, double alpha,
                       double theta, int list, hipStream_t s);
-// Whether a walk over about `groups` groups of systems of `mean` bodies on
-// average takes further waves.  Few groups leave most SIMDs with one wave at
-// most, and a wave's time is then its evaluation's latency (about 2/3) plus its
-// walk's: as long as all workgroups are resident at once (LDS: 5 on a CU in
-// FP32, 3 in FP64) the further waves pay unless a group's lists are hardly ever
-// full.  Beyond that they pay only where a group's work is long: large systems
-// and groups of more than 32 (a smaller group's lanes share the lists already).
+// Whether a walk over about `groups` groups takes further waves; mean: the size
+// of a body's system, averaged over the bodies (the larger systems' groups are
+// the long ones).  Few groups leave most SIMDs with one wave at most, and a
+// wave's time is then its evaluation's latency (about 2/3) plus its walk's: as
+// long as all workgroups are resident at once (LDS: 5 on a CU in FP32, 3 in FP64)
+// the further waves pay unless a group's lists are hardly ever full.  Beyond that
+// they pay only where a group's work is long: larger systems, the more so the
+// smaller the groups (whose lanes share the lists already), down to 17.
 // Walk (us, Plummer spheres, theta 0.5), one wave per group / 1 + 3:
 //   systems x bodies, group size   groups      FP32            FP64
 //      1 x 2,000     64               60    125 /   67     158 /   77
@@ -106,6 +107,7 @@ void launch_phys_walk(const Group* groups, int64_t grid_groups, const PhysNode* 
 //      8 x 4,096     32            1,496    173 /  145     212 /  194
 //     30 x 1,000     32            1,800     89 /  117     108 /  164
 //    200 x 200       64            2,000     46 /   75      52 /  107
+//    30 of 1-5,000   64            2,157    245 /  178     381 /  326
 //      4 x 16,384    32            2,936    435 /  277     542 /  423
 //      8 x 4,096     16            2,944    112 /  169     179 /  247
 //    100 x 1,000     64            3,300    117 /  171     226 /  273
@@ -114,15 +116,20 @@ void launch_phys_walk(const Group* groups, int64_t grid_groups, const PhysNode* 
 //   4000 x 64        64            4,000     34 /   94
 //      1 x 200,000   64            4,436    578 /  492   1,119 / 1,064  (theta 0.8: 282 / 285, 537 / 560)
 //     32 x 4,096     32            5,984    285 /  350     457 /  571
-//     20 x 16,384    64            7,460    799 /  645   1,482 / 1,382
+//    30 of 1-33,000  64            6,605    940 /  639   1,612 / 1,360  (theta 0.7: 716 / 466, 1,163 / 924)
 //      5 x 65,536    64            7,335    753 /  680   1,489 / 1,509  (theta 0.8: 392 / 418, 734 / 835)
 //    300 x 1,000     64            9,900    252 /  427     461 /  726
-inline bool phys_walk_split(int64_t groups, int64_t mean, int group_size, double theta, bool fp64) {
+// They also shorten the longest group: two clusters of 140,000 bodies (6,174
+// groups) take a third of the time (0.31 to 0.47 times), which is why even ones go
+// on to 8,192 groups, where they lose up to a fifth in FP64 and above theta 0.6
+// (a uniform ball of 280,000 bodies, 6,102 groups, FP64: 0.99 at theta 0.35, 1.14 at
+// 0.62).
+inline bool phys_walk_split(int64_t groups, int64_t mean, int group_size, bool fp64) {
   if (mean < 128) return false;
   if (groups <= (fp64 ? 768 : 1280)) return true;
-  if (mean < 4096 || group_size <= 16) return false;
-  if (group_size <= 32) return groups <= 3072;
-  return groups <= (fp64 || theta > 0.6 ? 4608 : 8192);
+  const bool narrow = group_size <= 32;
+  if (group_size <= 16 || mean < (narrow ? 3072 : 1536)) return false;
+  return groups <= (mean < (narrow ? 8192 : 3072) ? 2304 : 8192);
 }
 // FP64 direct sum with Plummer softening over all pairs of each system (G = 1).
 // part: room for direct_splits(n) * 4 * n partial sums when that is two parts

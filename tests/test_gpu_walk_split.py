@@ -1,5 +1,5 @@
 """Physics-mode walk: launches of few groups (up to 1,280, or 768 in FP64, or some
-thousand of large systems; not systems below 128 bodies) have further waves that
+thousand of larger systems; not systems below 128 bodies) have further waves that
 evaluate the lists, others one wave per group.  Both add the same terms in the
 same order, so a system's results are the same bits alone (few groups) and
 beside a large system that takes the launch over every such number.
