@@ -38,10 +38,10 @@ struct alignas(128) RefNode {
 static_assert(sizeof(RefNode) == 128, "RefNode layout");
 
 // The per-visit fields of a node for the walk's traversal, in an array of
-// their own beside the node records (two per 64-byte scalar cache line): a
-// visited node costs one 32-byte scalar load.  acc2 is the upper edge of the
-// opening test's band in FP32, (size/theta)^2 (1 + 2e-6) rounded up, or NaN
-// where that is out of FP32's normal range (every decision then exact).
+// their own beside the node records: a visited node costs a lane two 16-byte
+// loads.  acc2 is the upper edge of the opening test's band in FP32,
+// (size/theta)^2 (1 + 2e-6) - 1e-20 rounded up, or NaN where that is out of
+// FP32's normal range (no decision is taken from it then).
 struct alignas(32) WalkHead {
   double cx, cy, cz;       // centre of mass
   float acc2;

@@ -705,7 +705,8 @@ __device__ __forceinline__ void upward_node(const UnitView& v, UnitMoments* lm, 
   out.qxx = qxx; out.qyy = qyy; out.qzz = qzz; out.qxy = qxy; out.qxz = qxz; out.qyz = qyz;
   out.size = size;
   // Upper edge of the opening test's band for r^2 (NEXT tests r^2 + 1e-20,
-  // so the 1e-20 is taken off the edge); NaN, and every decision exact, where
+  // so the 1e-20 is taken off the edge); NaN (a group's test then forms the band
+  // in FP64, a target's is exact) beyond FP32's range and where
   // (size/theta)^2 <= 1e-16, where the 1e-20 would eat the band's margin.
   const double q = size * inv_theta;
   const double q2 = q * q;
@@ -842,13 +843,13 @@ constexpr double kBandLow = (1.0 - 2e-6) / (1.0 + 2.2e-6);
 // Each target's terms are NEXT's; they are added in another order than
 // NEXT's recursion: group part first, every list summed from zero and then
 // added to the target's total (in one running sum, the 2^20 bodies' median
-// error was 7.2e-16; so it is 5.1e-16, NEXT's own order 4.9e-16).  Measured, walk per step, against one
-// union traversal per 64 targets with deferred evaluation: cold sphere 2^20
-// 1.69 -> 1.31 ms; 200,003 bodies at theta 0.3, a tenth dark matter 2.83 ->
+// error was 7.2e-16; so it is 5.1e-16, NEXT's own order 4.9e-16).  Measured,
+// walk per step, against one union traversal per 64 targets with deferred
+// evaluation: cold sphere 2^20 1.69 -> 1.31 ms; 200,003 bodies at theta 0.3, a tenth dark matter 2.83 ->
 // 0.83; Plummer 16,384 0.37 -> 0.11; 50,021 with a fifth dark matter 0.82 ->
 // 0.16.  Bound at 2^20 by the lanes' record loads: the texture units are busy
-// 88 % of the time and the vector cache misses 38 % of its lines (16 waves of
-// some 80 KB each on 32 KB), VALU 45 %.  Loading the records cooperatively (4
+// 86 % (addresses) and 91 % (data) of the time and a fifth of the vector cache's
+// accesses go on to L2 (16 waves of some 80 KB each on 32 KB), VALU 47 %.  Loading the records cooperatively (4
 // lanes per record, through LDS, by DMA or registers) cut the accesses by a
 // third and was as fast (1.29-1.34), several waves per workgroup and lanes
 // kept to windows of the list were slower, and so are 5 or 6 waves per SIMD
